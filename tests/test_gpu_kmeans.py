@@ -45,6 +45,30 @@ def test_kmeans_bit_exact(ctx, method, shape):
     _check(res, ref)
 
 
+@pytest.mark.parametrize("shape", [(255, 128, 40), (257, 600, 24), (1025, 17, 60),
+                                   (3000, 128, 200), (2049, 100, 5)])
+def test_kmeans_plusplus_rows_out_of_scale(ctx, shape):
+    """The seeding's int8 screen at block edges (256 rows, 1,024 weights) and
+    rows wider than a staged chunk (600), over rows it cannot resolve: far
+    outliers, near-duplicates (1e-6 apart), zero and tiny rows, and a common
+    offset of 1,000.  Every pick and D must still be the exact ones."""
+    n, d, k = shape
+    for case in ("scales", "offset"):
+        x = _mixture(n + d, n, d, max(2, k // 3))
+        if case == "scales":
+            x[::7] *= np.float32(1e4)
+            x[1::11] = x[1] * np.float32(1 + 1e-6)
+            x[3::29] = 0
+            x[4::31] *= np.float32(1e-18)
+        else:
+            x += np.float32(1000)
+        print(f"kmeans++ {case} n={n} d={d} k={k}", flush=True)
+        cfg = KMeansClusteringConfiguration(maxIterations=1, initMethod="kMeansPlusPlus", seed=k)
+        res = KMeansClustering(ctx, cfg).cluster(x, k)
+        _check(res, O.kmeans_cluster(x, k, init_method="kMeansPlusPlus", max_iter=1, tol=1e-4,
+                                     seed=k))
+
+
 def test_kmeans_custom_weights_empty_clusters(ctx):
     """Custom start with centroids far from the data (empty clusters refilled
     from the seeded stream), weights, and a run to convergence."""

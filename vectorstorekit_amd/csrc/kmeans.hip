@@ -321,143 +321,216 @@ __global__ void k_gather_rows_i64(const float *src, int64_t ld, const int64_t *r
 // ---------------------------------------------------------------------------
 // k-means++ on the device
 // ---------------------------------------------------------------------------
-constexpr int KP_T = 256;
+constexpr int KP_T = 256;       // threads of a block, rows of an update block
+constexpr int KP_B = 4 * KP_T;  // rows of a weight-sum block
+constexpr int KP_SLOTS = 64;    // max slots per pick (a power of two, one wave's lanes)
+constexpr int KP_TILE = 33 * KP_T;  // floats of the update's row tile
 
-constexpr int KPU_C = 32;     // columns of one staged chunk in k_kpp_update
-constexpr int KP_SLOTS = 64;  // max slots per pick (a power of two, one wave's lanes)
-constexpr int KPU_GRID = 4096;  // waves of k_kpp_update at most (16 per CU)
-
-// cc[a] = |x_c - x_{chosen[a]}| for the picks a < r, c = chosen[r]: one
-// wave per a, lanes over the coordinates.  Only the triangle test of
-// k_kpp_update reads it, so any summation order with a small relative error
-// serves (this one's is under (d / 64 + 11) 2^-25).
-__global__ __launch_bounds__(256) void k_kpp_cc(const float *x, int64_t ld, int32_t d,
-                                                const int64_t *chosen, int r, float *cc) {
-#pragma clang fp contract(off)
-  const int64_t c = chosen[r];
-  if (c < 0) return;
-  const int a = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (a >= r) return;  // wave-uniform
-  const float *xc = x + c * ld, *xa = x + chosen[a] * ld;
-  float s = 0.f;
-  for (int32_t j = lane; j < d; j += 64) {
-    const float t = xc[j] - xa[j];
-    s = s + t * t;
+// The rows as int8 for the update's screen: x_i = s_i q_i + residual, s_i =
+// max |x_ij| / 127, q_ij the nearest integer; par[i] = (s_i, |s_i q_i|^2, a
+// bound e_i on the residual's norm, 0).  A row with a component that is not
+// finite has e_i = +inf, which the screen never decides.  Codes: 16-byte
+// chunk ch of row i at dword 4 ((i / 64 * nch + ch) * 64 + i % 64), so that
+// 64 rows' loads of one chunk are one kilobyte.  One wave per row.
+__global__ __launch_bounds__(KP_T) void k_kpp_codes(const float *x, int64_t ld, int32_t d,
+                                                    int64_t n, int32_t nch, uint32_t *codes,
+                                                    float4 *par) {
+  const int lane = threadIdx.x & 63;
+  for (int64_t i = (int64_t)blockIdx.x * (KP_T / 64) + (threadIdx.x >> 6); i < n;
+       i += (int64_t)gridDim.x * (KP_T / 64)) {
+    const float *xi = x + i * ld;
+    float mx = 0.f;
+    bool bad = false;
+    for (int32_t j = lane; j < d; j += 64) {
+      const float v = fabsf(xi[j]);
+      bad |= !(v <= 0x1.fffffep127f);
+      mx = fmaxf(mx, v);
+    }
+  #pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    bad = __ballot(bad) != 0;
+    const float sc = bad ? 0.f : mx * (1.0f / 127.0f);
+    const float inv = sc > 0.f ? 1.0f / sc : 0.f;  // (inf for a tiny sc: codes clamp)
+    uint32_t qq = 0;  // (exact: at most 127^2 2^17)
+    float rr = 0.f;
+    uint32_t *out = codes + 4 * ((i >> 6) * nch * 64 + (i & 63));
+    for (int32_t w = lane; w < 4 * nch; w += 64) {
+      uint32_t pack = 0;
+  #pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int32_t j = 4 * w + u;
+        const float v = j < d ? xi[j] : 0.f;
+        float c = bad ? 0.f : rintf(v * inv);
+        c = fminf(fmaxf(c, -127.f), 127.f);  // (NaN of 0 * inf: -127, a larger residual)
+        const float res = __builtin_fmaf(-sc, c, v);  // one rounding
+        qq += (uint32_t)((int32_t)c * (int32_t)c);
+        rr += res * res;
+        pack |= ((uint32_t)(int32_t)c & 255u) << (8 * u);
+      }
+      out[256 * (w >> 2) + (w & 3)] = pack;
+    }
+  #pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      qq += __shfl_xor(qq, o);
+      rr += __shfl_xor(rr, o);
+    }
+    if (lane == 0) {
+      // e: the sums' and residuals' roundings are far below 2^-10 of it and
+      // 2^-20 of the row's norm; an underflowed square adds at most 2^-60
+      const float nx = sc * sqrtf((float)qq);
+      const float e = sqrtf(rr) * (1.f + 0x1p-10f) + nx * 0x1p-20f + 0x1p-60f * sqrtf((float)d);
+      par[i] = make_float4(sc, sc * sc * (float)qq, bad || !(e < 0x1p60f) ? __int_as_float(0x7f800000) : e,
+                           0.f);
+    }
   }
-#pragma unroll
-  for (int m = 32; m > 0; m >>= 1) s = s + __shfl_xor(s, m);
-  if (lane == 0) cc[a] = sqrtf(s);
 }
 
 // D[i] = min(D[i], |x_i - x_c|) with c = chosen[r] (sequential sqrt-L2, as
-// computeMinDistances, :401-419), near[i] = the pick that set D[i]; the max
-// over rows of D^2 lands in maxbits[(r + 1) * KP_SLOTS + s] for the KP_SLOTS
-// slots s (non-negative floats order as their bits; spread so the atomics
-// do not queue on one address).
+// computeMinDistances, :401-419); the max over rows of D^2 lands in
+// maxbits[(r + 1) * KP_SLOTS + s] for the KP_SLOTS slots s (non-negative
+// floats order as their bits; spread so the atomics do not queue on one
+// address).
 //
-// One wave per block strides over groups of 64 rows.  A row is skipped
-// (not read) when its nearest pick a has |x_c - x_a| >= 2 D skipm,
-// skipm = 1 + (d + 4) 2^-22.  The exact distance is >= |x_c - x_a| -
-// |x_i - x_a|, and (d + 4) 2^-22 exceeds the relative errors of the three
-// computed distances taken together (a sequential one: under (d + 4) 2^-25;
-// k_kpp_cc's: under (d / 64 + 11) 2^-25, counted twice), so the computed
-// distance would be >= D and D[i] would not change.  The test is only taken
-// for 2^-60 <= D <= 2^60, where no sum under- or overflows enough to break
-// the relative bounds.  The rows that do need the distance queue in LDS;
-// each full batch of 64 is staged through LDS in 128-byte column chunks
-// (coalesced) and every lane sums its own row in coordinate order.
-__global__ __launch_bounds__(64) void k_kpp_update(const float *__restrict__ x, int64_t ld,
-                                                   int32_t d, int64_t n,
-                                                   const int64_t *__restrict__ chosen, int r,
-                                                   const float *__restrict__ cc, float skipm,
-                                                   float *__restrict__ D,
-                                                   int32_t *__restrict__ near,
-                                                   uint32_t *__restrict__ maxbits) {
+// A block owns 256 rows, a thread one of them.  Most rows keep their D, and
+// the int8 rows show it: |x_i - x_c| >= |s_i q_i - s_c q_c| - e_i - e_c, and
+// the first term's square is |s_i q_i|^2 + |s_c q_c|^2 - 2 s_i s_c (q_i.q_c),
+// the dot product exact in integers, the rest within 2^-20 of the two norms'
+// sum.  A row whose bound is at least D skipm, skipm = 1 + (d + 4) 2^-22, is
+// left alone: the sequential fp32 distance is within (d + 4) 2^-25 of the
+// real one, so it would not be below D.  (Only for 2^-40 <= D <= 2^60 and
+// norms below 2^100, where nothing under- or overflows enough to matter.)
+// The screen reads d bytes a row where the distance reads 4 d, and 100,000
+// rows' codes at 128 dims stay in the XCDs' L2s from pick to pick.  Measured
+// at 100,000 x 128, 1,024 picks: 8.9 us a pick, against 30.7 us (and 3.7 us
+// for the distances between the picks) with a triangle test against the
+// nearest pick, which an uncovered cluster's rows never pass.
+//
+// The m rows that do need the distance are compacted in LDS and staged there
+// in column chunks (coalesced), one lane then summing each row in coordinate
+// order.  Late rounds leave a block a handful of rows and the kernel is a
+// chain of memory latencies, so the chunk is as wide as the tile allows: 32
+// columns for 256 rows up to 512 for 16 (a 128-dim row then takes one pass
+// where 32-column chunks took four), the next chunk's loads in flight while
+// one is summed.
+__global__ __launch_bounds__(KP_T) void k_kpp_update(const float *__restrict__ x, int64_t ld,
+                                                     int32_t d, int64_t n,
+                                                     const int64_t *__restrict__ chosen, int r,
+                                                     const uint4 *__restrict__ codes,
+                                                     const float4 *__restrict__ par,
+                                                     int32_t nch, float skipm,
+                                                     float *__restrict__ D,
+                                                     uint32_t *__restrict__ maxbits) {
 #pragma clang fp contract(off)
-  __shared__ float tile[64 * (KPU_C + 1)];
-  __shared__ int64_t l_row[128];
-  __shared__ float l_dm[128];
+  __shared__ float tile[KP_TILE];
+  __shared__ float s_xc[512];
+  __shared__ int32_t l_row[KP_T];
+  __shared__ float l_dm[KP_T];
+  __shared__ int32_t s_cnt[KP_T / 64];
+  __shared__ uint32_t s_max[KP_T / 64];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int64_t row0 = (int64_t)blockIdx.x * KP_T;
   const int64_t c = chosen[r];
+  const bool live = row0 + tid < n;
+  const float dm = live ? D[row0 + tid] : 0.f;
   if (c < 0) return;  // an earlier pick found degenerate data
-  const int lane = threadIdx.x;
   const float *__restrict__ xc = x + c * ld;
-  uint32_t b = 0;  // max D^2 bits seen by this lane
-  // the distances of the first m <= 64 queued rows
-  auto run = [&](int m) {
-    float s = 0.f;
-    for (int32_t j0 = 0; j0 < d; j0 += KPU_C) {
-      const int cw = d - j0 < KPU_C ? d - j0 : KPU_C;
-      __syncthreads();  // the previous chunk has been read
+  uint32_t b = 0;  // max D^2 bits seen by this thread
+  bool need = live;
+  if (live && codes) {
+    const float4 pi = par[row0 + tid], pc = par[c];
+    const uint4 *qi = codes + ((row0 >> 6) + w) * nch * 64 + lane;
+    const uint4 *qc = codes + (c >> 6) * nch * 64 + (c & 63);
+    int32_t dot = 0;
+#pragma unroll 8
+    for (int ch = 0; ch < nch; ++ch) {
+      const uint4 a = qi[64 * ch], o = qc[64 * ch];
+      dot = __builtin_amdgcn_sdot4((int)a.x, (int)o.x, dot, false);
+      dot = __builtin_amdgcn_sdot4((int)a.y, (int)o.y, dot, false);
+      dot = __builtin_amdgcn_sdot4((int)a.z, (int)o.z, dot, false);
+      dot = __builtin_amdgcn_sdot4((int)a.w, (int)o.w, dot, false);
+    }
+    const float t = pi.y + pc.y;
+    const float sq = (t - 2.0f * (pi.x * pc.x) * (float)dot) - 0x1p-20f * t;
+    const float lb = (sqrtf(fmaxf(sq, 0.f)) - (pi.z + pc.z)) * (1.f - 0x1p-20f);
+    need = !(dm >= 0x1p-40f && dm <= 0x1p60f && t <= 0x1p100f && lb >= dm * skipm);
+  }
+  if (live && !need) b = __float_as_uint(dm * dm);
+  const uint64_t mask = __ballot(need);
+  if (lane == 0) s_cnt[w] = __popcll(mask);
+  __syncthreads();
+  int base = 0, m = 0;
 #pragma unroll
-      for (int t = 0; t < KPU_C; ++t) {
-        const int rr = t * (64 / KPU_C) + lane / KPU_C, col = lane % KPU_C;
-        if (rr < m && col < cw)
-          tile[rr * (KPU_C + 1) + col] = x[l_row[rr] * ld + j0 + col];
-      }
-      __syncthreads();
-      if (lane < m)
-        for (int jj = 0; jj < cw; ++jj) {
-          const float t = tile[lane * (KPU_C + 1) + jj] - xc[j0 + jj];
-          s = s + t * t;
-        }
-    }
-    if (lane < m) {
-      float dm = l_dm[lane];
-      const float dist = sqrtf(s);
-      if (dist < dm) {
-        dm = dist;
-        const int64_t i = l_row[lane];
-        D[i] = dm;
-        near[i] = r;
-      }
-      const uint32_t bw = __float_as_uint(dm * dm);
-      b = bw > b ? bw : b;
-    }
-  };
-  int cnt = 0;  // queued rows (wave-uniform)
-  for (int64_t row0 = (int64_t)blockIdx.x * 64; row0 < n; row0 += (int64_t)gridDim.x * 64) {
-    const int64_t i = row0 + lane;
-    bool need = false;
-    float dm = 0.f;
-    if (i < n) {
-      dm = D[i];
-      const int32_t a = near[i];
-      need = !(a >= 0 && dm >= 0x1p-60f && dm <= 0x1p60f && cc[a] >= 2.0f * dm * skipm);
-      if (!need) {
-        const uint32_t bw = __float_as_uint(dm * dm);
-        b = bw > b ? bw : b;
-      }
-    }
-    const uint64_t mask = __ballot(need);
+  for (int j = 0; j < KP_T / 64; ++j) {
+    if (j < w) base += s_cnt[j];
+    m += s_cnt[j];
+  }
+  if (m > 0) {  // block-uniform
     if (need) {
-      const int pos = cnt + (int)__builtin_amdgcn_mbcnt_hi(
-                                (uint32_t)(mask >> 32),
-                                __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-      l_row[pos] = i;
+      const int pos = base + (int)__builtin_amdgcn_mbcnt_hi(
+                                 (uint32_t)(mask >> 32),
+                                 __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+      l_row[pos] = tid;
       l_dm[pos] = dm;
     }
-    cnt += __popcll(mask);
-    if (cnt >= 64) {
-      __syncthreads();
-      run(64);
-      __syncthreads();
-      if (lane < cnt - 64) {
-        l_row[lane] = l_row[64 + lane];
-        l_dm[lane] = l_dm[64 + lane];
+    // columns per chunk: rows rounded up to a power of two x columns = 8192
+    const int sh = m <= 16 ? 9 : m <= 32 ? 8 : m <= 64 ? 7 : m <= 128 ? 6 : 5;
+    const int cw = 1 << sh, stride = cw + 1;  // (odd: a lane per row reads without conflicts)
+    __syncthreads();
+    constexpr int NV = 8192 / KP_T;
+    float v[NV];
+    auto load = [&](int32_t j0) {
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        const int e = u * KP_T + tid;
+        const int rr = e >> sh, col = j0 + (e & (cw - 1));
+        v[u] = rr < m && col < d ? x[(row0 + l_row[rr]) * ld + col] : 0.f;
       }
-      cnt -= 64;
+    };
+    load(0);
+    float s = 0.f;
+    for (int32_t j0 = 0; j0 < d; j0 += cw) {
+      if (j0 > 0) __syncthreads();  // the previous chunk has been read
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        const int e = u * KP_T + tid;
+        tile[(e >> sh) * stride + (e & (cw - 1))] = v[u];
+      }
+      for (int j = tid; j < cw && j0 + j < d; j += KP_T) s_xc[j] = xc[j0 + j];
+      __syncthreads();
+      if (j0 + cw < d) load(j0 + cw);
+      if (tid < m) {
+        const int jn = d - j0 < cw ? d - j0 : cw;
+        const float *t = tile + tid * stride;
+#pragma unroll 8
+        for (int j = 0; j < jn; ++j) {
+          const float e = t[j] - s_xc[j];
+          s = s + e * e;
+        }
+      }
+    }
+    if (tid < m) {
+      float old = l_dm[tid];
+      const float dist = sqrtf(s);
+      if (dist < old) {
+        old = dist;
+        D[row0 + l_row[tid]] = dist;
+      }
+      const uint32_t bw = __float_as_uint(old * old);
+      b = bw > b ? bw : b;
     }
   }
-  if (cnt > 0) {
-    __syncthreads();
-    run(cnt);
-  }
 #pragma unroll
-  for (int m = 32; m > 0; m >>= 1) {
-    const uint32_t o = __shfl_xor(b, m);
-    b = o > b ? o : b;
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint32_t v = __shfl_xor(b, o);
+    b = v > b ? v : b;
   }
-  if (lane == 0) atomicMax(&maxbits[(r + 1) * KP_SLOTS + blockIdx.x % KP_SLOTS], b);
+  if (lane == 0) s_max[w] = b;
+  __syncthreads();
+  if (tid == 0) {
+#pragma unroll
+    for (int j = 0; j < KP_T / 64; ++j) b = s_max[j] > b ? s_max[j] : b;
+    atomicMax(&maxbits[(r + 1) * KP_SLOTS + blockIdx.x % KP_SLOTS], b);
+  }
 }
 
 // the max of pick r + 1's KP_SLOTS slots, through LDS to the whole block
@@ -483,37 +556,12 @@ __device__ inline uint64_t kpp_fixed(float dm, float maxw) {
   return (uint64_t)((double)w / (double)maxw * 4294967296.0);
 }
 
-// bsum[b] = sum of the fixed weights of block b's rows
-__global__ __launch_bounds__(KP_T) void k_kpp_blocksum(const float *D, int64_t n,
-                                                       const uint32_t *maxbits,
-                                                       const int64_t *chosen, int r,
-                                                       uint64_t *bsum) {
-  __shared__ uint64_t ws[KP_T / 64];
-  __shared__ uint32_t s_mx;
-  if (chosen[r] < 0) return;
-  const float maxw = kpp_maxw(maxbits, r, &s_mx);
-  const int64_t i = blockIdx.x * (int64_t)KP_T + threadIdx.x;
-  uint64_t f = i < n ? kpp_fixed(D[i], maxw) : 0;
-#pragma unroll
-  for (int m = 32; m > 0; m >>= 1) {
-    const uint64_t lo = __shfl_xor((uint32_t)f, m), hi = __shfl_xor((uint32_t)(f >> 32), m);
-    f += (hi << 32) | lo;
-  }
-  if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = f;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint64_t s = 0;
-    for (int j = 0; j < KP_T / 64; ++j) s += ws[j];
-    bsum[blockIdx.x] = s;
-  }
-}
-
 __device__ inline uint64_t shfl_up_u64(uint64_t v, int o) {
   const uint32_t lo = __shfl_up((uint32_t)v, o), hi = __shfl_up((uint32_t)(v >> 32), o);
   return ((uint64_t)hi << 32) | lo;
 }
 
-// exclusive prefix over a 1024-thread block of one uint64 per thread;
+// exclusive prefix over the block's threads of one uint64 per thread;
 // *total receives the block's sum
 __device__ uint64_t block_excl_u64(uint64_t v, uint64_t *wsum, uint64_t *total) {
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -537,55 +585,87 @@ __device__ uint64_t block_excl_u64(uint64_t v, uint64_t *wsum, uint64_t *total) 
 
 // pick r + 1: u = Int.random(in: 0..<total) from the SeedableRNG stream
 // whose state is *rng; the chosen row is the first whose inclusive
-// fixed-weight prefix exceeds u.  One block of 1024 threads.  total = 0
-// (every row on a chosen centroid) is the reference's degenerateData
-// (:235-237): chosen[r + 1] = -1.
-__global__ __launch_bounds__(1024) void k_kpp_pick(const uint64_t *bsum, int64_t nb,
-                                                   const float *D, int64_t n,
-                                                   const uint32_t *maxbits,
-                                                   uint64_t *rng, int r,
-                                                   int64_t *chosen) {
-  __shared__ uint64_t wsum[16];
-  __shared__ uint64_t s_u, s_base;
+// fixed-weight prefix exceeds u.  total = 0 (every row on a chosen centroid)
+// is the reference's degenerateData (:235-237): chosen[r + 1] = -1.
+//
+// Every block sums the fixed weights of its 1024 rows; the block that counts
+// itself last in *done has them all and picks: one launch of 7.2 us at
+// 100,000 rows instead of a sum and a pick launch of 4.4 and 6.6 us.  No
+// fence is needed, and none is used (an agent-scope release writes back the
+// XCD's whole L2): a block's sum goes out by a returning exchange at agent
+// scope, its arrival is counted only after that returned, and the last block
+// reads the sums by agent-scope loads.  No block waits for another.
+__global__ __launch_bounds__(KP_T) void k_kpp_pick(uint64_t *bsum, int64_t nb, const float *D,
+                                                   int64_t n, const uint32_t *maxbits,
+                                                   uint64_t *rng, int r, int64_t *chosen,
+                                                   uint32_t *done) {
+  __shared__ uint64_t wsum[KP_T / 64];
+  __shared__ uint64_t s_base;
   __shared__ int64_t s_blk, s_row;
+  __shared__ uint32_t s_mx;
+  __shared__ bool s_last;
   const int t = threadIdx.x;
+  const int64_t i0 = (int64_t)blockIdx.x * KP_B;
+  float dv[KP_B / KP_T];
+#pragma unroll
+  for (int u = 0; u < KP_B / KP_T; ++u) {
+    const int64_t i = i0 + u * KP_T + t;
+    dv[u] = i < n ? D[i] : 0.f;  // (a zero distance weighs 0)
+  }
+  uint64_t st = *rng;  // (only the last block writes it, after its count)
   if (chosen[r] < 0) {
-    if (t == 0) chosen[r + 1] = -1;
+    if (blockIdx.x == 0 && t == 0) chosen[r + 1] = -1;
     return;
   }
-  // the total
+  const float maxw = kpp_maxw(maxbits, r, &s_mx);
+  uint64_t f = 0;
+#pragma unroll
+  for (int u = 0; u < KP_B / KP_T; ++u) f += kpp_fixed(dv[u], maxw);
+  uint64_t sum;
+  (void)block_excl_u64(f, wsum, &sum);
+  if (t == 0) {
+    uint64_t old = __hip_atomic_exchange(&bsum[blockIdx.x], sum, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" : "+v"(old) : : "memory");  // the exchange has returned
+    s_last = atomicAdd(done, 1u) == (uint32_t)nb - 1u;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  // thread t takes the sums of a run of consecutive blocks, so one scan over
+  // the threads gives the total and every run's prefix
+  const int64_t per = (nb + KP_T - 1) / KP_T;
+  const int64_t b0 = t * per, b1 = b0 + per < nb ? b0 + per : nb;
+  auto sum_of = [&](int64_t b) -> uint64_t {
+    return __hip_atomic_load(&bsum[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
   uint64_t part = 0;
-  for (int64_t b = t; b < nb; b += 1024) part += bsum[b];
+  for (int64_t b = b0; b < b1; ++b) part += sum_of(b);
+  if (t == 0) {
+    *done = 0;  // for the next pick's launch
+    s_blk = -1;
+    s_row = -1;
+  }
   uint64_t total;
-  (void)block_excl_u64(part, wsum, &total);
+  uint64_t before = block_excl_u64(part, wsum, &total);
   if (total == 0) {
     if (t == 0) chosen[r + 1] = -1;
     return;
   }
-  if (t == 0) {
-    uint64_t st = *rng;
-    s_u = swift_bounded(st, total);
-    *rng = st;
-    s_blk = -1;
-    s_row = -1;
+  const uint64_t u = swift_bounded(st, total);  // (every thread draws the same)
+  if (t == 0) *rng = st;
+  // the block holding u
+  if (before <= u && u < before + part) {
+    for (int64_t b = b0; b < b1; ++b) {
+      const uint64_t v = per == 1 ? part : sum_of(b);
+      if (u < before + v) {
+        s_blk = b;
+        s_base = before;
+        break;
+      }
+      before += v;
+    }
   }
   __syncthreads();
-  const uint64_t u = s_u;
-  // the block holding u
-  uint64_t carry = 0;
-  for (int64_t b0 = 0; b0 < nb; b0 += 1024) {
-    const int64_t b = b0 + t;
-    const uint64_t v = b < nb ? bsum[b] : 0;
-    uint64_t tile;
-    const uint64_t ex = carry + block_excl_u64(v, wsum, &tile);
-    if (b < nb && v > 0 && ex <= u && u < ex + v) {
-      s_blk = b;
-      s_base = ex;
-    }
-    carry += tile;
-    __syncthreads();
-    if (s_blk >= 0) break;
-  }
   // the row inside it (a block is always found: the blocks' sums partition
   // [0, total); the test keeps a broken invariant from reading out of range)
   const int64_t blk = s_blk;
@@ -593,13 +673,21 @@ __global__ __launch_bounds__(1024) void k_kpp_pick(const uint64_t *bsum, int64_t
     if (t == 0) chosen[r + 1] = -1;
     return;
   }
-  __shared__ uint32_t s_mx;
-  const float maxw = kpp_maxw(maxbits, r, &s_mx);
-  const int64_t i = blk * KP_T + t;
-  const uint64_t f = (t < KP_T && i < n) ? kpp_fixed(D[i], maxw) : 0;
+  // consecutive rows per thread, so that thread order is row order
+  const int64_t i1 = blk * KP_B + (int64_t)t * (KP_B / KP_T);
+  uint64_t fx[KP_B / KP_T], mine = 0;
+#pragma unroll
+  for (int j = 0; j < KP_B / KP_T; ++j) {
+    fx[j] = i1 + j < n ? kpp_fixed(D[i1 + j], maxw) : 0;
+    mine += fx[j];
+  }
   uint64_t tot2;
-  const uint64_t ex = s_base + block_excl_u64(f, wsum, &tot2);
-  if (t < KP_T && i < n && f > 0 && ex <= u && u < ex + f) s_row = i;
+  uint64_t ex = s_base + block_excl_u64(mine, wsum, &tot2);
+#pragma unroll
+  for (int j = 0; j < KP_B / KP_T; ++j) {
+    if (fx[j] > 0 && ex <= u && u < ex + fx[j]) s_row = i1 + j;
+    ex += fx[j];
+  }
   __syncthreads();
   if (t == 0) chosen[r + 1] = s_row;
 }
@@ -706,17 +794,16 @@ static bool init_plusplus(vsk_ctx *ctx, const float *dx, int64_t n, int32_t d,
   KernelTimer tm(ctx, "kmeans_plusplus", (double)n * k);
   float *D = static_cast<float *>(ctx->scratch_ptr("km.kppD", sizeof(float) * (size_t)n));
   fill_i32(ctx, reinterpret_cast<int32_t *>(D), n, 0x7F800000);  // +inf
-  int32_t *near = static_cast<int32_t *>(
-      ctx->scratch_ptr("km.kppnear", sizeof(int32_t) * (size_t)n));
-  fill_i32(ctx, near, n, -1);
-  float *cc = static_cast<float *>(ctx->scratch_ptr("km.kppcc", sizeof(float) * (size_t)k));
   const float skipm = 1.0f + (float)(d + 4) * 0x1p-22f;
   uint32_t *maxbits = static_cast<uint32_t *>(
       ctx->scratch_ptr("km.kppmax", sizeof(uint32_t) * (size_t)(k + 1) * KP_SLOTS));
   fill_i32(ctx, reinterpret_cast<int32_t *>(maxbits), (int64_t)(k + 1) * KP_SLOTS, 0);
-  const int64_t nb = ceil_div(n, KP_T);
+  const int64_t nb = ceil_div(n, KP_B);
   uint64_t *bsum = static_cast<uint64_t *>(
       ctx->scratch_ptr("km.kppbsum", sizeof(uint64_t) * (size_t)nb));
+  uint32_t *done =
+      static_cast<uint32_t *>(ctx->scratch_ptr("km.kppdone", sizeof(uint32_t)));
+  fill_i32(ctx, reinterpret_cast<int32_t *>(done), 1, 0);
   // [first row, stream state after drawing it]
   uint64_t st = seed;
   const int64_t first = (int64_t)swift_bounded(st, (uint64_t)n);
@@ -726,15 +813,23 @@ static bool init_plusplus(vsk_ctx *ctx, const float *dx, int64_t n, int32_t d,
                          ctx->stream));
   VSK_HIP(hipMemcpyAsync(rng, &init[1], sizeof(uint64_t), hipMemcpyHostToDevice,
                          ctx->stream));
+  // (an int8 dot product of 2^17 dims still fits 32 bits)
+  const int32_t nch = (int32_t)ceil_div(d, 16);
+  uint4 *codes = nullptr;
+  float4 *par = nullptr;
+  if (d <= 1 << 17) {
+    codes = static_cast<uint4 *>(ctx->scratch_ptr(
+        "km.kppcodes", sizeof(uint4) * (size_t)ceil_div(n, 64) * 64 * nch));
+    par = static_cast<float4 *>(ctx->scratch_ptr("km.kpppar", sizeof(float4) * (size_t)n));
+    k_kpp_codes<<<(unsigned)std::min<int64_t>(ceil_div(n, KP_T / 64), 16384), KP_T, 0,
+                  ctx->stream>>>(
+        dx, ld, d, n, nch, reinterpret_cast<uint32_t *>(codes), par);
+  }
   for (int r = 0; r + 1 < k; ++r) {
-    if (r > 0)
-      k_kpp_cc<<<(unsigned)ceil_div(r, 4), 256, 0, ctx->stream>>>(dx, ld, d, chosen, r, cc);
-    k_kpp_update<<<(unsigned)std::min<int64_t>(ceil_div(n, 64), KPU_GRID), 64, 0,
-                   ctx->stream>>>(
-        dx, ld, d, n, chosen, r, cc, skipm, D, near, maxbits);
-    k_kpp_blocksum<<<(unsigned)nb, KP_T, 0, ctx->stream>>>(D, n, maxbits, chosen, r,
-                                                           bsum);
-    k_kpp_pick<<<1, 1024, 0, ctx->stream>>>(bsum, nb, D, n, maxbits, rng, r, chosen);
+    k_kpp_update<<<(unsigned)ceil_div(n, KP_T), KP_T, 0, ctx->stream>>>(
+        dx, ld, d, n, chosen, r, codes, par, nch, skipm, D, maxbits);
+    k_kpp_pick<<<(unsigned)nb, KP_T, 0, ctx->stream>>>(bsum, nb, D, n, maxbits, rng, r,
+                                                       chosen, done);
   }
   check_launch("kmeans_plusplus");
   std::vector<int64_t> h((size_t)k);
