@@ -14,7 +14,7 @@ from oracle import oracle as O
 from parity import assert_sorted_unique, assert_topk_match
 from vectorstorekit_amd import VSKError, VectorDatabase
 from vectorstorekit_amd._lib import (METRIC_COSINE, METRIC_COSINE_NORMALIZED, METRIC_DOT,
-                                     METRIC_L1, METRIC_L2, METRIC_L2SQ)
+                                     METRIC_HAMMING, METRIC_L1, METRIC_L2, METRIC_L2SQ)
 
 pytestmark = pytest.mark.gpu
 
@@ -271,6 +271,30 @@ def test_screen_normalized_db_and_device_queries(sctx):
     od, oi = O.search_flat(qn, xn, 25, METRIC_COSINE_NORMALIZED)
     np.testing.assert_array_equal(gi.cpu().numpy(), oi)
     np.testing.assert_array_equal(gd.cpu().numpy(), od)
+
+
+@pytest.mark.parametrize("metric", ALL + [METRIC_HAMMING])
+def test_stream_scan_edges(ctx, metric):
+    """The exact scan as a stream over the rows (few queries or few tiles):
+    rows and queries around its 64-row waves and its 1, 4 and 8 queries a
+    wave, columns around its 32- and 64-column chunks, one dense chunk of
+    more than 16,384 rows (runs of 2,048 selected on their own, the last one
+    short) and rows with infinities and NaN; bit for bit the oracle."""
+    for n, nq, d, k in [(1, 1, 3, 1), (63, 2, 4, 5), (65, 4, 33, 64), (1000, 5, 64, 10),
+                        (2500, 9, 100, 128), (300, 64, 130, 7), (17_000, 1, 37, 128),
+                        (20_481, 3, 65, 100), (40_000, 16, 64, 11), (64, 100, 31, 64)]:
+        x, q = _data(n + nq + d, n, nq, d, normalize=metric == METRIC_COSINE_NORMALIZED)
+        if n > 500:
+            x[n // 2] = np.inf
+            x[n // 3, d - 1] = np.nan
+            x[5] = x[4]
+        print(f"stream metric={metric} n={n} nq={nq} d={d} k={k}", flush=True)
+        db = VectorDatabase(ctx, x)
+        gd, gi = db.search(q, k, metric)
+        od, oi = O.search_flat(q, x, k, metric)
+        np.testing.assert_array_equal(gi, oi)
+        np.testing.assert_array_equal(gd, od)
+        np.testing.assert_array_equal(db.distances(q, metric), O.distances(q, x, metric))
 
 
 @pytest.mark.parametrize("metric", SCREEN)

@@ -51,6 +51,10 @@ __device__ inline void emit(const FlatArgs &a, int64_t qi, int64_t row,
   if constexpr (MODE == MODE_MATRIX) {
     a.mat[qi * a.ldm + row] = METRIC == VSK_METRIC_L2 ? sqrtf(dist) : dist;
   } else {
+    if (MODE == MODE_DENSE && a.words) {
+      a.words[qi * a.cap + (row - a.r0)] = vsk_f2ord(dist);
+      return;
+    }
     uint64_t key = vsk_key(dist, (uint32_t)row);
     if constexpr (MODE == MODE_DENSE) {
       a.cand[qi * a.cap + (row - a.r0)] = key;
@@ -338,6 +342,145 @@ __global__ __launch_bounds__(256) void k_flat_valu(FlatArgs a, int32_t *argmin) 
   }
 }
 
+// The same distances as a stream over the rows, for launches of few queries
+// or few tiles.  A wave owns 64 rows and V queries: it gathers C columns of
+// its rows in whole 4 C-byte segments into its own LDS tile, the next C
+// columns' loads in flight meanwhile, and each lane adds its row's terms in
+// dimension order for every query.  The queries' columns are staged beside
+// them and read as broadcasts (scalar loads of them made every 16 columns
+// wait for the scalar cache: 1.5 x slower at V = 4).  No barrier: the waves
+// are independent, and 9 (C = 64) or 17 (C = 32) of them share a CU.  Query
+// groups of the same rows run next to each other on one XCD, whose L2 then
+// serves all but the first.
+//
+// Bound: HBM up to about 4 queries, then the VALU (2 or 3 operations a term).
+// Measured against the 64 x 32 tiles of k_flat_valu (dot product): 100,000 x
+// 768, 1 query 49 against 163 us (6.3 TB/s), 4 queries 53 against 165, 16
+// queries 95 against 167, 32 queries 159 against 173; 10,000 x 128, 1 query
+// 4.7 against 16 us, 100 queries about 15 against 18.
+template <int MODE, int OP, int V, int C>
+__global__ __launch_bounds__(64) void k_flat_stream(FlatArgs a, int32_t groups) {
+#pragma clang fp contract(off)
+  constexpr int NL = C / 4;      // row loads a chunk, 16 bytes a lane
+  constexpr int LD = C + 4;      // LDS row stride (floats): conflict-free 16-byte reads
+  constexpr int LPR = C / 4;     // lanes a row segment
+  constexpr int RPI = 64 / LPR;  // rows a load instruction
+  constexpr int QN = (V + RPI - 1) / RPI;  // query loads a chunk
+  __shared__ __attribute__((aligned(16))) float tile[64 * LD];
+  __shared__ __attribute__((aligned(16))) float qt[V * C];
+  const int lane = threadIdx.x;
+  // block L runs on XCD L % 8: there, groups of one row tile in turn
+  const int64_t l8 = blockIdx.x >> 3;
+  const int64_t q0 = (l8 % groups) * V;
+  const int64_t row0 = a.r0 + ((l8 / groups) * 8 + (blockIdx.x & 7)) * 64;
+  if (row0 >= a.r1) return;
+  const int seg = lane % LPR, sub = lane / LPR;
+  const int64_t last = a.r1 - 1 - row0;  // rows past the end read the last one
+  const float *src[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const int64_t r = sub + RPI * i;
+    src[i] = a.X + (row0 + (r < last ? r : last)) * a.ldx;
+  }
+  const float *qsrc[QN];  // (queries past the last read the last one)
+#pragma unroll
+  for (int u = 0; u < QN; ++u) {
+    const int64_t q = q0 + RPI * u + sub;
+    qsrc[u] = a.Q + (q < a.nq ? q : a.nq - 1) * a.ldq;
+  }
+  const int32_t cmax = a.kdim - 4;  // a segment past the row end is clamped
+  f4 buf[NL], qbuf[QN];
+  auto load = [&](int32_t c0) {
+    const int32_t col = c0 + 4 * seg < cmax ? c0 + 4 * seg : cmax;
+#pragma unroll
+    for (int u = 0; u < QN; ++u) qbuf[u] = *reinterpret_cast<const f4 *>(qsrc[u] + col);
+#pragma unroll
+    for (int i = 0; i < NL; ++i) buf[i] = *reinterpret_cast<const f4 *>(src[i] + col);
+  };
+  float acc[V];
+#pragma unroll
+  for (int v = 0; v < V; ++v) acc[v] = 0.f;
+  // one query a wave: its cosine norm is summed here too (the wave waits on
+  // memory), which saves a launch before the scan
+  float qsum = 0.f;
+  load(0);
+  for (int32_t k0 = 0; k0 < a.kdim; k0 += C) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i)
+      *reinterpret_cast<f4 *>(tile + (sub + RPI * i) * LD + 4 * seg) = buf[i];
+#pragma unroll
+    for (int u = 0; u < QN; ++u)
+      if (RPI * u + sub < V)
+        *reinterpret_cast<f4 *>(qt + (RPI * u + sub) * C + 4 * seg) = qbuf[u];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (k0 + C < a.kdim) load(k0 + C);
+    const float *xr = tile + lane * LD;
+    const int32_t kn = a.kdim - k0 < C ? a.kdim - k0 : C;
+#pragma unroll 4
+    for (int32_t k = 0; k < kn; k += 4) {
+      const f4 xv = *reinterpret_cast<const f4 *>(xr + k);
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        const f4 qv = *reinterpret_cast<const f4 *>(qt + v * C + k);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[v] += valu_term<OP>(qv[c], xv[c]);
+        if constexpr (OP == OP_COSSEQ && V == 1) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) qsum += qv[c] * qv[c];
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  if (lane > last) return;
+  const int64_t row = row0 + lane;
+  const float xn = OP == OP_COSSEQ ? a.xaux[row] : 0.f;
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    if (q0 + v >= a.nq) break;
+    if (a.active && !a.active[q0 + v]) continue;
+    const float qn = OP != OP_COSSEQ ? 0.f : V == 1 ? sqrtf(qsum) : a.qaux[q0 + v];
+    const float dist = OP == OP_COSSEQ ? 1.0f - acc[v] / (qn * xn + 1e-8f)
+                                       : valu_final<OP>(acc[v]);
+    emit<MODE, VSK_METRIC_L1>(a, q0 + v, row, dist,
+                              MODE == MODE_FILTER ? a.thresh[q0 + v] : 0);
+  }
+}
+
+template <int OP, int V, int C>
+static void launch_stream_v(vsk_ctx *ctx, const FlatArgs &a, int mode) {
+  const int64_t groups = ceil_div(a.nq, V);
+  const int64_t tiles = ceil_div(ceil_div(a.r1 - a.r0, 64), 8) * 8;
+  const dim3 grid((unsigned)(groups * tiles));
+  const int32_t g = (int32_t)groups;
+  if (mode == MODE_DENSE)
+    k_flat_stream<MODE_DENSE, OP, V, C><<<grid, 64, 0, ctx->stream>>>(a, g);
+  else if (mode == MODE_FILTER)
+    k_flat_stream<MODE_FILTER, OP, V, C><<<grid, 64, 0, ctx->stream>>>(a, g);
+  else
+    k_flat_stream<MODE_MATRIX, OP, V, C><<<grid, 64, 0, ctx->stream>>>(a, g);
+}
+
+// Queries a wave: as few as leave the launch about one round of resident
+// waves (9 or so a CU), since a small launch takes one wave's time; eight
+// when there is more to do, which reads the rows least often.  (10,000 x 128:
+// 8 queries one a wave 6.4, four a wave 7.4 us; 16 queries 9.6 and 8.1; 64
+// queries four a wave 15.3, eight 16.0; 128 queries 23.5 and 20.4.)
+template <int OP>
+static void launch_stream(vsk_ctx *ctx, const FlatArgs &a, int mode) {
+  const int64_t tiles = ceil_div(a.r1 - a.r0, 64), cus = ctx->cu_count;
+  if (a.nq == 1 || tiles * a.nq <= 8 * cus)
+    launch_stream_v<OP, 1, 64>(ctx, a, mode);
+  else if (tiles * ceil_div(a.nq, 4) <= 10 * cus)
+    launch_stream_v<OP, 4, 64>(ctx, a, mode);
+  else
+    launch_stream_v<OP, 8, 32>(ctx, a, mode);
+}
+
 template <int METRIC>
 static void launch_mfma(vsk_ctx *ctx, dim3 grid, const FlatArgs &a, int mode) {
   if (mode == MODE_DENSE)
@@ -348,41 +491,32 @@ static void launch_mfma(vsk_ctx *ctx, dim3 grid, const FlatArgs &a, int mode) {
     k_flat_mfma<MODE_MATRIX, METRIC><<<grid, 256, 0, ctx->stream>>>(a);
 }
 
-template <int OP, int U, int V>
-static void launch_valu(vsk_ctx *ctx, dim3 grid, const FlatArgs &a, int mode,
-                        int32_t *argmin) {
+// the exact VALU scan in tiles of 128 rows x 64 queries
+template <int OP>
+static void launch_valu_tiles(vsk_ctx *ctx, dim3 grid, const FlatArgs &a, int mode,
+                              int32_t *argmin) {
   if (mode == MODE_DENSE)
-    k_flat_valu<MODE_DENSE, OP, U, V><<<grid, 256, 0, ctx->stream>>>(a, argmin);
+    k_flat_valu<MODE_DENSE, OP, 4, 8><<<grid, 256, 0, ctx->stream>>>(a, argmin);
   else if (mode == MODE_FILTER)
-    k_flat_valu<MODE_FILTER, OP, U, V><<<grid, 256, 0, ctx->stream>>>(a, argmin);
+    k_flat_valu<MODE_FILTER, OP, 4, 8><<<grid, 256, 0, ctx->stream>>>(a, argmin);
   else if (mode == MODE_MATRIX)
-    k_flat_valu<MODE_MATRIX, OP, U, V><<<grid, 256, 0, ctx->stream>>>(a, argmin);
+    k_flat_valu<MODE_MATRIX, OP, 4, 8><<<grid, 256, 0, ctx->stream>>>(a, argmin);
   else
-    k_flat_valu<MODE_ARGMIN, OP, U, V><<<grid, 256, 0, ctx->stream>>>(a, argmin);
+    k_flat_valu<MODE_ARGMIN, OP, 4, 8><<<grid, 256, 0, ctx->stream>>>(a, argmin);
 }
 
-// the exact VALU scan in tiles of 128 rows x 64 queries, or, when those
-// leave fewer than 4 workgroups per CU, 64 rows x 32 queries (a quarter of
-// the work per thread: small problems are latency-bound)
+// metrics of the exact VALU scan
+static bool metric_is_valu(int32_t metric) {
+  return metric == VSK_METRIC_L1 || metric == VSK_METRIC_HAMMING || metric >= METRIC_L2_EXACT;
+}
+
 template <int OP>
-static void launch_valu_sized(vsk_ctx *ctx, FlatArgs a, int mode, int32_t *argmin,
-                              bool small) {
-  const int64_t rows = a.r1 - a.r0;
-  const int64_t tq = small ? 32 : FB_Q, tn = small ? 64 : FB_N;
-  const int64_t qt = ceil_div(a.nq, tq);
-  int64_t splits = mode == MODE_ARGMIN ? 1 : ceil_div(4096, qt);
-  const int64_t max_splits = ceil_div(rows, tn);
-  if (splits > max_splits) splits = max_splits;
-  if (splits > 65535) splits = 65535;
-  if (splits < 1) splits = 1;
-  a.rows_per_split = ceil_div(ceil_div(rows, splits), tn) * tn;
-  splits = ceil_div(rows, a.rows_per_split);
-  if (qt > 0x7FFFFFFF) fail(VSK_ERR_INVALID_BUFFER_SIZE, "too many queries");
-  const dim3 grid((unsigned)qt, (unsigned)splits);
-  if (small)
-    launch_valu<OP, 2, 4>(ctx, grid, a, mode, argmin);
+static void launch_exact(vsk_ctx *ctx, dim3 grid, const FlatArgs &a, int mode,
+                         int32_t *argmin, bool stream) {
+  if (stream)
+    launch_stream<OP>(ctx, a, mode);
   else
-    launch_valu<OP, 4, 8>(ctx, grid, a, mode, argmin);
+    launch_valu_tiles<OP>(ctx, grid, a, mode, argmin);
 }
 
 // grid: query tiles x row splits, enough workgroups to fill 256 CUs (argmin
@@ -400,23 +534,28 @@ void launch_flat(vsk_ctx *ctx, FlatArgs a, int mode, int32_t *argmin) {
   splits = ceil_div(rows, a.rows_per_split);
   if (qt > 0x7FFFFFFF) fail(VSK_ERR_INVALID_BUFFER_SIZE, "too many queries");
   dim3 grid((unsigned)qt, (unsigned)splits);
-  const bool valu = a.metric == VSK_METRIC_L1 || a.metric == VSK_METRIC_HAMMING ||
-                    a.metric >= METRIC_L2_EXACT;
+  const bool valu = metric_is_valu(a.metric);
   static const char *names[2][4] = {
       {"flat_mfma_dense", "flat_mfma_filter", "flat_mfma_matrix", "flat_mfma_argmin"},
       {"flat_valu_dense", "flat_valu_filter", "flat_valu_matrix", "flat_valu_argmin"}};
   const char *name = names[valu ? 1 : 0][mode];
   KernelTimer t(ctx, name, (double)a.nq * (double)rows);
   if (valu) {
-    const bool small = mode != MODE_ARGMIN && qt * splits < 4 * (int64_t)ctx->cu_count;
+    // up to 64 queries, or fewer than 4 tiles a CU: the stream over the rows
+    // (at 64 queries the two take the same time over 100,000 x 768, 346 and
+    // 355 us; at 128 the tiles need 501, the stream 529)
+    // (a grid of at most 2^25 waves)
+    const bool stream = mode != MODE_ARGMIN &&
+                        (a.nq <= 64 || qt * splits < 4 * (int64_t)ctx->cu_count) &&
+                        ceil_div(rows, 64) * ceil_div(a.nq, 8) <= 1 << 25;
     switch (a.metric) {
-    case VSK_METRIC_L1: launch_valu_sized<OP_L1>(ctx, a, mode, argmin, small); break;
-    case VSK_METRIC_HAMMING: launch_valu_sized<OP_HAM>(ctx, a, mode, argmin, small); break;
-    case METRIC_L2_EXACT: launch_valu_sized<OP_L2SEQ>(ctx, a, mode, argmin, small); break;
-    case METRIC_L2SQ_EXACT: launch_valu_sized<OP_L2SQSEQ>(ctx, a, mode, argmin, small); break;
-    case METRIC_CN_EXACT: launch_valu_sized<OP_CNSEQ>(ctx, a, mode, argmin, small); break;
-    case METRIC_DOT_EXACT: launch_valu_sized<OP_DOTSEQ>(ctx, a, mode, argmin, small); break;
-    case METRIC_COS_EXACT: launch_valu_sized<OP_COSSEQ>(ctx, a, mode, argmin, small); break;
+    case VSK_METRIC_L1: launch_exact<OP_L1>(ctx, grid, a, mode, argmin, stream); break;
+    case VSK_METRIC_HAMMING: launch_exact<OP_HAM>(ctx, grid, a, mode, argmin, stream); break;
+    case METRIC_L2_EXACT: launch_exact<OP_L2SEQ>(ctx, grid, a, mode, argmin, stream); break;
+    case METRIC_L2SQ_EXACT: launch_exact<OP_L2SQSEQ>(ctx, grid, a, mode, argmin, stream); break;
+    case METRIC_CN_EXACT: launch_exact<OP_CNSEQ>(ctx, grid, a, mode, argmin, stream); break;
+    case METRIC_DOT_EXACT: launch_exact<OP_DOTSEQ>(ctx, grid, a, mode, argmin, stream); break;
+    case METRIC_COS_EXACT: launch_exact<OP_COSSEQ>(ctx, grid, a, mode, argmin, stream); break;
     default: fail(VSK_ERR_INVALID_ARGUMENT, "no exact kernel for this metric");
     }
   } else {
@@ -468,8 +607,7 @@ float *q_aux(vsk_ctx *ctx, const float *dq, int64_t nq, int32_t d, int32_t ld,
 }
 
 static bool use_bf16x3(const vsk_ctx *ctx, int32_t metric) {
-  return !ctx->flat_fp32 && metric != VSK_METRIC_L1 && metric != VSK_METRIC_HAMMING &&
-         metric < METRIC_L2_EXACT;
+  return !ctx->flat_fp32 && !metric_is_valu(metric);
 }
 
 SplitPtrs make_split(vsk_ctx *ctx, const vsk_db *db, const float *dq,
@@ -543,13 +681,25 @@ bool flat_topk_device(vsk_ctx *ctx, const vsk_db *db, const float *dq,
 void approx_topk(vsk_ctx *ctx, const vsk_db *db, const float *dq, int64_t nq,
                  int32_t k, int32_t metric, uint64_t *best, int passes,
                  float *qnh, float *qnr, int64_t max_growth) {
-  const int64_t cap = passes == 1 ? screen_cap(k) : default_cap(k);
+  int64_t cap = passes == 1 ? screen_cap(k) : default_cap(k);
+  // few queries by the exact scan: every row's key in one dense chunk, which
+  // saves a second scan and selection (a first chunk of cap rows fills a
+  // fraction of the chip: 100,000 x 768, one query, 93 of 253 us went there);
+  // where the keys, written and read, are no more traffic than the rows, and
+  // up to 32 MB of them, so that they stay in the memory-side cache
+  if (passes != 1 && metric_is_valu(metric) && k <= VSK_SPLIT_K && cap < db->n &&
+      4 * nq <= db->ld && nq * db->n <= (int64_t)1 << 22 &&
+      (ctx->max_tile_bytes <= 0 || nq * db->n * 8 <= ctx->max_tile_bytes))
+    cap = db->n;
   const int64_t qb = query_batch(ctx, nq, cap);
   for (int64_t b0 = 0; b0 < nq; b0 += qb) {
     const int64_t nb = nq - b0 < qb ? nq - b0 : qb;
     const float *qbat = dq + b0 * db->ld;
     if (metric == METRIC_COS_EXACT) ensure_seq_norms(ctx, db);
-    float *qa = q_aux(ctx, qbat, nb, db->d, db->ld, metric);
+    // (a single query's cosine norm is summed by its scan)
+    float *qa = metric == METRIC_COS_EXACT && nb == 1
+                    ? nullptr
+                    : q_aux(ctx, qbat, nb, db->d, db->ld, metric);
     FlatArgs base{};
     base.X = db->x.as<float>();
     base.ldx = db->ld;
@@ -572,6 +722,7 @@ void approx_topk(vsk_ctx *ctx, const vsk_db *db, const float *dq, int64_t nq,
       a.thresh = r.thresh;
       a.active = r.active;
       a.cand = r.cand;
+      a.words = r.cand32;
       a.cap = r.cap;
       a.counts = r.counts;
       if (x3 && passes == 1) {
@@ -585,7 +736,7 @@ void approx_topk(vsk_ctx *ctx, const vsk_db *db, const float *dq, int64_t nq,
         launch_flat(ctx, a, r.dense ? MODE_DENSE : MODE_FILTER, nullptr);
     };
     progressive_topk(ctx, nb, db->n, k, cap, scan, best + b0 * k,
-                     "flat_select", max_growth);
+                     "flat_select", max_growth, nullptr, passes != 1 && metric_is_valu(metric));
   }
 }
 
@@ -762,8 +913,6 @@ vsk_status vsk_distances(vsk_ctx *ctx, const vsk_db *db, const float *q,
   a.ldx = db->ld;
   a.Q = dq;
   a.ldq = db->ld;
-  a.xaux = x_aux(db, metric);
-  a.qaux = q_aux(ctx, dq, nq, db->d, db->ld, metric);
   a.kdim = db->ld;
   a.nq = (int32_t)nq;
   a.r0 = 0;
@@ -780,13 +929,14 @@ vsk_status vsk_distances(vsk_ctx *ctx, const vsk_db *db, const float *q,
   // bit for bit, and exactly symmetric when the rows are the queries.
   if (exact_metric(metric) >= 0) {
     a.metric = exact_metric(metric);
-    a.xaux = nullptr;
-    a.qaux = nullptr;
     if (metric == VSK_METRIC_COSINE) {
       ensure_seq_norms(ctx, db);
       a.xaux = x_aux(db, METRIC_COS_EXACT);
-      a.qaux = q_aux(ctx, dq, nq, db->d, db->ld, METRIC_COS_EXACT);
+      if (nq > 1) a.qaux = q_aux(ctx, dq, nq, db->d, db->ld, METRIC_COS_EXACT);
     }
+  } else {
+    a.xaux = x_aux(db, metric);
+    a.qaux = q_aux(ctx, dq, nq, db->d, db->ld, metric);
   }
   if (use_bf16x3(ctx, a.metric))
     launch_flat_bf16x3(ctx, a, make_split(ctx, db, dq, nq, true, nullptr, nullptr),

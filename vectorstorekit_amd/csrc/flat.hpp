@@ -56,6 +56,8 @@ struct FlatArgs {
   const uint64_t *thresh;
   const uint8_t *active;
   uint64_t *cand;
+  // exact scan, dense mode: 32-bit ordered distances here instead of keys
+  uint32_t *words;
   int64_t cap;
   int32_t *counts;
   float *mat;  // MODE_MATRIX output, row-major nq x ldm

@@ -23,11 +23,12 @@ namespace vsk {
 constexpr int SEL_THREADS = 256;
 
 // element i of a query's keys: the previous list, then the candidates --
-// 64-bit keys, or (W32) 32-bit distances keyed by their index in the list
+// 64-bit keys, or (W32) 32-bit distances keyed by their index in the list,
+// counted from i0
 template <bool W32>
 __device__ inline uint64_t sel_elem(const uint64_t *P, int64_t np, const uint64_t *C,
-                                    const uint32_t *C32, int64_t i) {
-  if constexpr (W32) return ((uint64_t)C32[i] << 32) | (uint32_t)i;
+                                    const uint32_t *C32, uint32_t i0, int64_t i) {
+  if constexpr (W32) return ((uint64_t)C32[i] << 32) | (i0 + (uint32_t)i);
   return i < np ? P[i] : C[i - np];
 }
 
@@ -229,6 +230,7 @@ __device__ void wave_sort_u64(uint64_t (&v)[R]) {
 // cost occupancy, which launches of many queries need more.
 template <int REG, bool W32, bool FAST = false, int SEGB = 0>
 __global__ __launch_bounds__(SEL_THREADS) void k_select(SelectArgs a) {
+  // (a split selection's output list: run q % split_n of query q / split_n)
   const int64_t q = blockIdx.x;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -240,6 +242,13 @@ __global__ __launch_bounds__(SEL_THREADS) void k_select(SelectArgs a) {
   int64_t base = a.seg_off ? a.seg_off[q] : q * a.cap;
   int64_t cnt = a.counts ? (int64_t)a.counts[q]
                          : (a.seg_off ? a.seg_off[q + 1] - base : a.cap);
+  uint32_t i0 = 0;
+  if (a.split_len > 0) {
+    const int64_t sn = (a.cap + a.split_len - 1) / a.split_len, s0 = q % sn * a.split_len;
+    base = q / sn * a.cap + s0;
+    i0 = (uint32_t)s0;
+    cnt = a.cap - s0 < a.split_len ? a.cap - s0 : a.split_len;
+  }
   bool overflow = false;
   if (a.counts && !a.seg_off && cnt > a.cap) {
     overflow = true;
@@ -264,23 +273,34 @@ __global__ __launch_bounds__(SEL_THREADS) void k_select(SelectArgs a) {
     __syncthreads();
   }
   const bool inreg = REG > 0 && !seg && total <= (int64_t)REG * SEL_THREADS;  // uniform
-  uint64_t regs[REG > 0 ? REG : 1];
+  // (W32: the 32-bit distances; their keys are made again on each pass)
+  std::conditional_t<W32, uint32_t, uint64_t> regs[REG > 0 ? REG : 1];
   if (inreg) {
 #pragma unroll
     for (int r = 0; r < REG; ++r) {
       const int64_t i = tid + (int64_t)r * SEL_THREADS;
-      regs[r] = i < total ? sel_elem<W32>(P, np, C, C32, i) : VSK_KEY_NONE;
+      if constexpr (W32)
+        regs[r] = i < total ? C32[i] : 0;
+      else
+        regs[r] = i < total ? sel_elem<W32>(P, np, C, C32, i0, i) : VSK_KEY_NONE;
     }
   }
   auto each_key = [&](auto &&f) {
     if (inreg) {
 #pragma unroll
-      for (int r = 0; r < REG; ++r)
-        if (tid + (int64_t)r * SEL_THREADS < total) f(regs[r]);
+      for (int r = 0; r < REG; ++r) {
+        const uint32_t i = (uint32_t)(tid + r * SEL_THREADS);
+        if (i >= total) continue;
+        if constexpr (W32)
+          f(((uint64_t)regs[r] << 32) | (i0 + i));
+        else
+          f(regs[r]);
+      }
       return;
     }
     if (!seg) {
-      for (int64_t i = tid; i < total; i += SEL_THREADS) f(sel_elem<W32>(P, np, C, C32, i));
+      for (int64_t i = tid; i < total; i += SEL_THREADS)
+        f(sel_elem<W32>(P, np, C, C32, i0, i));
       return;
     }
     for (int64_t i = tid; i < np; i += SEL_THREADS) f(P[i]);
@@ -1531,12 +1551,28 @@ void launch_select(vsk_ctx *ctx, const SelectArgs &a, const char *name) {
     check_launch(name);
     return;
   }
+  if (a.split_len > 0) {
+    if (a.prev || a.counts || a.seg_off || a.seg_n || a.active || a.thresh ||
+        a.k > VSK_SPLIT_K || a.split_len > 8 * SEL_THREADS)
+      fail(VSK_ERR_INVALID_ARGUMENT, "a split selection takes plain dense lists");
+    const int64_t blocks = a.nq * ceil_div(a.cap, a.split_len);
+    if (blocks > 0x7FFFFFFF) fail(VSK_ERR_INVALID_BUFFER_SIZE, "grid too large");
+    if (a.cand32)
+      k_select<8, true, true><<<(unsigned)blocks, SEL_THREADS, 0, ctx->stream>>>(a);
+    else
+      k_select<8, false, true><<<(unsigned)blocks, SEL_THREADS, 0, ctx->stream>>>(a);
+    check_launch(name);
+    return;
+  }
   // keys per query: the previous list (k) and up to cap candidates
   const int64_t most = a.cap + (a.prev ? a.k : 0);
   const bool fast = a.k <= 128 && !a.seg_n;
   if (a.cand32) {
     if (a.prev || a.seg_n) fail(VSK_ERR_INVALID_ARGUMENT, "32-bit lists take no previous list or segments");
-    k_select<32, true><<<(unsigned)a.nq, SEL_THREADS, 0, ctx->stream>>>(a);
+    if (a.k <= 128)
+      k_select<64, true, true><<<(unsigned)a.nq, SEL_THREADS, 0, ctx->stream>>>(a);
+    else
+      k_select<64, true><<<(unsigned)a.nq, SEL_THREADS, 0, ctx->stream>>>(a);
   } else if (a.regs && !a.seg_off && most > 32 * SEL_THREADS) {
     if (fast)
       k_select<64, false, true><<<(unsigned)a.nq, SEL_THREADS, 0, ctx->stream>>>(a);
@@ -1587,7 +1623,7 @@ int64_t tile_keys(const vsk_ctx *ctx, int64_t keys, int64_t bytes_per_key) {
 void progressive_topk(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t k,
                       int64_t cap, const ScanFn &scan, uint64_t *best,
                       const char *select_name, int64_t max_growth,
-                      const TopkWorkspace *ws) {
+                      const TopkWorkspace *ws, bool words) {
   if (nq <= 0) return;
   if (n <= 0) {
     fill_u64(ctx, best, nq * (int64_t)k, VSK_KEY_NONE);
@@ -1646,6 +1682,7 @@ void progressive_topk(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t k,
     int64_t seg_stride = 0;
     {
       ScanRequest rq{r0, r0 + c, thresh, nullptr, cand, cap, counts, dense};
+      if (words && dense && c >= n) rq.cand32 = reinterpret_cast<uint32_t *>(cand);
       if (!dense && seg_n) {
         rq.seg_n = seg_n;
         rq.seg_nseg = &nseg;
@@ -1658,6 +1695,7 @@ void progressive_topk(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t k,
     sa.k = k;
     sa.prev = dense ? nullptr : best;
     sa.cand = cand;
+    if (words && dense && c >= n) sa.cand32 = reinterpret_cast<const uint32_t *>(cand);
     sa.cap = cap;
     sa.counts = dense ? nullptr : counts;
     sa.best_out = best;
@@ -1667,6 +1705,24 @@ void progressive_topk(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t k,
     // small dense lists (IVF probing over the centroids, small problems)
     // are read into registers once
     sa.regs = dense && cap <= 64 * SEL_THREADS;  // (no previous list)
+    // A whole database in one dense chunk too long for that: runs of 2,048
+    // keys by a workgroup each, then their winners (one workgroup over
+    // 100,000 keys reads the list four or five times, at one CU's rate).
+    if (dense && c >= n && !sa.regs && !ws && k <= VSK_SPLIT_K) {
+      const int32_t len = 8 * SEL_THREADS;
+      const int64_t runs = ceil_div(cap, len);
+      SelectArgs sp = sa;
+      sp.split_len = len;
+      sp.thresh = nullptr;
+      sp.regs = false;
+      sp.best_out = static_cast<uint64_t *>(
+          ctx->scratch_ptr("topk.runs", sizeof(uint64_t) * (size_t)(nq * runs * k)));
+      launch_select(ctx, sp, select_name);
+      sa.cand = sp.best_out;
+      sa.cand32 = nullptr;
+      sa.cap = runs * k;
+      sa.regs = sa.cap <= 64 * SEL_THREADS;
+    }
     if (!dense) {
       if (defer) {
         // (the mask is written, never read)

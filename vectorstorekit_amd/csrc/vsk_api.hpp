@@ -58,7 +58,7 @@ struct SelectArgs {
   const uint64_t *prev = nullptr;
   const uint64_t *cand = nullptr;
   // 32-bit distances instead of cand (no prev): key = (value << 32) | the
-  // value's index in its query's list
+  // value's index in its query's list (of cap, also in a split selection)
   const uint32_t *cand32 = nullptr;
   int64_t cap = 0;
   const int64_t *seg_off = nullptr;
@@ -82,7 +82,14 @@ struct SelectArgs {
   // thresh a key T with exactly those k keys <= T (a chunk's list that only
   // the next chunk's selection reads)
   bool sorted = true;
+  // > 0: lists of cap keys taken in runs of split_len by a workgroup each:
+  // output (query q, run s) is the k smallest of its run, sorted, at
+  // best_out[(q * split_n + s) * k] (split_n = ceil(cap / split_len); no
+  // counts, previous list, segments or thresholds)
+  int32_t split_len = 0;
 };
+// the largest k of a split selection
+constexpr int32_t VSK_SPLIT_K = 128;
 void launch_select(vsk_ctx *ctx, const SelectArgs &a, const char *name);
 
 // maximum segments per query of a segmented scan
@@ -106,6 +113,10 @@ struct ScanRequest {
   int32_t *seg_n = nullptr;
   int32_t *seg_nseg = nullptr;
   int64_t *seg_stride = nullptr;
+  // set (instead of cand) where a dense chunk holds the whole database and
+  // the caller's scan takes it (progressive_topk's words): 32-bit ordered
+  // distances, row r's at cand32[q*cap + r]
+  uint32_t *cand32 = nullptr;
 };
 using ScanFn = std::function<void(const ScanRequest &)>;
 
@@ -129,11 +140,13 @@ struct TopkWorkspace {
 // holds at most cap/(2k) times the rows already seen, and at most max_growth
 // times when that is positive.
 // ws: the buffers to use (sized for nq and min(cap, n)); null = the
-// context's scratch slots.
+// context's scratch slots.  words: a dense chunk of every row may be asked
+// for as 32-bit distances (half the bytes written and selected from; the
+// row is the position).
 void progressive_topk(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t k,
                       int64_t cap, const ScanFn &scan, uint64_t *best,
                       const char *select_name, int64_t max_growth = 0,
-                      const TopkWorkspace *ws = nullptr);
+                      const TopkWorkspace *ws = nullptr, bool words = false);
 
 // candidate buffer capacity per query used by the progressive scans
 int64_t default_cap(int32_t k);
