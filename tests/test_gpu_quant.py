@@ -166,6 +166,41 @@ def test_pq_encode_codebook_layouts(ctx, shape):
     np.testing.assert_array_equal(pq.encode(x), O.pq_encode(x, cb))
 
 
+@pytest.mark.parametrize("dsub", [4, 8, 16])
+@pytest.mark.parametrize("M,ksub", [(1, 129), (3, 256), (5, 200), (16, 256)])
+def test_pq_encode_matrix_cores_bit_exact(ctx, M, ksub, dsub):
+    """The matrix-core encoder at the edges of its 64-row waves and of its
+    16-codeword tiles, on data its screen cannot decide: codewords in exact
+    and near ties (the lower index, the smaller fp32 sum), rows on codewords,
+    a large common offset, magnitudes of 1e-25 and 1e25, zeros, infinities
+    and NaN, and rows that start at 4 bytes past an aligned address."""
+    import torch
+
+    rng = np.random.default_rng(M + ksub + dsub)
+    for n, offset, scale in [(1, 0, 1), (63, 0, 1), (65, 100, 1), (1000, 0, 1), (700, 0, 1e-25),
+                             (500, 0, 1e25), (300, 1e4, 1)]:
+        cb = rng.standard_normal((M, ksub, dsub)).astype(np.float32) + np.float32(offset)
+        cb[:, 7] = cb[:, 3]  # exact ties
+        cb[:, 100] = cb[:, 50] * np.float32(1 + 2e-7)
+        x = rng.standard_normal((n, M * dsub)).astype(np.float32) + np.float32(offset)
+        x[::5] = cb[:, rng.integers(0, ksub, len(x[::5]))].transpose(1, 0, 2).reshape(-1, M * dsub)
+        x[1::9] = np.tile(cb[:, 50].reshape(-1), (len(x[1::9]), 1))
+        cb, x = cb * np.float32(scale), x * np.float32(scale)
+        x[2::50] = 0
+        if n == 1000:
+            x[10, ::3], x[20, 1], x[30] = np.inf, np.nan, -np.inf
+        print(f"pq encode M={M} ksub={ksub} dsub={dsub} n={n} scale={scale}", flush=True)
+        with np.errstate(all="ignore"):
+            want = O.pq_encode(x, cb)
+        pq = ProductQuantizer(ctx, cb)
+        np.testing.assert_array_equal(pq.encode(x), want)
+        flat = torch.zeros(1 + x.size, device="cuda")
+        flat[1:] = torch.from_numpy(x).reshape(-1)
+        torch.cuda.synchronize()
+        got = pq.encode(flat[1:].view(n, M * dsub))
+        np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("metric", [METRIC_L1, METRIC_L2, METRIC_L2SQ, METRIC_COSINE])
 def test_pq_rerank_bit_exact(ctx, metric):
     x, q, cb = _pq_data(5, 30_000, 64, 8, 256, 20)

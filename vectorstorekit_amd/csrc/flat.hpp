@@ -357,6 +357,16 @@ bool screen_finish(vsk_ctx *ctx, const vsk_db *db, const float *dq, int32_t k,
 void segmented_sort_u64(vsk_ctx *ctx, const uint64_t *in, uint64_t *out, int64_t nseg,
                         int64_t len);
 
+// The matrix-core PQ encoder (pq_encode.hip): whether it takes a codebook
+// shape, the operand image of M such codebooks (made once per quantizer), and
+// the codes of n rows (x: n x M dsub fp32 on the device)
+bool pq_encode_mfma_applies(int32_t ksub, int32_t dsub);
+size_t pq_encode_operand_bytes(int32_t M, int32_t dsub);
+void pq_encode_operands(vsk_ctx *ctx, const float *cb, int32_t M, int32_t ksub, int32_t dsub,
+                        void *ops);
+void pq_encode_mfma(vsk_ctx *ctx, const float *x, int64_t n, const float *cb, void *ops,
+                    int32_t M, int32_t ksub, int32_t dsub, uint8_t *codes);
+
 // a PQ quantizer's shape for other translation units: returns d
 int32_t pq_shape(const vsk_pq *pq, int32_t *M, int32_t *ksub);
 bool pq_shape_matches(const vsk_pq *pq, int32_t d, int32_t M, int32_t ksub);

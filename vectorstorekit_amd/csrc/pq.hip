@@ -29,6 +29,7 @@
 struct vsk_pq {
   int32_t M = 0, ksub = 0, dsub = 0, d = 0;
   vsk::DevBuf codebooks;  // M x ksub x dsub fp32
+  vsk::DevBuf enc_ops;    // their matrix-core encoder operands, where it applies
   std::vector<float> host_codebooks;  // the same, for identity checks and files
   vsk::DevBuf codes;      // n x M uint8
   int64_t n = 0, cap_rows = 0;
@@ -209,7 +210,10 @@ static void launch_encode(vsk_ctx *ctx, const vsk_pq *pq, const float *dx,
                           int64_t n, uint8_t *codes) {
   const size_t lds = sizeof(float) * (size_t)pq->ksub * pq->dsub;
   KernelTimer t(ctx, "pq_encode", (double)n * pq->M);
-  if (lds <= 64 * 1024) {
+  if (pq->enc_ops.p) {
+    pq_encode_mfma(ctx, dx, n, pq->codebooks.as<float>(), pq->enc_ops.p, pq->M, pq->ksub,
+                   pq->dsub, codes);
+  } else if (lds <= 64 * 1024) {
     int64_t bx = ceil_div(n, 256);
     if (bx > 2048) bx = 2048;
     dim3 grid((unsigned)bx, (unsigned)pq->M);
@@ -1028,6 +1032,10 @@ vsk_status vsk_pq_create(vsk_ctx *ctx, const float *codebooks, int32_t M,
   pq->host_codebooks.resize((size_t)M * ksub * dsub);
   VSK_HIP(hipMemcpyAsync(pq->host_codebooks.data(), pq->codebooks.p, bytes,
                          hipMemcpyDeviceToHost, ctx->stream));
+  if (pq_encode_mfma_applies(ksub, dsub)) {
+    pq->enc_ops.reserve(pq_encode_operand_bytes(M, dsub));
+    pq_encode_operands(ctx, pq->codebooks.as<float>(), M, ksub, dsub, pq->enc_ops.p);
+  }
   cs.finish();
   *out = pq.release();
   VSK_API_END(ctx);
