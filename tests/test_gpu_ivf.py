@@ -266,6 +266,42 @@ def test_ivf_build_one_call_matches_create_add(ctx):
     assert (i == -1).all() and np.isinf(d).all()
 
 
+@pytest.mark.parametrize("shape", [(1, 9, 4, 3, 1, 12), (64, 900, 33, 5, 9, 100),
+                                   (300, 20_000, 128, 40, 20, 10), (17, 4000, 300, 7, 17, 64)])
+def test_ivf_ungrouped_scan_bit_exact(ctx, shape):
+    """The list scan without groups (few terms): lists around its 64-row
+    waves, empty lists, columns around its 64-column chunks, fewer candidates
+    than k, a far row (infinite L2^2), both metrics, and a row filter; and an index of
+    one long and many short lists, which is grouped."""
+    nlist, n, d, nq, nprobe, k = shape
+    x, q, c = _mixture(nlist + d, nlist, n, d, nq)
+    x[n // 2, d - 1] = 1e30
+    for skew in (False, True):
+        if skew:
+            x = x.copy()
+            x[:] = x[0] + np.float32(1e-3) * np.arange(n, dtype=np.float32)[:, None]
+        print(f"ivf ungrouped {shape} skew={skew}", flush=True)
+        idx = _index(ctx, c, x, nprobe=nprobe)
+        lists = O.ivf_assign(x, c)
+        for metric in ("euclidean", "euclideanSquared"):
+            gd, gi = idx.search(q, k, metric=metric)
+            od, oi = O.ivf_search(q, x, np.arange(n), lists, c, nprobe, k,
+                                  squared=metric == "euclideanSquared")
+            np.testing.assert_array_equal(gi, oi)
+            np.testing.assert_array_equal(gd, od)
+        allow = np.arange(n) % 3 == 1
+        gd, gi = idx.search(q, k, allow=allow)
+        od, oi = O.ivf_search(q, x, np.arange(n), lists, c, nprobe, n)
+        for i in range(nq):
+            keep = (oi[i] >= 0) & allow[oi[i]]
+            want = np.full(k, -1, np.int64)
+            m = min(k, int(keep.sum()))
+            want[:m] = oi[i][keep][:m]
+            np.testing.assert_array_equal(gi[i], want)
+            np.testing.assert_array_equal(gd[i, :m], od[i][keep][:m])
+            assert np.isinf(gd[i, m:]).all()
+
+
 def test_ivf_squared_metric_bit_exact(ctx):
     x, q, c = _mixture(12, 48, 12_000, 64, 60)
     ids = np.arange(len(x), dtype=np.int64)

@@ -209,12 +209,25 @@ void launch_screen_tail(vsk_ctx *ctx, const ScreenTailArgs &a, const char *name)
 // ascending into best_out[q * k ...] (NONE past the words): query q's words
 // are words[wseg[q] + i], i < cnt[q] (wseg a multiple of 4); only queries
 // with active[q] (all when null).  The keys are those of a scan writing
-// (word << 32) | position.
+// (word << 32) | position.  With wseg and cnt null, every query has wstride
+// words (a multiple of 4) at q * wstride.
+// lists (keys set): instead of best_out, the results -- the word as the
+// distance and the stored id of row position % pitch of the list that the
+// query's probe key position / pitch names; (+inf, -1) past the words.
+struct ListResults {
+  const uint64_t *keys = nullptr;
+  int32_t np = 0, pitch = 1;
+  const int64_t *list_off = nullptr, *ids = nullptr;
+  float *out_dist = nullptr;
+  int64_t *out_ids = nullptr;
+};
 struct WordSelectArgs {
   int64_t nq = 0;
   int32_t k = 0;
   const uint32_t *words = nullptr;
   const int64_t *wseg = nullptr, *cnt = nullptr;
+  int64_t wstride = 0;
+  ListResults lists;
   uint64_t *best_out = nullptr;
   const uint8_t *active = nullptr;
 };

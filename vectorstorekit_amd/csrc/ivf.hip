@@ -73,6 +73,10 @@ struct vsk_ivf {
   // per list the largest distance of its rows from its centroid (for the
   // list scan's per-query bound), valid with the plane
   mutable vsk::DevBuf xrad;
+  // top_rows[i]: the rows of the i largest lists together (i <= nlist),
+  // valid while tversion == version
+  mutable std::vector<int64_t> top_rows;
+  mutable int64_t tversion = -1;
 };
 
 namespace vsk {
@@ -569,6 +573,99 @@ __global__ __launch_bounds__(256) void k_list_scan(ListScanArgs a) {
         a.words[obase[j] + i] = vsk_f2ord(a.squared ? acc[j] : sqrtf(acc[j]));
   }
   (void)qidx;
+}
+
+// The exact list scan without groups, for searches whose lists are shared by
+// few queries: a wave per (query, probe slot, 64 rows of its list), the rows
+// streamed through LDS in whole 256-byte segments with the next 64 columns'
+// loads in flight (the flat stream scan's layout), the query's columns staged
+// beside them.  Word i of probe slot p sits at p * pitch + i of the query's
+// np * pitch words (pitch: the longest list, rounded up to 64), which orders
+// candidates as their positions do; slots past a list's end, missing probes
+// and rows the filter excludes read kWordNone.  One thread a row over groups
+// of up to 16 queries, with the pairs grouped by list first, took five more
+// launches and 26 us for one query's 10 lists of 195 rows x 128; this scan
+// takes 5 us.
+struct DirectScanArgs {
+  const float *rows, *Q;
+  int32_t ld, np, pitch, squared;
+  const uint64_t *keys;  // the probes' ranked keys, np a query
+  const int64_t *list_off;
+  const uint32_t *lmask;
+  uint32_t *words;
+};
+__global__ __launch_bounds__(64) void k_list_stream(DirectScanArgs a) {
+#pragma clang fp contract(off)
+  constexpr int C = 64, LD = C + 4;
+  __shared__ __attribute__((aligned(16))) float tile[64 * LD];
+  __shared__ __attribute__((aligned(16))) float qt[C];
+  const int lane = threadIdx.x;
+  const int32_t tiles = a.pitch / 64;
+  const int64_t pair = blockIdx.x / tiles, q = pair / a.np;
+  const int32_t i0 = (int32_t)(blockIdx.x - pair * tiles) * 64;
+  const uint64_t key = a.keys[pair];
+  uint32_t *out = a.words + pair * a.pitch + i0 + lane;
+  int64_t v0 = 0, len = 0;
+  if (key != VSK_KEY_NONE) {
+    const int32_t l = (int32_t)(uint32_t)key;
+    v0 = a.list_off[l];
+    len = a.list_off[l + 1] - v0;
+  }
+  if (i0 >= len) {
+    *out = kWordNone;
+    return;
+  }
+  const int seg = lane & 15, sub = lane >> 4;
+  const int64_t last = len - 1 - i0;  // rows past the end read the last one
+  const float *src[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int64_t r = sub + 4 * i;
+    src[i] = a.rows + (v0 + i0 + (r < last ? r : last)) * a.ld;
+  }
+  const float *qq = a.Q + q * a.ld;
+  const int32_t cmax = a.ld - 4;  // a segment past the row end is clamped
+  f4 buf[16], qbuf;
+  auto load = [&](int32_t c0) {
+    const int32_t col = c0 + 4 * seg < cmax ? c0 + 4 * seg : cmax;
+    qbuf = *reinterpret_cast<const f4 *>(qq + col);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) buf[i] = *reinterpret_cast<const f4 *>(src[i] + col);
+  };
+  float s = 0.f;
+  load(0);
+  for (int32_t k0 = 0; k0 < a.ld; k0 += C) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      *reinterpret_cast<f4 *>(tile + (sub + 4 * i) * LD + 4 * seg) = buf[i];
+    if (sub == 0) *reinterpret_cast<f4 *>(qt + 4 * seg) = qbuf;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (k0 + C < a.ld) load(k0 + C);
+    const float *xr = tile + lane * LD;
+    const int32_t kn = a.ld - k0 < C ? a.ld - k0 : C;
+#pragma unroll 4
+    for (int32_t k = 0; k < kn; k += 4) {
+      const f4 xv = *reinterpret_cast<const f4 *>(xr + k);
+      const f4 qv = *reinterpret_cast<const f4 *>(qt + k);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const float t = qv[c] - xv[c];
+        s = s + t * t;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  uint32_t word = kWordNone;
+  if (lane <= last) {
+    const int64_t v = v0 + i0 + lane;
+    if (!a.lmask || ((a.lmask[v >> 5] >> (v & 31)) & 1u))
+      word = vsk_f2ord(a.squared ? s : sqrtf(s));
+  }
+  *out = word;
 }
 
 // IVF-PQ list scan: ADC sum = sum over segments m, in order, of
@@ -1240,13 +1337,17 @@ static bool list_screen_applies(vsk_ctx *ctx, const vsk_ivf *ivf, int32_t metric
 // candidates a query can have with np probes: the sizes of the np largest
 // lists summed (every row when every list is probed)
 static int64_t probe_bound(const vsk_ivf *ivf, int32_t np) {
-  if (np >= ivf->nlist) return ivf->total;
-  std::vector<int64_t> sz(ivf->nlist);
-  for (int32_t l = 0; l < ivf->nlist; ++l) sz[l] = ivf->off[l + 1] - ivf->off[l];
-  std::nth_element(sz.begin(), sz.begin() + np, sz.end(), std::greater<int64_t>());
-  int64_t s = 0;
-  for (int32_t i = 0; i < np; ++i) s += sz[i];
-  return s;
+  if (ivf->tversion != ivf->version) {
+    // (sorted once per change of the rows: 10 us at 1,024 lists, which a
+    // search of one query would notice)
+    std::vector<int64_t> sz(ivf->nlist);
+    for (int32_t l = 0; l < ivf->nlist; ++l) sz[l] = ivf->off[l + 1] - ivf->off[l];
+    std::sort(sz.begin(), sz.end(), std::greater<int64_t>());
+    ivf->top_rows.assign(ivf->nlist + 1, 0);
+    for (int32_t l = 0; l < ivf->nlist; ++l) ivf->top_rows[l + 1] = ivf->top_rows[l] + sz[l];
+    ivf->tversion = ivf->version;
+  }
+  return ivf->top_rows[np < ivf->nlist ? np : ivf->nlist];
 }
 
 // the stored rows' bf16 plane (roundup(d, 64) columns), |x|^2 per row and
@@ -1953,6 +2054,68 @@ static void probe_screen(vsk_ctx *ctx, const vsk_ivf *ivf, const float *dq, int6
 // query codes; 2: PQ codes, qextra = the vsk_pq whose tables score them
 // allow (may be null): the row filter, a bitmap over the stored rows' ids
 // of allow_bits bits (k_allow_list_bits)
+// Whether a search scans its lists without grouping queries by list.  The
+// ungrouped scan reads a list once per query that probes it (from the L2
+// after the first) but needs no grouping launches, and its waves are many and
+// short.  Measured (us, ungrouped and grouped): 200,000 x 128 in 1,024 lists,
+// 10 probes: 1 query 45 and 83, 256 queries (6e7 terms) 76 and 110, 1,000
+// (2.5e8) 156 and 146; 1M x 128, 4,096 lists, 32 probes: 256 queries (2 a
+// list, 2.6e8) 234 and 282, 1,000 (8 a list) 679 and 412; 200,000 x 768, 512
+// lists, 16 probes: 64 queries (2 a list, 3e8) 231 and 381, 256 (8 a list)
+// 717 and 492.  So: up to 2^27 terms, or 2^29 with at most four queries a
+// list.  Words are laid out by the longest list, so skewed lists (twice the
+// words) are grouped too.
+static bool direct_applies(const vsk_ivf *ivf, int64_t nq, int32_t np, int64_t pitch) {
+  const double terms = (double)nq * np * ((double)ivf->total / ivf->nlist) * ivf->ld;
+  if (pitch <= 0 || np * pitch > 2 * probe_bound(ivf, np) + 4096) return false;
+  return terms <= 0x1p27 || (terms <= 0x1p29 && nq * np <= 4 * (int64_t)ivf->nlist);
+}
+
+// the ungrouped list scan of all queries, and one selection that writes the
+// results (no position bases, no offsets, no decoding launch)
+static void direct_search(vsk_ctx *ctx, const vsk_ivf *ivf, const float *dq, int64_t nq,
+                          int32_t np, int32_t pitch, int32_t k, bool squared,
+                          const uint64_t *keys, const uint32_t *lmask, float *out_dist,
+                          int64_t *out_ids) {
+  const int64_t stride = (int64_t)np * pitch;
+  const int64_t qb = std::max<int64_t>(
+      1, std::min<int64_t>(nq, tile_keys(ctx, (int64_t)1 << 26, 4) / stride));
+  uint32_t *words = static_cast<uint32_t *>(
+      ctx->scratch_ptr("ivf.direct", sizeof(uint32_t) * (size_t)(qb * stride)));
+  for (int64_t b0 = 0; b0 < nq; b0 += qb) {
+    const int64_t nb = nq - b0 < qb ? nq - b0 : qb;
+    DirectScanArgs a;
+    a.rows = ivf->rows.as<float>();
+    a.Q = dq + b0 * ivf->ld;
+    a.ld = ivf->ld;
+    a.np = np;
+    a.pitch = pitch;
+    a.squared = squared ? 1 : 0;
+    a.keys = keys + b0 * np;
+    a.list_off = ivf->list_off.as<int64_t>();
+    a.lmask = lmask;
+    a.words = words;
+    {
+      KernelTimer t(ctx, "ivf_list_scan");
+      k_list_stream<<<(unsigned)(nb * np * (pitch / 64)), 64, 0, ctx->stream>>>(a);
+      check_launch("ivf_list_scan");
+    }
+    WordSelectArgs sa;
+    sa.nq = nb;
+    sa.k = k;
+    sa.words = words;
+    sa.wstride = stride;
+    sa.lists.keys = a.keys;
+    sa.lists.np = np;
+    sa.lists.pitch = pitch;
+    sa.lists.list_off = a.list_off;
+    sa.lists.ids = ivf->ids.as<int64_t>();
+    sa.lists.out_dist = out_dist + b0 * k;
+    sa.lists.out_ids = out_ids + b0 * k;
+    launch_select_words(ctx, sa, "ivf_select");
+  }
+}
+
 static vsk_status ivf_search_any(vsk_ctx *ctx, const vsk_ivf *ivf, const float *q,
                                  const void *qextra, int64_t nq, int32_t nprobe, int32_t k,
                                  int32_t metric, int32_t kind, void *out_dist,
@@ -2054,6 +2217,17 @@ static vsk_status ivf_search_any(vsk_ctx *ctx, const vsk_ivf *ivf, const float *
     ivf_rank_all(ctx, ivf, dq, nq, probes);
   } else {
     ivf_probe_device(ctx, ivf, dq, nq, np, probes, sqp.one.qh ? &sqp.one : nullptr, &pkeys);
+  }
+  if (pkeys && kind == 0 && !screen) {
+    const int64_t pitch = ceil_div(probe_bound(ivf, 1), 64) * 64;
+    if (direct_applies(ivf, nq, np, pitch)) {
+      direct_search(ctx, ivf, dq, nq, np, (int32_t)pitch, k, metric == VSK_METRIC_L2SQ, pkeys,
+                    lmask, od.ptr<float>(), oi.ptr<int64_t>());
+      od.copy_back();
+      oi.copy_back();
+      cs.finish();
+      return VSK_OK;
+    }
   }
   // 2. candidate counts and probe position bases
   int64_t *pos_base = static_cast<int64_t *>(

@@ -1476,7 +1476,10 @@ __global__ __launch_bounds__(SEL_THREADS) void k_select_words(WordSelectArgs a) 
   const int tid = threadIdx.x, lane = tid & 63;
   if (a.active && !a.active[q]) return;
   WordList<REG> L;
-  L.load(a.words + a.wseg[q], a.cnt[q]);
+  if (a.wseg)
+    L.load(a.words + a.wseg[q], a.cnt[q]);
+  else
+    L.load(a.words + q * a.wstride, a.wstride);
   auto each = [&](auto &&f) { L.each(f); };
   __shared__ KthShared sh;
   __shared__ uint64_t sel[VSK_MAX_K];
@@ -1526,6 +1529,22 @@ __global__ __launch_bounds__(SEL_THREADS) void k_select_words(WordSelectArgs a) 
   int m = s_cnt;
   if (m > (int)k) m = (int)k;  // (exactly k, or fewer words in all)
   block_sort(sel, m);
+  if (a.lists.keys) {
+    const ListResults &r = a.lists;
+    for (int i = tid; i < (int)k; i += SEL_THREADS) {
+      float dist = __int_as_float(0x7f800000);
+      int64_t id = -1;
+      if (i < m) {
+        const uint32_t pos = (uint32_t)sel[i], p = pos / (uint32_t)r.pitch;
+        const uint32_t l = (uint32_t)r.keys[q * r.np + p];
+        dist = vsk_ord2f((uint32_t)(sel[i] >> 32));
+        id = r.ids[r.list_off[l] + (pos - p * (uint32_t)r.pitch)];
+      }
+      r.out_dist[q * (int64_t)k + i] = dist;
+      r.out_ids[q * (int64_t)k + i] = id;
+    }
+    return;
+  }
   uint64_t *out = a.best_out + q * (int64_t)k;
   for (int i = tid; i < (int)k; i += SEL_THREADS) out[i] = i < m ? sel[i] : VSK_KEY_NONE;
 }
