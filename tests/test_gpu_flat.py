@@ -298,6 +298,36 @@ def test_stream_scan_edges(ctx, metric):
 
 
 @pytest.mark.parametrize("metric", SCREEN)
+@pytest.mark.parametrize("scale", [2.0 ** -60, 1.0, 2.0 ** 40])
+def test_screen_planes_and_chunks(sctx, metric, scale):
+    """The screen's 16-bit planes and first chunks: values far from 1, rows
+    and queries that differ by 2^20 among themselves, zero rows and zero
+    queries; row tiles that end short (the first chunk's 32-bit distances
+    then one at a time), dimensions around a stage's 64 columns, query counts
+    on both sides of 1,024 (where the chunks' capacity changes), lists that
+    the selection holds in LDS and lists too long for that (k = 600); bit for
+    bit the oracle."""
+    for n, nq, d, k in [(1, 1, 1, 1), (255, 3, 64, 10), (257, 257, 63, 9), (20_003, 40, 65, 30),
+                        (9000, 1024, 130, 20), (9001, 1025, 128, 20), (30_001, 20, 129, 600)]:
+        x, q = _data(n + nq + d, n, nq, d, normalize=metric == METRIC_COSINE_NORMALIZED)
+        if metric != METRIC_COSINE_NORMALIZED:
+            x *= np.float32(scale)
+            q *= np.float32(scale)
+            if n > 300:
+                x[7::50] *= np.float32(2.0 ** -20)
+                x[11::97] = 0
+            if nq > 30:
+                q[5::9] *= np.float32(2.0 ** -20)
+                q[29] = 0
+        print(f"planes metric={metric} scale={scale:g} n={n} nq={nq} d={d} k={k}", flush=True)
+        db = VectorDatabase(sctx, x)
+        gd, gi = db.search(q, k, metric)
+        od, oi = O.search_flat(q, x, k, metric)
+        np.testing.assert_array_equal(gi, oi)
+        np.testing.assert_array_equal(gd, od)
+
+
+@pytest.mark.parametrize("metric", SCREEN)
 def test_small_problem_exact_scan(ctx, metric):
     """Config 1's size (at most 2^28 query x row x dimension terms) takes the
     exact sequential scan alone, without the screen, and returns the CPU

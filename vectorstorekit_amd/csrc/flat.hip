@@ -651,6 +651,45 @@ SplitPtrs make_split(vsk_ctx *ctx, const vsk_db *db, const float *dq,
   return s;
 }
 
+// the screen's planes: the database's (made once) and the query batch's
+static SplitPtrs make_half(vsk_ctx *ctx, const vsk_db *db, const float *dq, int64_t nq,
+                           int32_t metric, float *qnh, float *qnr) {
+  // whole 64-dimension stages of the screen (zero padding)
+  const int32_t ldb = (db->d + 63) & ~63;
+  const bool cosine = metric == VSK_METRIC_COSINE;
+  const bool bf16 = metric == VSK_METRIC_COSINE_NORMALIZED;
+  auto &pl = db->plane[bf16 ? 1 : 0];
+  if (!cosine && !pl.h.p) {
+    pl.state.reserve(4 * sizeof(uint32_t));
+    pl.h.reserve(plane_bytes(db->n, ldb));
+    uint32_t *st = pl.state.as<uint32_t>();
+    half_rows(ctx, bf16 ? PLANE_BF16 : PLANE_HALF, db->x.as<float>(), db->sqnorm.as<float>(),
+              nullptr, db->n, db->d, db->ld, pl.h.as<uint16_t>(), ldb, nullptr, st);
+    uint32_t hb[2];
+    VSK_HIP(hipMemcpyAsync(hb, st, sizeof(hb), hipMemcpyDeviceToHost, ctx->stream));
+    stream_sync(ctx);
+    std::memcpy(&pl.max_hi, &hb[0], sizeof(float));
+    std::memcpy(&pl.max_res, &hb[1], sizeof(float));
+  }
+  uint16_t *qh = static_cast<uint16_t *>(
+      ctx->scratch_ptr("flat.qhalf", sizeof(uint16_t) * (size_t)nq * ldb));
+  SplitPtrs s{};
+  s.xh = cosine ? db->cos_half.as<uint16_t>() : pl.h.as<uint16_t>();
+  s.qh = qh;
+  s.ldxb = ldb;
+  s.ldqb = ldb;
+  s.kb = ldb;
+  if (bf16) {
+    split_bf16(ctx, dq, nq, db->d, db->ld, qh, nullptr, ldb, qnh, qnr, nullptr);
+    return s;
+  }
+  float *qsc = static_cast<float *>(ctx->scratch_ptr("flat.qscale", sizeof(float) * (size_t)nq));
+  half_queries(ctx, dq, nq, db->d, db->ld, qh, ldb, qsc, qnh, qnr);
+  s.qsc = qsc;
+  s.xmax = cosine ? nullptr : pl.state.as<uint32_t>() + 3;
+  return s;
+}
+
 // top-k over a resident database for queries already on the device
 bool flat_topk_device(vsk_ctx *ctx, const vsk_db *db, const float *dq,
                       int64_t nq, int32_t k, int32_t metric, uint64_t *best,
@@ -682,6 +721,16 @@ void approx_topk(vsk_ctx *ctx, const vsk_db *db, const float *dq, int64_t nq,
                  int32_t k, int32_t metric, uint64_t *best, int passes,
                  float *qnh, float *qnr, int64_t max_growth) {
   int64_t cap = passes == 1 ? screen_cap(k) : default_cap(k);
+  // The screen at up to 1,024 queries: four times the slots its chunks are
+  // expected to fill.  With screen_cap's two times, a launch of few query
+  // tiles spreads a query's slots over some 56 workgroups, about 18
+  // candidates in 36 slots each, and of 333 queries one or two overflowed:
+  // the call ran again, its chunks re-scanned (200,003 x 384, k = 50:
+  // 1.52 ms a call, now 0.37).
+  if (passes == 1 && nq <= 1024 && ctx->max_tile_bytes <= 0) {
+    // (whole row tiles, so that every chunk starts on one)
+    cap = std::max<int64_t>(cap, std::min<int64_t>(ceil_div(32 * (int64_t)k, 256) * 256, 16384));
+  }
   // few queries by the exact scan: every row's key in one dense chunk, which
   // saves a second scan and selection (a first chunk of cap rows fills a
   // fraction of the chip: 100,000 x 768, one query, 93 of 253 us went there);
@@ -712,9 +761,12 @@ void approx_topk(vsk_ctx *ctx, const vsk_db *db, const float *dq, int64_t nq,
     base.metric = metric;
     const bool x3 = use_bf16x3(ctx, metric);
     SplitPtrs sp{};
-    if (x3)
-      sp = make_split(ctx, db, qbat, nb, passes == 3, qnh ? qnh + b0 : nullptr,
-                      qnr ? qnr + b0 : nullptr);
+    if (x3 && passes == 1) {
+      sp = make_half(ctx, db, qbat, nb, metric, qnh + b0, qnr + b0);
+      if (metric == VSK_METRIC_COSINE) base.xaux = db->cos_inv.as<float>();
+    } else if (x3) {
+      sp = make_split(ctx, db, qbat, nb, true, nullptr, nullptr);
+    }
     ScanFn scan = [&](const ScanRequest &r) {
       FlatArgs a = base;
       a.r0 = r.r0;
@@ -736,7 +788,7 @@ void approx_topk(vsk_ctx *ctx, const vsk_db *db, const float *dq, int64_t nq,
         launch_flat(ctx, a, r.dense ? MODE_DENSE : MODE_FILTER, nullptr);
     };
     progressive_topk(ctx, nb, db->n, k, cap, scan, best + b0 * k,
-                     "flat_select", max_growth, nullptr, passes != 1 && metric_is_valu(metric));
+                     "flat_select", max_growth, nullptr, passes == 1 || metric_is_valu(metric));
   }
 }
 

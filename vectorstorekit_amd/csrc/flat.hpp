@@ -84,6 +84,13 @@ __device__ inline uint16_t bf16_rn(float v) {
   return (uint16_t)(u >> 16);
 }
 
+// fp16 of a scaled value, nearest even, with values below the smallest normal
+// fp16 taken as 0 (no subnormal operand enters an MFMA); beyond 65,504 the
+// result is an infinity, whose residual is not finite either
+__device__ inline _Float16 plane_f16(float vs) {
+  return (_Float16)(fabsf(vs) < 0x1p-14f ? 0.f : vs);
+}
+
 // float not below a non-negative double (the error bounds round up)
 __device__ inline float f_up(double v) {
   float f = (float)v;
@@ -239,7 +246,52 @@ struct SplitPtrs {
   const uint16_t *qh, *ql;  // query planes, stride ldqb
   int64_t ldxb, ldqb;
   int32_t kb;               // padded dimension (multiple of 64)
+  // the screen (fp16 planes in xh and qh): each query's power of two, and the
+  // rows' -- plane_scale of *xmax on the device, or xscale when xmax is null
+  const float *qsc = nullptr;
+  const uint32_t *xmax = nullptr;
+  float xscale = 1.f;
 };
+
+// the power of two of a row plane whose largest |x|^2 has these float bits:
+// the largest |x| comes to at most 2^11 (components far from fp16's limits,
+// and 2^-14, its smallest normal number, 25 binades below); 1 for rows that
+// are zero, tiny, huge or not finite (their residuals then say so)
+__host__ __device__ inline float plane_scale(uint32_t maxsq_bits) {
+  const int e = (int)(maxsq_bits >> 23) - 127;  // |x|^2 < 2^(e+1)
+  if (e < -100 || e > 99) return 1.f;
+  const int h = e + 1 >= 0 ? (e + 2) / 2 : -((-e - 1) / 2);  // ceil((e + 1) / 2)
+  const uint32_t bits = (uint32_t)(11 - h + 127) << 23;
+#ifdef __HIP_DEVICE_COMPILE__
+  return __uint_as_float(bits);
+#else
+  float f;
+  __builtin_memcpy(&f, &bits, 4);
+  return f;
+#endif
+}
+// The screen's row planes are stored as the screen copies them: for each tile
+// of 256 rows and stage of 64 columns, 256 x 64 values (32 contiguous KB).
+// From row-major planes a stage is 256 pieces of 128 bytes a pitch apart,
+// which streamed from HBM at 0.9 TB/s when one query tile left nothing to
+// reuse (1M x 768, 64 queries: 1.45 ms, now 1.27).  Planes hold whole tiles.
+__host__ __device__ inline int64_t plane_at(int64_t r, int32_t c, int32_t ldb) {
+  return (((r >> 8) * (ldb >> 6) + (c >> 6)) << 14) + ((r & 255) << 6) + (c & 63);
+}
+inline size_t plane_bytes(int64_t n, int32_t ldb) {
+  return sizeof(uint16_t) * (size_t)(ceil_div(n, 256) * 256) * ldb;
+}
+// the rows' plane (kind: PLANE_*; PLANE_HALF reads |x|^2 from sq,
+// PLANE_COSINE |x| from norm, and writes 1e-8 / |x| to inv); state[4]
+// (device): the maxima of |h| and of the residual's norm, a flag for
+// unusable norms, the largest |x|^2
+enum { PLANE_HALF = 0, PLANE_COSINE = 1, PLANE_BF16 = 2 };
+void half_rows(vsk_ctx *ctx, int kind, const float *x, const float *sq, const float *norm,
+               int64_t n, int32_t d, int32_t ld, uint16_t *h, int32_t ldb, float *inv,
+               uint32_t *state);
+// the queries' fp16 plane, their powers of two, |h| and |q - h|
+void half_queries(vsk_ctx *ctx, const float *q, int64_t nq, int32_t d, int32_t ld, uint16_t *h,
+                  int32_t ldb, float *qsc, float *nhi, float *nres);
 // hi = bf16(x) and (lo non-null) lo = bf16(x - hi) of an (n x ld) fp32
 // matrix, ldb columns; nhi/nres (optional): per-row |hi| and |x - hi|,
 // rounded up, with their maxima over the rows atomically max-ed (as float
@@ -290,7 +342,7 @@ const float *x_aux(const vsk_db *db, int32_t metric);
 void ensure_seq_norms(vsk_ctx *ctx, const vsk_db *db);
 float *q_aux(vsk_ctx *ctx, const float *dq, int64_t nq, int32_t d, int32_t ld,
              int32_t metric);
-// bf16 planes and norms of a query batch for screen_argmin: hi plane
+// bf16 planes and norms of a query batch for the IVF screens: hi plane
 // (stride ldb = roundup(d, 64)), |hi|, |q - hi| and |q|^2 per query
 // the screen's bound check over each query's kc kept screen keys (see
 // flat_screen.hip): ok[q] when the kept keys hold the exact top k, and
@@ -317,9 +369,13 @@ struct ArgminQueries {
   // planes (then qnh = |qh| + |ql|, qnr = |q - qh - ql|, nprod = 2d)
   const uint16_t *ql = nullptr;
   int32_t nprod = 0;
+  const float *qsc = nullptr;  // fp16 plane: each query's power of two
 };
 ArgminQueries argmin_queries(vsk_ctx *ctx, const float *dq, int64_t nq, int32_t d,
                              int32_t ld, const char *slot);
+// the same with the fp16 plane of the flat screen (screen_argmin, PQ)
+ArgminQueries half_argmin_queries(vsk_ctx *ctx, const float *dq, int64_t nq, int32_t d,
+                                  int32_t ld, const char *slot);
 // whether the screen serves an argmin of nq queries over n rows of d dims
 bool screen_argmin_applies(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t d);
 // exact nearest row of each query (sqrt-L2 summed in dimension order, the

@@ -88,6 +88,154 @@ __global__ __launch_bounds__(256) void k_split_rows(
   }
 }
 
+// The screen's row plane in the layout plane_at, one wave per row:
+//  PLANE_HALF    h = fp16(x 2^e), e one power for all rows, from their
+//                largest |x|^2 (plane_scale)
+//  PLANE_COSINE  h = fp16(x / |x| 2^11), and inv[r] = 1e-8 / |x|
+//  PLANE_BF16    h = bf16(x)
+// maxbits[0..1]: the maxima over the rows of |h 2^-e| and |x - h 2^-e| (of
+// x / |x| for cosine) as float bits, maxbits[2] set when a cosine row's norm
+// is too small or not finite (atomic max; squares summed in double, rounded
+// up).
+__global__ __launch_bounds__(256) void k_half_rows(int kind, const float *x, int64_t n, int32_t d,
+                                                   int32_t ld, const uint32_t *maxsq,
+                                                   const float *norm, uint16_t *h, int32_t ldb,
+                                                   float *inv, uint32_t *maxbits) {
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x & 63;
+  const bool cosine = kind == PLANE_COSINE;
+  const float scale = cosine ? 0x1p11f : kind == PLANE_HALF ? plane_scale(*maxsq) : 1.f;
+  const double back = 1.0 / (double)scale;
+  uint32_t mh = 0, mr = 0, bad = 0;
+  for (int64_t r = blockIdx.x * 4 + (threadIdx.x >> 6); r < n; r += (int64_t)gridDim.x * 4) {
+    const float nx = cosine ? norm[r] : 1.f;
+    double sh = 0.0, sr = 0.0;
+    bool any = false;
+    for (int32_t c = lane; c < ldb; c += 64) {
+      float v = c < d ? x[r * ld + c] : 0.f;
+      any |= v != 0.f;
+      if (cosine) v = nx > 0.f ? v / nx : 0.f;
+      const float vs = v * scale;
+      float hv;
+      if (kind == PLANE_BF16) {
+        const uint16_t b = bf16_rn(vs);
+        h[plane_at(r, c, ldb)] = b;
+        hv = __uint_as_float((uint32_t)b << 16);
+      } else {
+        const _Float16 f = plane_f16(vs);
+        h[plane_at(r, c, ldb)] = __builtin_bit_cast(uint16_t, f);
+        hv = (float)f;
+      }
+      const float rv = vs - hv;  // exact
+      sh += (double)hv * (double)hv;
+      sr += (double)rv * (double)rv;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      sh += __shfl_xor(sh, o);
+      sr += __shfl_xor(sr, o);
+    }
+    if (cosine) {
+      if (lane == 0) inv[r] = nx > 0.f ? fminf(1e-8f / nx, 1e30f) : 1e30f;
+      if (__ballot(any) && (!((double)nx >= 0x1p-60) || !((double)nx <= 0x1p60))) {
+        bad = 1;
+        continue;
+      }
+    }
+    // (2^-100: an underflow of x 2^e; 2^-23: the rounding of x / |x|)
+    const float a = f_up(sqrt(sh) * back * (1.0 + 1e-12));
+    const float b = f_up((sqrt(sr) + (kind == PLANE_BF16 ? 0.0 : 0x1p-100)) * back *
+                             (1.0 + 1e-12) +
+                         (cosine ? 0x1p-23 : 0.0));
+    mh = __float_as_uint(a) > mh ? __float_as_uint(a) : mh;
+    mr = __float_as_uint(b) > mr ? __float_as_uint(b) : mr;
+  }
+  if (lane == 0) {
+    atomicMax(&maxbits[0], mh);
+    atomicMax(&maxbits[1], mr);
+    if (bad) atomicMax(&maxbits[2], 1u);
+  }
+}
+
+// The queries' plane: h = fp16(q 2^e), e a power of its own for each query
+// (its largest component to 2^10 .. 2^11), 2^e in qsc, |h 2^-e| and
+// |q - h 2^-e| in nhi and nres, |q|^2 in sq (when given); one wave per row.
+__global__ __launch_bounds__(256) void k_half_queries(const float *x, int64_t n, int32_t d,
+                                                      int32_t ld, _Float16 *h, int32_t ldb,
+                                                      float *qsc, float *nhi, float *nres) {
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x & 63;
+  for (int64_t r = blockIdx.x * 4 + (threadIdx.x >> 6); r < n; r += (int64_t)gridDim.x * 4) {
+    float mx = 0.f;
+    for (int32_t c = lane; c < d; c += 64) mx = fmaxf(mx, fabsf(x[r * ld + c]));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    const float scale =
+        mx >= 0x1p-50f && mx <= 0x1p50f ? ldexpf(1.f, 10 - ilogbf(mx)) : 1.f;
+    const double back = 1.0 / (double)scale;
+    double sh = 0.0, sr = 0.0;
+    for (int32_t c = lane; c < ldb; c += 64) {
+      const float vs = (c < d ? x[r * ld + c] : 0.f) * scale;
+      const _Float16 hv = plane_f16(vs);
+      h[r * ldb + c] = hv;
+      const float rv = vs - (float)hv;  // exact
+      sh += (double)(float)hv * (double)(float)hv;
+      sr += (double)rv * (double)rv;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      sh += __shfl_xor(sh, o);
+      sr += __shfl_xor(sr, o);
+    }
+    if (lane == 0) {
+      qsc[r] = scale;
+      nhi[r] = f_up(sqrt(sh) * back * (1.0 + 1e-12));
+      nres[r] = f_up((sqrt(sr) + 0x1p-100) * back * (1.0 + 1e-12));
+    }
+  }
+}
+
+// the largest of n non-negative floats, as bits, into *out (cleared by the
+// caller; a NaN counts as larger than everything)
+__global__ __launch_bounds__(256) void k_max_bits(const float *v, int64_t n, uint32_t *out) {
+  uint32_t m = 0;
+  for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    const uint32_t b = __float_as_uint(v[i]) & 0x7FFFFFFFu;
+    m = b > m ? b : m;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint32_t b = __shfl_xor(m, o);
+    m = b > m ? b : m;
+  }
+  if ((threadIdx.x & 63) == 0 && m) atomicMax(out, m);
+}
+
+void half_rows(vsk_ctx *ctx, int kind, const float *x, const float *sq, const float *norm,
+               int64_t n, int32_t d, int32_t ld, uint16_t *h, int32_t ldb, float *inv,
+               uint32_t *state) {
+  KernelTimer t(ctx, "half_plane");
+  fill_i32(ctx, reinterpret_cast<int32_t *>(state), 4, 0);
+  if (kind == PLANE_HALF) {
+    const int64_t gm = ceil_div(n, 256);
+    k_max_bits<<<(unsigned)(gm < 1024 ? gm : 1024), 256, 0, ctx->stream>>>(sq, n, state + 3);
+    check_launch("half_plane_max");
+  }
+  const int64_t g = ceil_div(n, 4);
+  k_half_rows<<<(unsigned)(g < 16384 ? g : 16384), 256, 0, ctx->stream>>>(
+      kind, x, n, d, ld, state + 3, norm, h, ldb, inv, state);
+  check_launch("half_plane");
+}
+
+void half_queries(vsk_ctx *ctx, const float *q, int64_t nq, int32_t d, int32_t ld, uint16_t *h,
+                  int32_t ldb, float *qsc, float *nhi, float *nres) {
+  KernelTimer t(ctx, "half_queries");
+  const int64_t g = ceil_div(nq, 4);
+  k_half_queries<<<(unsigned)(g < 16384 ? g : 16384), 256, 0, ctx->stream>>>(
+      q, nq, d, ld, reinterpret_cast<_Float16 *>(h), ldb, qsc, nhi, nres);
+  check_launch("half_queries");
+}
+
 template <int MODE, int METRIC>
 __device__ inline void emit_x(const FlatArgs &a, int64_t qi, int64_t row,
                               float dist, uint64_t th) {
@@ -382,9 +530,10 @@ constexpr int XS_N = 256, XS_Q = 256, XS_K = 64, XS_R = 128;
 constexpr int XS_GQ = 4;
 constexpr int XS_STAGE = (XS_N + XS_Q) * XS_R;  // bytes per stage buffer
 // two stage buffers, then per query: slot limit, slot count, active flag,
-// |q|^2 or |q| (metric), threshold as a distance, threshold key, index of
-// the first reserved slot in the candidate array
-constexpr int XS_LDS = 2 * XS_STAGE + 6 * XS_Q * 4 + 2 * XS_Q * 8;
+// |q|^2 or |q| (metric), the scale of its products and its inverse, the
+// filter's bound on a score, threshold key, index of the first reserved slot
+// in the candidate array
+constexpr int XS_LDS = 2 * XS_STAGE + 7 * XS_Q * 4 + 2 * XS_Q * 8;
 // MODE_TOP2: a (smallest key, second smallest distance) slot per row wave
 // and query
 // and the row norms of four row tiles (copied with the tile's first stage)
@@ -399,6 +548,32 @@ constexpr int XS_LDS_XA = XS_LDS + 4 * XS_N * 4;
 constexpr int XS_QCAP = 32;
 constexpr int XS_LDS_QUEUE = XS_LDS_XA + 8 * XS_QCAP * (64 + 4);
 static_assert(XS_LDS_QUEUE <= 160 * 1024, "LDS of one workgroup");
+// the screened distance from a dot product (cosine: over normalised rows,
+// xa = 1e-8 / |x|, so that dot / (|q| + xa) is the reference's quotient)
+template <int METRIC>
+__device__ inline float xs_dist(float dot, float qa, float xa) {
+  if constexpr (METRIC == VSK_METRIC_COSINE)
+    return 1.0f - dot / (qa + xa);
+  else
+    return dist_from_dot<METRIC>(dot, qa, xa);
+}
+
+// The planes are fp16 under a power of two (half_rows, half_queries): the
+// residuals, and with them the bound and the rows rescored, are an eighth of
+// bf16's at the same MFMA rate.  200,003 x 384 clustered rows, 333 queries,
+// k = 50: with bf16 every query missed the bound and ran a second, wider
+// screen (a call 3.1 to 3.4 ms); with fp16 none does (0.37 ms).  Normalised cosine keeps the bf16 planes: which near
+// ties its tiers settle is part of what the tests pin.
+template <int METRIC>
+constexpr bool xs_bf16 = METRIC == VSK_METRIC_COSINE_NORMALIZED;
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ f4 xs_mfma(bf8 x, bf8 q, f4 acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, q, acc, 0, 0, 0);
+}
+__device__ __forceinline__ f4 xs_mfma(h8 x, h8 q, f4 acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(x, q, acc, 0, 0, 0);
+}
+
 template <int MODE, int METRIC>
 constexpr bool xs_norms_in_lds() {
   return MODE == MODE_TOP2 ||
@@ -463,7 +638,7 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
       (int32_t)(((a.nq - q0) < XS_Q ? (a.nq - q0) : XS_Q) * s.ldqb * 2);
   const __amdgpu_buffer_rsrc_t rq =
       __builtin_amdgcn_make_buffer_rsrc((void *)(s.qh + q0 * s.ldqb), 0, qbytes, kBufFlags);
-  const int32_t ldx2 = (int32_t)s.ldxb * 2;  // the query plane has the same pitch
+  const int32_t ldq2 = (int32_t)s.ldqb * 2;
   const int cl = lane >> 4;
   // filter appends: the workgroup takes a.sub slots of each of its
   // queries' candidate lists up front (one device atomic per query, not one
@@ -481,8 +656,9 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
   int32_t *s_cnt = s_lim + XS_Q;
   int32_t *s_ok = s_cnt + XS_Q;
   float *s_qa = reinterpret_cast<float *>(s_ok + XS_Q);
-  float *s_thf = s_qa + XS_Q;
-  float *s_tdot = s_thf + XS_Q;
+  float *s_sc = s_qa + XS_Q;   // the plane values' products are s_sc times the real ones
+  float *s_inv = s_sc + XS_Q;  // (powers of two)
+  float *s_tdot = s_inv + XS_Q;
   uint64_t *s_th = reinterpret_cast<uint64_t *>(s_tdot + XS_Q);
   int64_t *s_pb = reinterpret_cast<int64_t *>(s_th + XS_Q);
   uint64_t *s_t1 = reinterpret_cast<uint64_t *>(lds + XS_LDS);  // [4][XS_Q]
@@ -503,6 +679,13 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
     const bool ok = q < a.nq && (!a.active || a.active[q]);
     s_ok[tid] = ok ? 1 : 0;
     s_qa[tid] = (ok && a.qaux) ? a.qaux[q] : 0.f;
+    const float sc = xs_bf16<METRIC> ? 1.f
+                     : (ok ? s.qsc[q] : 1.f) *
+                     (METRIC == VSK_METRIC_COSINE ? 0x1p11f
+                      : s.xmax                    ? plane_scale(*s.xmax)
+                                                  : s.xscale);
+    s_sc[tid] = sc;
+    s_inv[tid] = 1.0f / sc;
     if constexpr (MODE == MODE_FILTER) {
       const uint64_t th = ok ? a.thresh[q] : 0;
       const uint32_t th_hi = (uint32_t)(th >> 32);
@@ -510,7 +693,6 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
       const float thf = !ok ? -__int_as_float(0x7f800000)
                             : (th_hi == 0xFFFFFFFFu ? __int_as_float(0x7f800000)
                                                     : vsk_ord2f(th_hi));
-      s_thf[tid] = thf;
       // the same bound on the raw dot product (normalised cosine: a dot
       // below 1 - thf less a margin of the rounding of 1 - dot cannot pass;
       // dot: -dot <= thf exactly when dot >= -thf)
@@ -521,7 +703,9 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
         if ((double)f > m) f = __uint_as_float(f > 0.f ? __float_as_uint(f) - 1u
                                                : (f < 0.f ? __float_as_uint(f) + 1u
                                                           : 0x80000001u));
-        s_tdot[tid] = f;
+        // (no query: nothing passes, rather than a NaN that every block's
+        // test would stop at)
+        s_tdot[tid] = ok ? f * sc : __int_as_float(0x7f800000);
       } else if constexpr (METRIC == VSK_METRIC_L2SQ || METRIC == VSK_METRIC_L2) {
         // L2: a score can pass the exact test (fma(-2, dot, qa + xa), its
         // max with 0, <= thf) only when dot - xa/2 >= (qa - thf)/2 less a
@@ -544,7 +728,7 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
                                                  : (f < 0.f ? __float_as_uint(f) + 1u
                                                             : 0x80000001u));
         }
-        s_tdot[tid] = f;
+        s_tdot[tid] = f * sc;
       } else if constexpr (METRIC == VSK_METRIC_COSINE) {
         // cosine (with the reference's epsilon): a <= thf is
         // dot >= (1 - thf) den, den = |q||x| + 1e-8 > 0; the bound t2 on
@@ -564,9 +748,9 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
                                                  : (f < 0.f ? __float_as_uint(f) + 1u
                                                             : 0x80000001u));
         }
-        s_tdot[tid] = f;
+        s_tdot[tid] = f * sc;
       } else {
-        s_tdot[tid] = -thf;
+        s_tdot[tid] = -thf * sc;
       }
       // segmented: this split's fixed segment; else slots taken from the
       // query's append counter
@@ -594,21 +778,25 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
   // the next copy overwrites.
   // (units 4w+u and 4w+u+2 differ by 16 rows, the same swizzle: one lane
   // offset per parity of u, the row step in the scalar offset)
-  int32_t voff[2];
+  int32_t voff[2], qoff[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
-    const int r = 8 * (4 * w + u) + (lane >> 3);
-    voff[u] = r * ldx2 + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
+    const int r = 8 * (4 * w + u) + (lane >> 3), c = ((lane & 7) ^ ((r >> 1) & 7)) << 4;
+    voff[u] = r * XS_R + c;
+    qoff[u] = r * ldq2 + c;
   }
   int dst = 0;          // next stage to copy: stage dst of the tile at dt0
   int64_t dt0 = s0;     // (past the slice: zero-length rows, nothing read)
   int dtile = 0;        // index of that tile in the slice
   int dbuf = 0;
+  const uint16_t *xsrc = s.xh + (s0 >> 8) * nst * (XS_N * XS_K);  // the next stage's rows
   auto copy_next = [&]() {
     const int64_t left = s1 - dt0;
     const int64_t rows = left < XS_N ? (left > 0 ? left : 0) : XS_N;
+    // the stage's 256 rows x 64 dims are 32 contiguous KB of the plane
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(s.xh + dt0 * s.ldxb), 0, (int32_t)(rows * ldx2), kBufFlags);
+        (void *)xsrc, 0, (int32_t)(rows * XS_R), kBufFlags);
+    xsrc += XS_N * XS_K;
     if constexpr (XA) {
       if (dst == 0 && w < 4) {
         // the tile's row norms, 64 per wave (rows past the slice read 0)
@@ -630,14 +818,13 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
         uint8_t *bx = lds + dbuf * (QR ? XS_N * XS_R : XS_STAGE) + 4 * (w + 4 * h) * 1024;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const int32_t so = kofs + (u >> 1) * 16 * ldx2 + h * 128 * ldx2;
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
-              rx, (__attribute__((address_space(3))) void *)(bx + u * 1024), 16, voff[u & 1], so,
-              0, 0);
+              rx, (__attribute__((address_space(3))) void *)(bx + u * 1024), 16, voff[u & 1],
+              ((u >> 1) * 16 + h * 128) * XS_R, 0, 0);
           if constexpr (!QR)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 rq, (__attribute__((address_space(3))) void *)(bx + XS_N * XS_R + u * 1024), 16,
-                voff[u & 1], so, 0, 0);
+                qoff[u & 1], kofs + ((u >> 1) * 16 + h * 128) * ldq2, 0, 0);
         }
       }
     }
@@ -659,18 +846,22 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
       return lds + (gg & 1) * XS_STAGE + XS_N * XS_R;
   };
   // operands: two sets, this step's and the next one's (read one step ahead)
-  bf8 ra[2][4], rb[2][8];
+  // (read through a bit cast: a plain copy of a uint4 loses the type that tells
+  // the compiler the reads apart from the copies in flight, and it then waits
+  // for all of them before the first read of every stage: 5 % of the launch)
+  using op8 = std::conditional_t<xs_bf16<METRIC>, bf8, h8>;
+  op8 ra[2][4], rb[2][8];
   auto read_ops = [&](int gg, int kk, int n) {
     const uint8_t *bq = queries_of(gg), *bx = rows_of(gg);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       rb[n][j] = __builtin_bit_cast(
-          bf8, *reinterpret_cast<const uint4 *>(
+          op8, *reinterpret_cast<const uint4 *>(
                    bq + swz8(wq * 128 + j * 16 + (lane & 15), kk * 4 + cl)));
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       ra[n][i] = __builtin_bit_cast(
-          bf8, *reinterpret_cast<const uint4 *>(
+          op8, *reinterpret_cast<const uint4 *>(
                    bx + swz8(wr * 64 + i * 16 + (lane & 15), kk * 4 + cl)));
   };
   if constexpr (QR) {
@@ -682,9 +873,9 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
           uint8_t *bq = lds + 2 * XS_N * XS_R + hh * XS_Q * XS_R + 4 * (w + 4 * h) * 1024;
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            const int32_t so = hh * XS_K * 2 + (u >> 1) * 16 * ldx2 + h * 128 * ldx2;
+            const int32_t so = hh * XS_K * 2 + ((u >> 1) * 16 + h * 128) * ldq2;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rq, (__attribute__((address_space(3))) void *)(bq + u * 1024), 16, voff[u & 1],
+                rq, (__attribute__((address_space(3))) void *)(bq + u * 1024), 16, qoff[u & 1],
                 so, 0, 0);
           }
         }
@@ -716,6 +907,7 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
       const bool ok = s_ok[lq] != 0;
       const float td = s_tdot[lq];
       const float qa = a.qaux ? s_qa[lq] : 0.f;
+      const float m2 = -2.0f * s_inv[lq];
       const uint64_t th = s_th[lq];
       uint32_t m = 0;
 #pragma unroll
@@ -733,7 +925,7 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
         const int64_t row = rb + 16 * (b >> 2) + (b & 3);
         if (row >= s1) continue;  // past the slice
         // |q|^2 - 2 (dot - |x|^2/2), one rounding
-        const float dist = fmaxf(__builtin_fmaf(-2.0f, q_val[ln * 16 + b], qa), 0.0f);
+        const float dist = fmaxf(__builtin_fmaf(m2, q_val[ln * 16 + b], qa), 0.0f);
         const uint64_t key = vsk_key(dist, (uint32_t)row);
         if (key <= th) {
           const int pos = atomicAdd(&s_cnt[lq], 1);
@@ -750,26 +942,35 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
     // previous epilogue, which then has the registers to itself
     read_ops(g, 0, 0);
     // the accumulators start at zero, or in filter mode on L2 and L2^2 at
-    // -|x|^2/2 of the lane's rows (the tile's norms reached LDS with its
+    // -|x|^2/2 (scaled) of the lane's rows (the tile's norms reached LDS with its
     // first stage): acc is then dot - |x|^2/2, the quantity the filter's
     // bound is on
     f4 acc[4][8];
     const int xl = XS_SHIFT ? lane_here() : lane;
+    float hs[8];  // minus half of each query's scale
+    if constexpr (XS_SHIFT) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) hs[j] = -0.5f * s_sc[wq * 128 + 16 * j + (xl & 15)];
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       f4 init = f4{0.f, 0.f, 0.f, 0.f};
       if constexpr (XS_SHIFT)
         init = *reinterpret_cast<const f4 *>(s_xa + (tcur & 3) * XS_N + wr * 64 +
-                                             4 * (xl >> 4) + 16 * i) *
-               -0.5f;
+                                             4 * (xl >> 4) + 16 * i);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[i][j] = init;
+      for (int j = 0; j < 8; ++j) {
+        if constexpr (XS_SHIFT)
+          acc[i][j] = init * hs[j];
+        else
+          acc[i][j] = init;
+      }
     }
 #define XS_MMA(N)                                                               \
   do {                                                                          \
     _Pragma("unroll") for (int i = 0; i < 4; ++i) {                             \
       _Pragma("unroll") for (int j = 0; j < 8; ++j) acc[i][j] =                 \
-          __builtin_amdgcn_mfma_f32_16x16x32_bf16(ra[N][i], rb[N][j], acc[i][j], 0, 0, 0); \
+          xs_mfma(ra[N][i], rb[N][j], acc[i][j]); \
     }                                                                           \
   } while (0)
     // (the operand reads are spread over the MFMAs: as a block, the eight
@@ -813,7 +1014,7 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
     const int lq0 = wq * 128 + (lane & 15);
     const int32_t *l_ok = s_ok + lq0, *l_lim = s_lim + lq0;
     int32_t *l_cnt = s_cnt + lq0;
-    const float *l_qa = s_qa + lq0, *l_thf = s_thf + lq0, *l_tdot = s_tdot + lq0;
+    const float *l_qa = s_qa + lq0, *l_inv = s_inv + lq0, *l_tdot = s_tdot + lq0;
     // rows of this lane inside the slice: bit 4i+r for row rbase + 16i + r
     uint32_t vmask = 0xFFFFu;
     if (!full) {
@@ -841,6 +1042,26 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
       const float qa = a.qaux ? l_qa[16 * j] : 0.f;
       if constexpr (MODE == MODE_DENSE) {
         if (!l_ok[16 * j]) continue;
+        const float iv = xs_bf16<METRIC> ? 1.f : l_inv[16 * j];
+        if (a.words && full && !(a.cap & 3)) {
+          // 32-bit distances, four rows a store
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int64_t row = rbase + i * 16;
+            f4 xv = f4{0.f, 0.f, 0.f, 0.f};
+            if (a.xaux) {
+#pragma unroll
+              for (int r = 0; r < 4; ++r) xv[r] = a.xaux[row + r];
+            }
+            uint4 o;
+            o.x = vsk_f2ord(xs_dist<METRIC>(acc[i][j][0] * iv, qa, xv[0]));
+            o.y = vsk_f2ord(xs_dist<METRIC>(acc[i][j][1] * iv, qa, xv[1]));
+            o.z = vsk_f2ord(xs_dist<METRIC>(acc[i][j][2] * iv, qa, xv[2]));
+            o.w = vsk_f2ord(xs_dist<METRIC>(acc[i][j][3] * iv, qa, xv[3]));
+            *reinterpret_cast<uint4 *>(a.words + qi * a.cap + (row - a.r0)) = o;
+          }
+          continue;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -848,8 +1069,11 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
             const int64_t row = rbase + i * 16 + r;
             if (!full && row >= s1) continue;
             const float xa = a.xaux ? a.xaux[row] : 0.f;
-            a.cand[qi * a.cap + (row - a.r0)] =
-                vsk_key(dist_from_dot<METRIC>(acc[i][j][r], qa, xa), (uint32_t)row);
+            const float dist = xs_dist<METRIC>(acc[i][j][r] * iv, qa, xa);
+            if (a.words)
+              a.words[qi * a.cap + (row - a.r0)] = vsk_f2ord(dist);
+            else
+              a.cand[qi * a.cap + (row - a.r0)] = vsk_key(dist, (uint32_t)row);
           }
       } else if constexpr (MODE == MODE_TOP2) {
         // The screened distance less the query's constant |q|^2,
@@ -860,6 +1084,7 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
         // argmin's bound adds; equal screened distances stay within that of
         // each other, so the bound test still refuses to decide them.
         const float inf = __int_as_float(0x7f800000);
+        const float c2 = -2.0f * l_inv[16 * j];
         float m1 = inf, m2 = inf;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -867,7 +1092,7 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
           for (int r = 0; r < 4; ++r) {
             const int e = 4 * i + r;
             const float xa = s_xa[(tcur & 3) * XS_N + wr * 64 + 4 * cl + 16 * i + r];
-            float t = __builtin_fmaf(-2.0f, acc[i][j][r], xa);
+            float t = __builtin_fmaf(c2, acc[i][j][r], xa);
             t = __uint_as_float((__float_as_uint(t) & ~63u) | (uint32_t)e);
             if (!full) t = ((vmask >> e) & 1u) ? t : inf;
             m2 = __builtin_amdgcn_fmed3f(m1, m2, t);
@@ -954,7 +1179,7 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
             for (int r = 0; r < 4; ++r)
               m |= (acc[i][j][r] < tdot) ? 0u : (1u << (4 * i + r));
         } else if constexpr (METRIC == VSK_METRIC_COSINE) {
-          // dot - t2 (|q||x| + 1e-8) >= 0 with the row norms from LDS; the
+          // dot - t2 (|q| + 1e-8/|x|) >= 0 with 1e-8/|x| from LDS; the
           // block's largest first (a NaN score is dropped by the max: it
           // needs a non-finite input, whose query fails the screen's check)
           const float t2 = l_tdot[16 * j];
@@ -964,7 +1189,7 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const float xn = s_xa[(tcur & 3) * XS_N + wr * 64 + 4 * cl + 16 * i + r];
-              mx = fmaxf(mx, __builtin_fmaf(-t2, __builtin_fmaf(qa, xn, 1e-8f), acc[i][j][r]));
+              mx = fmaxf(mx, __builtin_fmaf(-t2, qa + xn, acc[i][j][r]));
             }
           if (!__builtin_amdgcn_ballot_w64(!(mx < 0.f))) continue;
 #pragma unroll
@@ -972,38 +1197,10 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const float xn = s_xa[(tcur & 3) * XS_N + wr * 64 + 4 * cl + 16 * i + r];
-              m |= (__builtin_fmaf(-t2, __builtin_fmaf(qa, xn, 1e-8f), acc[i][j][r]) < 0.f)
+              m |= (__builtin_fmaf(-t2, qa + xn, acc[i][j][r]) < 0.f)
                        ? 0u
                        : (1u << (4 * i + r));
             }
-        } else {
-          const float th_f = l_thf[16 * j];
-          // the block's largest dot - |x|^2/2 first, against the query's
-          // bound on it (with its margin, no score whose exact test below
-          // passes is under it): when it is below in every lane, no score of
-          // the block can pass.  A NaN score is dropped by the max; it needs
-          // a non-finite input, whose bound is not finite, so such a query
-          // fails the screen's check and is redone exactly.
-          const float tdot = l_tdot[16 * j];
-          float mx = -__int_as_float(0x7f800000);
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              mx = fmaxf(mx, acc[i][j][r] -
-                                 0.5f * s_xa[(tcur & 3) * XS_N + wr * 64 + 4 * cl + 16 * i + r]);
-          if (!__builtin_amdgcn_ballot_w64(!(mx < tdot))) continue;
-          // the same bound per score: a superset of the scores whose exact
-          // test below passes (the exact key test then decides each one)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              // (rows past the slice read 0 and are masked off below)
-              const float xa = s_xa[(tcur & 3) * XS_N + wr * 64 + 4 * cl + 16 * i + r];
-              m |= (acc[i][j][r] - 0.5f * xa < tdot) ? 0u : (1u << (4 * i + r));
-            }
-          (void)th_f;
         }
         m &= vmask;
         if (!__builtin_amdgcn_ballot_w64(m != 0)) continue;  // the common case
@@ -1012,6 +1209,7 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
           const uint64_t th = l_th[16 * j];
           const int32_t lim = l_lim[16 * j];
           const int64_t pb = l_pb[16 * j];
+          const float iv = xs_bf16<METRIC> ? 1.f : l_inv[16 * j];
           // this query's 16 scores of the lane as named values behind an
           // empty asm: a select between two loads of one array would be
           // folded into one dynamically indexed load, which sends the array
@@ -1039,14 +1237,14 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
             float dist;
             if constexpr (XS_SHIFT) {
               // |q|^2 - 2 (dot - |x|^2/2), one rounding
-              dist = fmaxf(__builtin_fmaf(-2.0f, dot, qa), 0.0f);
+              dist = fmaxf(__builtin_fmaf(-2.0f * iv, dot, qa), 0.0f);
             } else {
               float xa = 0.f;
               if constexpr (XA)
                 xa = s_xa[(tcur & 3) * XS_N + wr * 64 + 4 * cl + 16 * (b >> 2) + (b & 3)];
               else if (a.xaux)
                 xa = a.xaux[row];
-              dist = dist_from_dot<METRIC>(dot, qa, xa);
+              dist = xs_dist<METRIC>(dot * iv, qa, xa);
             }
             const uint64_t key = vsk_key(dist, (uint32_t)row);
             if (key <= th) {
@@ -1152,8 +1350,8 @@ void launch_flat_screen(vsk_ctx *ctx, FlatArgs a, const SplitPtrs &s, int mode,
   if (rows <= 0 || a.nq <= 0) return;
   if (mode == MODE_MATRIX || mode == MODE_ARGMIN)
     fail(VSK_ERR_UNSUPPORTED, "the screen has no matrix or VALU argmin mode");
-  if (s.ldqb != s.ldxb || s.kb > s.ldxb || (s.kb & 63))
-    fail(VSK_ERR_INVALID_ARGUMENT, "screen planes need one pitch and a padded dimension");
+  if (s.ldqb != s.ldxb || s.kb != s.ldxb || (s.kb & 63) || (a.r0 & (XS_N - 1)))
+    fail(VSK_ERR_INVALID_ARGUMENT, "screen planes need one pitch and whole row tiles");
   static bool lds_set = false;
   if (!lds_set) {
     set_lds_metric<VSK_METRIC_L2SQ, false>();

@@ -53,64 +53,21 @@ bool screen_applies(int32_t metric, int32_t k) {
   return k <= VSK_MAX_K;
 }
 
-// per row (one wave): |bf16(x)| and |x - bf16(x)| (sums of squares in
-// double, square roots rounded up) over the fp32 norm |x| the screen
-// divides by, their maxima over the rows with |x| > 0 as float bits
-// (atomic max, ratios rounded up) in rel[0..1]; rel[2] = 1 when a row with
-// a nonzero component has a norm below 2^-60 or not finite
-__global__ __launch_bounds__(256) void k_cos_rel(const float *x, int64_t n, int32_t d,
-                                                 int32_t ld, const float *norm, uint32_t *rel) {
-  const int lane = threadIdx.x & 63;
-  uint32_t mh = 0, mr = 0, bad = 0;
-  for (int64_t r = blockIdx.x * 4 + (threadIdx.x >> 6); r < n; r += (int64_t)gridDim.x * 4) {
-    double sh = 0.0, sr = 0.0;
-    for (int32_t c = lane; c < d; c += 64) {
-      const float v = x[r * ld + c];
-      const float hv = __uint_as_float((uint32_t)bf16_rn(v) << 16);
-      const float rv = v - hv;  // exact
-      sh += (double)hv * (double)hv;
-      sr += (double)rv * (double)rv;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      sh += __shfl_xor(sh, o);
-      sr += __shfl_xor(sr, o);
-    }
-    const double nx = (double)norm[r];
-    if (sh == 0.0 && sr == 0.0) continue;  // a zero row: exactly 1 either way
-    if (!(nx >= 0x1p-60) || !(nx <= 0x1p60)) {
-      bad = 1;
-      continue;
-    }
-    const float a = f_up(sqrt(sh) / nx * (1.0 + 1e-12));
-    const float b = f_up(sqrt(sr) / nx * (1.0 + 1e-12));
-    mh = __float_as_uint(a) > mh ? __float_as_uint(a) : mh;
-    mr = __float_as_uint(b) > mr ? __float_as_uint(b) : mr;
-  }
-  if (lane == 0) {
-    if (mh | mr) {
-      atomicMax(&rel[0], mh);
-      atomicMax(&rel[1], mr);
-    }
-    if (bad) atomicMax(&rel[2], 1u);
-  }
-}
-
 bool cosine_screen_ok(vsk_ctx *ctx, const vsk_db *db) {
   if (db->cos_state == 0) {
-    uint32_t *rel = static_cast<uint32_t *>(ctx->scratch_ptr("screen.cosrel", 16));
-    fill_i32(ctx, reinterpret_cast<int32_t *>(rel), 4, 0);
-    int64_t g = ceil_div(db->n, 4);
-    if (g > 16384) g = 16384;
-    k_cos_rel<<<(unsigned)g, 256, 0, ctx->stream>>>(db->x.as<float>(), db->n, db->d, db->ld,
-                                                    db->norm.as<float>(), rel);
-    check_launch("cos_rel");
+    const int32_t ldb = (db->d + 63) & ~63;
+    db->cos_half.reserve(plane_bytes(db->n, ldb));
+    db->cos_inv.reserve(sizeof(float) * (size_t)db->n);
+    uint32_t *st = static_cast<uint32_t *>(ctx->scratch_ptr("screen.cosrel", 16));
+    half_rows(ctx, PLANE_COSINE, db->x.as<float>(), nullptr, db->norm.as<float>(), db->n, db->d,
+              db->ld, db->cos_half.as<uint16_t>(), ldb, db->cos_inv.as<float>(), st);
     uint32_t h[3];
-    VSK_HIP(hipMemcpyAsync(h, rel, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
+    VSK_HIP(hipMemcpyAsync(h, st, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
     stream_sync(ctx);
     std::memcpy(&db->cos_rel_hi, &h[0], sizeof(float));
     std::memcpy(&db->cos_rel_res, &h[1], sizeof(float));
     db->cos_state = h[2] ? -1 : 1;
+    if (h[2]) db->cos_half.release();
   }
   return db->cos_state > 0;
 }
@@ -377,8 +334,9 @@ static std::vector<int32_t> screen_tier(vsk_ctx *ctx, const vsk_db *db,
   ca.metric = metric;
   ca.qnh = qn;
   ca.qnr = qn + nb;
-  ca.xh = db->split_max_hi;
-  ca.xr = db->split_max_res;
+  const auto &pl = db->plane[metric == VSK_METRIC_COSINE_NORMALIZED ? 1 : 0];
+  ca.xh = pl.max_hi;
+  ca.xr = pl.max_res;
   if (metric == VSK_METRIC_COSINE) {
     // relative maxima and the queries' fp32 norms (those the screen divided by)
     ca.xh = db->cos_rel_hi;
@@ -573,14 +531,18 @@ __global__ __launch_bounds__(64) void k_argmin_finish(
 
 // gathers the undecided queries: their fp32 rows, hi-plane rows and |q|^2
 __global__ void k_gather_argmin_queries(const float *Q, int64_t ld, const uint16_t *qh,
-                                        int32_t ldb, const float *qsq, const int32_t *idx,
-                                        int64_t m, float *Q2, uint16_t *qh2, float *qsq2) {
+                                        int32_t ldb, const float *qsq, const float *qsc,
+                                        const int32_t *idx, int64_t m, float *Q2,
+                                        uint16_t *qh2, float *qsq2, float *qsc2) {
   const int64_t i = blockIdx.x;
   if (i >= m) return;
   const int64_t src = idx[i];
   for (int64_t c = threadIdx.x; c < ld; c += blockDim.x) Q2[i * ld + c] = Q[src * ld + c];
   for (int64_t c = threadIdx.x; c < ldb; c += blockDim.x) qh2[i * ldb + c] = qh[src * ldb + c];
-  if (threadIdx.x == 0) qsq2[i] = qsq[src];
+  if (threadIdx.x == 0) {
+    qsq2[i] = qsq[src];
+    qsc2[i] = qsc[src];
+  }
 }
 
 // The collected candidates of each undecided query: one wave per query, a
@@ -656,6 +618,24 @@ ArgminQueries argmin_queries(vsk_ctx *ctx, const float *dq, int64_t nq, int32_t 
   return qp;
 }
 
+ArgminQueries half_argmin_queries(vsk_ctx *ctx, const float *dq, int64_t nq, int32_t d,
+                                  int32_t ld, const char *slot) {
+  ArgminQueries qp;
+  qp.ldb = (d + 63) & ~63;
+  const std::string sl(slot);
+  uint16_t *qh = static_cast<uint16_t *>(
+      ctx->scratch_ptr(sl + ".qh", sizeof(uint16_t) * (size_t)nq * qp.ldb));
+  float *nrm = static_cast<float *>(ctx->scratch_ptr(sl + ".qn", sizeof(float) * 4 * (size_t)nq));
+  half_queries(ctx, dq, nq, d, ld, qh, qp.ldb, nrm + 3 * nq, nrm, nrm + nq);
+  row_norms(ctx, dq, nq, d, ld, nrm + 2 * nq, nullptr);
+  qp.qh = qh;
+  qp.qnh = nrm;
+  qp.qnr = nrm + nq;
+  qp.qsq = nrm + 2 * nq;
+  qp.qsc = nrm + 3 * nq;
+  return qp;
+}
+
 bool screen_argmin_applies(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t d) {
   if (ctx->flat_no_screen || ctx->flat_fp32 || ctx->exact_only) return false;
   if (n >= 0x7FFFFFFFll || d < 32) return false;  // narrow rows: the padding to 64 dims costs
@@ -668,17 +648,16 @@ void screen_argmin(vsk_ctx *ctx, const float *X, const float *xsq, int64_t n,
                    const ArgminQueries &qp, int32_t *argmin, float *dist) {
   KernelTimer tm(ctx, "screen_argmin", (double)nq * (double)n);
   const int32_t ldb = qp.ldb;
-  // the rows' hi plane and the maxima of |hi| and |x - hi| over them
+  // the rows' fp16 plane and the maxima of |h| and |x - h| over them
   uint16_t *xh = static_cast<uint16_t *>(
-      ctx->scratch_ptr("sam.xh", sizeof(uint16_t) * (size_t)n * ldb));
-  uint32_t *maxbits = static_cast<uint32_t *>(ctx->scratch_ptr("sam.max", 2 * sizeof(uint32_t)));
-  fill_i32(ctx, reinterpret_cast<int32_t *>(maxbits), 2, 0);
-  split_bf16(ctx, X, n, d, ld, xh, nullptr, ldb, nullptr, nullptr, maxbits);
-  SplitPtrs sp;
+      ctx->scratch_ptr("sam.xh", plane_bytes(n, ldb)));
+  uint32_t *maxbits = static_cast<uint32_t *>(ctx->scratch_ptr("sam.max", 4 * sizeof(uint32_t)));
+  half_rows(ctx, PLANE_HALF, X, xsq, nullptr, n, d, ld, xh, ldb, nullptr, maxbits);
+  SplitPtrs sp{};
   sp.xh = xh;
-  sp.xl = nullptr;
   sp.qh = qp.qh;
-  sp.ql = nullptr;
+  sp.qsc = qp.qsc;
+  sp.xmax = maxbits + 3;
   sp.ldxb = ldb;
   sp.ldqb = ldb;
   sp.kb = ldb;
@@ -721,6 +700,7 @@ void screen_argmin(vsk_ctx *ctx, const float *X, const float *xsq, int64_t n,
     a.mat = a2;
     SplitPtrs sb = sp;
     sb.qh = qp.qh + b0 * ldb;
+    sb.qsc = qp.qsc + b0;
     // splits without rows write nothing: their pairs must read as empty
     fill_u64(ctx, k1, nb * top, VSK_KEY_NONE);
     fill_i32(ctx, reinterpret_cast<int32_t *>(a2), nb * top, 0x7f800000);
@@ -748,9 +728,10 @@ void screen_argmin(vsk_ctx *ctx, const float *X, const float *xsq, int64_t n,
   float *q2 = static_cast<float *>(ctx->scratch_ptr("sam.fq", sizeof(float) * (size_t)m * ld));
   uint16_t *qh2 = static_cast<uint16_t *>(
       ctx->scratch_ptr("sam.fqh", sizeof(uint16_t) * (size_t)m * ldb));
-  float *qsq2 = static_cast<float *>(ctx->scratch_ptr("sam.fqsq", sizeof(float) * (size_t)m));
-  k_gather_argmin_queries<<<(unsigned)m, 128, 0, ctx->stream>>>(dq, ld, qp.qh, ldb, qp.qsq,
-                                                                 fidx, m, q2, qh2, qsq2);
+  float *qsq2 = static_cast<float *>(ctx->scratch_ptr("sam.fqsq", sizeof(float) * 2 * (size_t)m));
+  float *qsc2 = qsq2 + m;
+  k_gather_argmin_queries<<<(unsigned)m, 128, 0, ctx->stream>>>(
+      dq, ld, qp.qh, ldb, qp.qsq, qp.qsc, fidx, m, q2, qh2, qsq2, qsc2);
   check_launch("screen_argmin_gather");
   uint64_t *cand = static_cast<uint64_t *>(
       ctx->scratch_ptr("sam.cand", sizeof(uint64_t) * (size_t)m * kCollect));
@@ -783,6 +764,7 @@ void screen_argmin(vsk_ctx *ctx, const float *X, const float *xsq, int64_t n,
     a.counts = cnt + r0;
     SplitPtrs sb = sp;
     sb.qh = qh2 + r0 * ldb;
+    sb.qsc = qsc2 + r0;
     launch_flat_screen(ctx, a, sb, MODE_FILTER, nullptr, nullptr);
   }
   k_argmin_collect<<<(unsigned)m, 64, 0, ctx->stream>>>(cand, kCollect, cnt, m, X, ld, q2, d,

@@ -1125,7 +1125,7 @@ static FlatArgs centroid_args(const vsk_ivf *ivf, const float *dq, int64_t nq) {
 static void ivf_assign_device(vsk_ctx *ctx, const vsk_ivf *ivf, const float *dx,
                               int64_t n, int32_t *out) {
   if (screen_argmin_applies(ctx, n, ivf->nlist, ivf->d)) {
-    const ArgminQueries qp = argmin_queries(ctx, dx, n, ivf->d, ivf->ld, "ivf.aq");
+    const ArgminQueries qp = half_argmin_queries(ctx, dx, n, ivf->d, ivf->ld, "ivf.aq");
     float *dist = static_cast<float *>(ctx->scratch_ptr("ivf.adist", sizeof(float) * (size_t)n));
     screen_argmin(ctx, ivf->centroids.x.as<float>(), ivf->centroids.sqnorm.as<float>(),
                   ivf->nlist, ivf->d, ivf->ld, dx, n, qp, out, dist);

@@ -913,10 +913,10 @@ vsk_status vsk_kmeans(vsk_ctx *ctx, const float *x, int64_t n, int32_t d,
   hipStream_t aux = ctx->aux_stream();
   hipEvent_t ev_assigned[2] = {ctx->take_event(), ctx->take_event()};
   hipEvent_t ev_summed[2] = {ctx->take_event(), ctx->take_event()};
-  // the rows' bf16 planes for the screened assignment, made once
+  // the rows' fp16 plane for the screened assignment, made once
   ArgminQueries qp;
   if (max_iter > 0 && screen_argmin_applies(ctx, n, k, d))
-    qp = argmin_queries(ctx, dx, n, d, ld, "km.q");
+    qp = half_argmin_queries(ctx, dx, n, d, ld, "km.q");
   // one Lloyd iteration i: centroids cbuf[i & 1] -> cbuf[(i + 1) & 1]
   auto enqueue = [&](int32_t i) {
     const float *cur = cbuf + (size_t)(i & 1) * k * ld;

@@ -24,6 +24,8 @@
 // queries to a 16-byte half entry, survivors staged in LDS); k_pq_adc any other
 // shape.  Ranking is on the sum (sqrt is monotone); sqrt is applied to the
 // outputs only.
+#include <cstring>
+
 #include "flat.hpp"
 
 struct vsk_pq {
@@ -34,13 +36,14 @@ struct vsk_pq {
   vsk::DevBuf codes;      // n x M uint8
   int64_t n = 0, cap_rows = 0;
   // the bf16 screen of the ADC scan: the decoded rows x^ (each segment's
-  // codeword) as a bf16 plane of xldb columns, |x^|^2 per row, and the
-  // maxima over the rows of |bf16(x^)| and |x^ - bf16(x^)|; made by the
+  // codeword) as an fp16 plane of xldb columns, |x^|^2 per row, and the
+  // maxima over the rows of |h| and |x^ - h|; made by the
   // first screened search and again when rows were added since (xrows)
   mutable vsk::DevBuf xplane, xsq;
   mutable int32_t xldb = 0;
   mutable int64_t xrows = 0;
   mutable double xh_max = 0, xr_max = 0;
+  mutable float xscale = 1.f;  // the plane's power of two
 };
 
 namespace vsk {
@@ -630,7 +633,7 @@ static void launch_adc16(vsk_ctx *ctx, const AdcArgs &in, bool dense) {
 template <int DS>
 __global__ __launch_bounds__(256) void k_pq_plane(const uint8_t *codes, int64_t n, int32_t M,
                                                   int32_t ksub, const float *cb, int32_t ldb,
-                                                  uint16_t *plane, float *sq,
+                                                  float scale, uint16_t *plane, float *sq,
                                                   uint32_t *maxbits) {
 #pragma clang fp contract(off)
   const int rpb = 256 / M;
@@ -645,14 +648,17 @@ __global__ __launch_bounds__(256) void k_pq_plane(const uint8_t *codes, int64_t 
 #pragma unroll
     for (int j = 0; j < DS; ++j) {
       const float v = c[j];
-      h[j] = bf16_rn(v);
-      const float hv = __uint_as_float((uint32_t)h[j] << 16);
-      const float rv = v - hv;
+      const float vs = v * scale;
+      const _Float16 hf = plane_f16(vs);
+      h[j] = __builtin_bit_cast(uint16_t, hf);
+      const float hv = (float)hf;
+      const float rv = vs - hv;  // exact
       s2 = s2 + v * v;
       sh += (double)hv * (double)hv;
       sr += (double)rv * (double)rv;
     }
-    uint16_t *dst = plane + r * ldb + m * DS;
+    // (DS divides 64: a segment lies in one stage)
+    uint16_t *dst = plane + plane_at(r, m * DS, ldb);
     if constexpr (DS % 2 == 0) {
 #pragma unroll
       for (int j = 0; j < DS; j += 2)
@@ -669,8 +675,10 @@ __global__ __launch_bounds__(256) void k_pq_plane(const uint8_t *codes, int64_t 
     sr += __shfl_xor(sr, o);
   }
   if (valid && m == 0) sq[r] = s2;
-  uint32_t mh = valid ? __float_as_uint(f_up(sqrt(sh) * (1.0 + 1e-12))) : 0u;
-  uint32_t mr = valid ? __float_as_uint(f_up(sqrt(sr) * (1.0 + 1e-12))) : 0u;
+  const double back = 1.0 / (double)scale;
+  uint32_t mh = valid ? __float_as_uint(f_up(sqrt(sh) * back * (1.0 + 1e-12))) : 0u;
+  uint32_t mr =
+      valid ? __float_as_uint(f_up((sqrt(sr) + 0x1p-100) * back * (1.0 + 1e-12))) : 0u;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const uint32_t a = __shfl_xor(mh, o), b = __shfl_xor(mr, o);
@@ -783,10 +791,26 @@ __global__ __launch_bounds__(256) void k_pq_rescore_keys(
 static void pq_screen_plane(vsk_ctx *ctx, const vsk_pq *pq) {
   if (pq->xrows == pq->n && pq->xplane.p) return;
   const int32_t ldb = (pq->d + 63) & ~63;
-  pq->xplane.reserve(sizeof(uint16_t) * (size_t)pq->n * ldb);
+  pq->xplane.reserve(plane_bytes(pq->n, ldb));
   pq->xsq.reserve(sizeof(float) * (size_t)pq->n);
   uint16_t *plane = pq->xplane.as<uint16_t>();
-  if (ldb > pq->d) fill_i32(ctx, reinterpret_cast<int32_t *>(plane), (int64_t)pq->n * ldb / 2, 0);
+  if (ldb > pq->d)
+    fill_i32(ctx, reinterpret_cast<int32_t *>(plane), (int64_t)(plane_bytes(pq->n, ldb) / 4), 0);
+  // a power of two for the plane from the largest row the codebooks can make
+  float most = 0.f;
+  for (int32_t m = 0; m < pq->M; ++m) {
+    float mx = 0.f;
+    for (int32_t c = 0; c < pq->ksub; ++c) {
+      const float *w = pq->host_codebooks.data() + ((size_t)m * pq->ksub + c) * pq->dsub;
+      float s = 0.f;
+      for (int32_t j = 0; j < pq->dsub; ++j) s += w[j] * w[j];
+      mx = s > mx ? s : mx;
+    }
+    most += mx;
+  }
+  uint32_t mbits;
+  std::memcpy(&mbits, &most, sizeof mbits);
+  const float sc = pq->xscale = plane_scale(mbits);
   uint32_t *mb = static_cast<uint32_t *>(ctx->scratch_ptr("pq.planemax", 2 * sizeof(uint32_t)));
   fill_i32(ctx, reinterpret_cast<int32_t *>(mb), 2, 0);
   const int64_t rpb = 256 / pq->M;
@@ -797,12 +821,12 @@ static void pq_screen_plane(vsk_ctx *ctx, const vsk_pq *pq) {
     const uint8_t *codes = pq->codes.as<uint8_t>();
     float *sq = pq->xsq.as<float>();
     switch (pq->dsub) {
-    case 1: k_pq_plane<1><<<grid, 256, 0, ctx->stream>>>(codes, pq->n, pq->M, pq->ksub, cb, ldb, plane, sq, mb); break;
-    case 2: k_pq_plane<2><<<grid, 256, 0, ctx->stream>>>(codes, pq->n, pq->M, pq->ksub, cb, ldb, plane, sq, mb); break;
-    case 4: k_pq_plane<4><<<grid, 256, 0, ctx->stream>>>(codes, pq->n, pq->M, pq->ksub, cb, ldb, plane, sq, mb); break;
-    case 8: k_pq_plane<8><<<grid, 256, 0, ctx->stream>>>(codes, pq->n, pq->M, pq->ksub, cb, ldb, plane, sq, mb); break;
-    case 16: k_pq_plane<16><<<grid, 256, 0, ctx->stream>>>(codes, pq->n, pq->M, pq->ksub, cb, ldb, plane, sq, mb); break;
-    default: k_pq_plane<32><<<grid, 256, 0, ctx->stream>>>(codes, pq->n, pq->M, pq->ksub, cb, ldb, plane, sq, mb); break;
+    case 1: k_pq_plane<1><<<grid, 256, 0, ctx->stream>>>(codes, pq->n, pq->M, pq->ksub, cb, ldb, sc, plane, sq, mb); break;
+    case 2: k_pq_plane<2><<<grid, 256, 0, ctx->stream>>>(codes, pq->n, pq->M, pq->ksub, cb, ldb, sc, plane, sq, mb); break;
+    case 4: k_pq_plane<4><<<grid, 256, 0, ctx->stream>>>(codes, pq->n, pq->M, pq->ksub, cb, ldb, sc, plane, sq, mb); break;
+    case 8: k_pq_plane<8><<<grid, 256, 0, ctx->stream>>>(codes, pq->n, pq->M, pq->ksub, cb, ldb, sc, plane, sq, mb); break;
+    case 16: k_pq_plane<16><<<grid, 256, 0, ctx->stream>>>(codes, pq->n, pq->M, pq->ksub, cb, ldb, sc, plane, sq, mb); break;
+    default: k_pq_plane<32><<<grid, 256, 0, ctx->stream>>>(codes, pq->n, pq->M, pq->ksub, cb, ldb, sc, plane, sq, mb); break;
     }
     check_launch("pq_screen_plane");
   }
@@ -1202,7 +1226,7 @@ static vsk_status pq_search_body(vsk_ctx *ctx, const vsk_pq *pq, const float *q,
   uint64_t *sthr = nullptr;
   if (screen) {
     pq_screen_plane(ctx, pq);
-    qp = argmin_queries(ctx, dq, nq, pq->d, pq->d, "pq.sq");
+    qp = half_argmin_queries(ctx, dq, nq, pq->d, pq->d, "pq.sq");
     sthr = static_cast<uint64_t *>(ctx->scratch_ptr("pq.sthr", sizeof(uint64_t) * nq));
   }
   for (int64_t b0 = 0; b0 < nq; b0 += qb) {
@@ -1237,6 +1261,8 @@ static vsk_status pq_search_body(vsk_ctx *ctx, const vsk_pq *pq, const float *q,
         SplitPtrs sp{};
         sp.xh = pq->xplane.as<uint16_t>();
         sp.qh = qp.qh + b0 * qp.ldb;
+        sp.qsc = qp.qsc + b0;
+        sp.xscale = pq->xscale;
         sp.ldxb = pq->xldb;
         sp.ldqb = qp.ldb;
         sp.kb = pq->xldb;

@@ -228,7 +228,10 @@ __device__ void wave_sort_u64(uint64_t (&v)[R]) {
 // is used: with few queries a launch (a workgroup or two a CU) each pass
 // otherwise waits on the memory latency once per segment.  The loads' registers
 // cost occupancy, which launches of many queries need more.
-template <int REG, bool W32, bool FAST = false, int SEGB = 0>
+// SEGL: a segmented list of at most SEGL keys with the previous list is
+// compacted into LDS on its first reading, and every further pass reads it
+// there (200,003 x 384, 333 queries: 20 us a call).
+template <int REG, bool W32, bool FAST = false, int SEGB = 0, int SEGL = 0>
 __global__ __launch_bounds__(SEL_THREADS) void k_select(SelectArgs a) {
   // (a split selection's output list: run q % split_n of query q / split_n)
   const int64_t q = blockIdx.x;
@@ -285,7 +288,15 @@ __global__ __launch_bounds__(SEL_THREADS) void k_select(SelectArgs a) {
         regs[r] = i < total ? sel_elem<W32>(P, np, C, C32, i0, i) : VSK_KEY_NONE;
     }
   }
+  __shared__ uint64_t lkeys[SEGL > 0 ? SEGL : 1];
+  __shared__ int lcount;
+  bool inlds = false;
+  int ln = 0;
   auto each_key = [&](auto &&f) {
+    if (SEGL > 0 && inlds) {
+      for (int i = tid; i < ln; i += SEL_THREADS) f(lkeys[i]);
+      return;
+    }
     if (inreg) {
 #pragma unroll
       for (int r = 0; r < REG; ++r) {
@@ -337,6 +348,26 @@ __global__ __launch_bounds__(SEL_THREADS) void k_select(SelectArgs a) {
   __shared__ SelShared sh;
   __shared__ uint64_t sel[VSK_MAX_K];
   __shared__ int sel_count;
+  if constexpr (SEGL > 0) {
+    if (seg) {
+      int own = 0;  // the segments' keys
+      for (int s = tid; s < a.nseg; s += SEL_THREADS) own += seg_cnt[s];
+      if (tid == 0) lcount = (int)np;
+      __syncthreads();
+      if (own) atomicAdd(&lcount, own);
+      __syncthreads();
+      ln = lcount;
+      __syncthreads();
+      if (ln <= SEGL) {  // uniform
+        if (tid == 0) lcount = 0;
+        __syncthreads();
+        each_key([&](uint64_t key) { lkeys[atomicAdd(&lcount, 1)] = key; });
+        __syncthreads();
+        ln = lcount;
+        inlds = true;
+      }
+    }
+  }
   // Short cut for k <= 128 over a list in registers: each wave's k-th
   // smallest of its lanes' smallest keys (k <= 64) or of their two smallest
   // keys (k <= 128) has k keys at or below it, so the smallest of those
@@ -1588,10 +1619,19 @@ void launch_select(vsk_ctx *ctx, const SelectArgs &a, const char *name) {
   const bool fast = a.k <= 128 && !a.seg_n;
   if (a.cand32) {
     if (a.prev || a.seg_n) fail(VSK_ERR_INVALID_ARGUMENT, "32-bit lists take no previous list or segments");
-    if (a.k <= 128)
-      k_select<64, true, true><<<(unsigned)a.nq, SEL_THREADS, 0, ctx->stream>>>(a);
+    // (as few registers as hold the list: 2,048 words a query over 10,000
+    // queries took 113 us with 8 a thread, 316 with 64)
+    const unsigned g = (unsigned)a.nq;
+#define SEL_W32(R)                                                              \
+  (a.k <= 128 ? k_select<R, true, true><<<g, SEL_THREADS, 0, ctx->stream>>>(a) \
+              : k_select<R, true><<<g, SEL_THREADS, 0, ctx->stream>>>(a))
+    if (a.cap <= 8 * SEL_THREADS)
+      SEL_W32(8);
+    else if (a.cap <= 32 * SEL_THREADS)
+      SEL_W32(32);
     else
-      k_select<64, true><<<(unsigned)a.nq, SEL_THREADS, 0, ctx->stream>>>(a);
+      SEL_W32(64);
+#undef SEL_W32
   } else if (a.regs && !a.seg_off && most > 32 * SEL_THREADS) {
     if (fast)
       k_select<64, false, true><<<(unsigned)a.nq, SEL_THREADS, 0, ctx->stream>>>(a);
@@ -1602,6 +1642,9 @@ void launch_select(vsk_ctx *ctx, const SelectArgs &a, const char *name) {
       k_select<32, false, true><<<(unsigned)a.nq, SEL_THREADS, 0, ctx->stream>>>(a);
     else
       k_select<32, false><<<(unsigned)a.nq, SEL_THREADS, 0, ctx->stream>>>(a);
+  } else if (a.seg_n && a.nq < 4 * (int64_t)ctx->cu_count && a.k <= 512) {
+    // (chunks are expected to bring eight times k keys: up to 4,096)
+    k_select<0, false, false, 8, 4096><<<(unsigned)a.nq, SEL_THREADS, 0, ctx->stream>>>(a);
   } else if (a.seg_n && a.nq < 4 * (int64_t)ctx->cu_count) {
     k_select<0, false, false, 8><<<(unsigned)a.nq, SEL_THREADS, 0, ctx->stream>>>(a);
   } else {
@@ -1701,7 +1744,7 @@ void progressive_topk(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t k,
     int64_t seg_stride = 0;
     {
       ScanRequest rq{r0, r0 + c, thresh, nullptr, cand, cap, counts, dense};
-      if (words && dense && c >= n) rq.cand32 = reinterpret_cast<uint32_t *>(cand);
+      if (words && dense) rq.cand32 = reinterpret_cast<uint32_t *>(cand);
       if (!dense && seg_n) {
         rq.seg_n = seg_n;
         rq.seg_nseg = &nseg;
@@ -1714,7 +1757,7 @@ void progressive_topk(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t k,
     sa.k = k;
     sa.prev = dense ? nullptr : best;
     sa.cand = cand;
-    if (words && dense && c >= n) sa.cand32 = reinterpret_cast<const uint32_t *>(cand);
+    if (words && dense) sa.cand32 = reinterpret_cast<const uint32_t *>(cand);
     sa.cap = cap;
     sa.counts = dense ? nullptr : counts;
     sa.best_out = best;

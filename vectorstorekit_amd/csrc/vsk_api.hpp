@@ -113,9 +113,9 @@ struct ScanRequest {
   int32_t *seg_n = nullptr;
   int32_t *seg_nseg = nullptr;
   int64_t *seg_stride = nullptr;
-  // set (instead of cand) where a dense chunk holds the whole database and
-  // the caller's scan takes it (progressive_topk's words): 32-bit ordered
-  // distances, row r's at cand32[q*cap + r]
+  // set (instead of cand) for the first chunk where the caller's scan takes
+  // it (progressive_topk's words): 32-bit ordered distances, row r's at
+  // cand32[q*cap + r]
   uint32_t *cand32 = nullptr;
 };
 using ScanFn = std::function<void(const ScanRequest &)>;
@@ -140,9 +140,9 @@ struct TopkWorkspace {
 // holds at most cap/(2k) times the rows already seen, and at most max_growth
 // times when that is positive.
 // ws: the buffers to use (sized for nq and min(cap, n)); null = the
-// context's scratch slots.  words: a dense chunk of every row may be asked
-// for as 32-bit distances (half the bytes written and selected from; the
-// row is the position).
+// context's scratch slots.  words: the first chunk may be asked for as
+// 32-bit distances (half the bytes written and selected from; the row is the
+// position).
 void progressive_topk(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t k,
                       int64_t cap, const ScanFn &scan, uint64_t *best,
                       const char *select_name, int64_t max_growth = 0,

@@ -190,17 +190,28 @@ struct vsk_db {
   vsk::DevBuf x;       // n x ld fp32
   vsk::DevBuf sqnorm;  // n: sum x^2 (fp32)
   vsk::DevBuf norm;    // n: sqrt(sum x^2)
-  // bf16 hi/lo planes for the bf16 MFMA kernels, built on first use (the
-  // lo plane only for the bf16x3 kernel; the screen reads hi alone), and
-  // the maxima over the rows of |hi| and |x - hi| (the screen's bound)
+  // row-major bf16 hi/lo planes for the bf16x3 kernel and the IVF probe's
+  // screen, built
+  // on first use (the lo plane only for bf16x3), and the maxima over the rows
+  // of |hi| and |x - hi|
   mutable vsk::DevBuf split, split_lo;
+  // the flat screen's tiled planes of the rows, [0] fp16, [1] bf16 (normalised
+  // cosine), each made by the first search that screens with it: the state on
+  // the device (half_rows) and, read back, the maxima of |h| and |x - h|
+  struct ScreenPlane {
+    vsk::DevBuf h, state;
+    float max_hi = 0.f, max_res = 0.f;
+  };
+  mutable ScreenPlane plane[2];
   // the reference's |x| per row (seq_norms), built when the exact cosine
   // first needs it
   mutable vsk::DevBuf seqnorm;
-  // the screen's bound for cosine: maxima over the rows with 0 < |x| of
-  // |bf16(x)| / |x| and |x - bf16(x)| / |x| (|x| the fp32 norm above);
-  // cos_state 0 = not made, 1 = made, -1 = a row's norm is too small or not
-  // finite for the bound (cosine then takes the exact scan)
+  // the screen's plane for cosine: the rows over their fp32 norms in fp16,
+  // 1e-8 / |x| per row, and the maxima over the rows with 0 < |x| of the
+  // plane rows' norms and residuals; cos_state 0 = not made, 1 = made, -1 = a
+  // row's norm is too small or not finite for the bound (cosine then takes
+  // the exact scan)
+  mutable vsk::DevBuf cos_half, cos_inv;
   mutable int32_t cos_state = 0;
   mutable float cos_rel_hi = 0.f, cos_rel_res = 0.f;
   mutable int32_t ldb = 0;
