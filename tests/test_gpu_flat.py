@@ -327,6 +327,24 @@ def test_screen_planes_and_chunks(sctx, metric, scale):
         np.testing.assert_array_equal(gd, od)
 
 
+@pytest.mark.parametrize("nq", [256, 257, 513, 769, 1025, 1281])
+def test_query_tile_groups(sctx, nq):
+    """Query tiles that fill a group of the screen's launch (256 queries, four
+    tiles a group) and of the three-pass kernel's (128 a tile) only in part:
+    every tile is scanned over every row.  Screen bit for bit; three-pass
+    within the float bar."""
+    from vectorstorekit_amd.engine import Context, HIPAccelerationConfiguration
+
+    x, q = _data(nq, 20_001, nq, 64)
+    print(f"query tile groups nq={nq}", flush=True)
+    _check(sctx, x, q, 10, METRIC_L2SQ, exact=True)
+    c = Context(0, configuration=HIPAccelerationConfiguration(kernel="bf16x3"))
+    try:
+        _check(c, x, q, 10, METRIC_L2SQ)
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("metric", SCREEN)
 def test_small_problem_exact_scan(ctx, metric):
     """Config 1's size (at most 2^28 query x row x dimension terms) takes the

@@ -726,7 +726,7 @@ void approx_topk(vsk_ctx *ctx, const vsk_db *db, const float *dq, int64_t nq,
   // tiles spreads a query's slots over some 56 workgroups, about 18
   // candidates in 36 slots each, and of 333 queries one or two overflowed:
   // the call ran again, its chunks re-scanned (200,003 x 384, k = 50:
-  // 1.52 ms a call, now 0.37).
+  // 1.52 ms a call, with room 0.37).
   if (passes == 1 && nq <= 1024 && ctx->max_tile_bytes <= 0) {
     // (whole row tiles, so that every chunk starts on one)
     cap = std::max<int64_t>(cap, std::min<int64_t>(ceil_div(32 * (int64_t)k, 256) * 256, 16384));

@@ -272,9 +272,10 @@ __host__ __device__ inline float plane_scale(uint32_t maxsq_bits) {
 }
 // The screen's row planes are stored as the screen copies them: for each tile
 // of 256 rows and stage of 64 columns, 256 x 64 values (32 contiguous KB).
-// From row-major planes a stage is 256 pieces of 128 bytes a pitch apart,
-// which streamed from HBM at 0.9 TB/s when one query tile left nothing to
-// reuse (1M x 768, 64 queries: 1.45 ms, now 1.27).  Planes hold whole tiles.
+// From row-major planes a stage is 256 pieces of 128 bytes a pitch apart:
+// 1M x 768, filter launches of 1,024 queries 1.48 ms, tiled 1.36; of 512
+// queries 0.80 and 0.73; below, and at 128 dimensions, within 3 %.  Planes
+// hold whole tiles.
 __host__ __device__ inline int64_t plane_at(int64_t r, int32_t c, int32_t ldb) {
   return (((r >> 8) * (ldb >> 6) + (c >> 6)) << 14) + ((r & 255) << 6) + (c & 63);
 }
