@@ -74,6 +74,33 @@ def test_ivf_pq_bit_exact(ctx, shape):
     np.testing.assert_array_equal(ids, ei)
 
 
+@pytest.mark.parametrize("shape", [(300, 900, 16, 4, 5, 300, 30), (260, 3000, 8, 2, 6, 257, 20),
+                                   (513, 700, 3, 4, 4, 513, 9), (1, 513, 16, 2, 3, 1, 5),
+                                   (2, 256, 8, 4, 3, 2, 256)])
+def test_ivf_pq_position_sequence(ctx, shape):
+    """The code scan's threads walk a query's positions as one sequence over
+    its probed lists: more probes than the 256 it holds at a time, lists that
+    are empty or a few rows long, sequences that end on either of a thread's
+    two rows; rows read as one load (M = 16, 8) and word by word."""
+    nlist, n, M, dsub, nq, nprobe, k = shape
+    d = M * dsub
+    rng = np.random.default_rng(nlist + M)
+    x = rng.standard_normal((n, d)).astype(np.float32)
+    q = rng.standard_normal((nq, d)).astype(np.float32)
+    c = rng.standard_normal((nlist, d)).astype(np.float32)
+    c[::7] += 100  # empty lists
+    cb = x[rng.choice(n, 256, replace=False)].reshape(256, M, dsub).transpose(1, 0, 2).copy()
+    idx = _index(ctx, c, x, nprobe)
+    pq = ProductQuantizer(ctx, cb)
+    idx.encodePQ(pq)
+    print(f"pq position sequence {shape}", flush=True)
+    dist, ids = idx.searchPQ(q, k)
+    ed, ei = O.ivf_pq_search(q, cb, O.pq_encode(x, cb), np.arange(n), O.ivf_assign(x, c), c,
+                             nprobe, k)
+    np.testing.assert_array_equal(dist, ed)
+    np.testing.assert_array_equal(ids, ei)
+
+
 def test_ivf_sq8_all_lists_is_the_flat_sq8_scan(ctx):
     x, q, c = _mixture(5, 16, 4000, 64, 30)
     idx = _index(ctx, c, x, 16)

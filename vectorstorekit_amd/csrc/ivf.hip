@@ -674,29 +674,69 @@ __global__ __launch_bounds__(64) void k_list_stream(DirectScanArgs a) {
 // (sum, position).  One workgroup per query: its tables stay in LDS while it
 // walks its probed lists (a table is 4 M ksub bytes, a probed list's codes
 // a few KB, so keeping the table and streaming the codes moves the least).
+//
+// The query's candidate positions run through its lists without a gap, so the
+// threads take them 256 apart as one sequence, two at a time, each moving its
+// list forward when it passes an end: no list's last threads idle, and no
+// list waits for the one before.  Bound: the LDS lookups, 64 random banks
+// each (about 5 cycles: 175 us of the time below).  MW > 0: rows of 4 MW
+// codes with 256 codewords a segment, read as one load, every lookup's
+// segment an immediate offset.  1M rows in 4,096 lists, M = 16, 10,000
+// queries, 32 probes: 219 us; list by list, one row a thread, 545.
+template <int MW>
 __global__ __launch_bounds__(256) void k_list_scan_pq_q(ListScanArgs a) {
 #pragma clang fp contract(off)
+  constexpr int PB = 256;  // probes at a time
   extern __shared__ float tl[];  // M x ksub
+  __shared__ uint32_t s_end[PB];  // the position after each probe's list
+  __shared__ int64_t s_row[PB];   // its first row less its first position
   const int64_t q = blockIdx.x;
-  const int tsz = a.M * a.ksub;
-  for (int i = threadIdx.x; i < tsz; i += blockDim.x) tl[i] = a.lut[q * tsz + i];
-  __syncthreads();
-  const int64_t seg = a.wseg[q];
-  for (int p = 0; p < a.np; ++p) {
-    const int32_t l = a.probes[q * a.np + p];
-    if (l < 0) continue;
-    const int64_t v0 = a.list_off[l], v1 = a.list_off[l + 1];
-    const int64_t tb = a.pos_base[q * a.np + p];
-    for (int64_t v = v0 + threadIdx.x; v < v1; v += blockDim.x) {
-      const uint32_t *x = reinterpret_cast<const uint32_t *>(a.codes + v * a.cstride);
-      float acc = 0.f;
-      for (int m0 = 0; m0 < a.M; m0 += 4) {
-        const uint32_t w = x[m0 >> 2];
-        const int mm = a.M - m0 < 4 ? a.M - m0 : 4;
-        for (int t = 0; t < mm; ++t)
-          acc = acc + tl[(m0 + t) * a.ksub + (int)((w >> (8 * t)) & 0xFFu)];
+  const int tsz = a.M * a.ksub, tid = threadIdx.x;
+  for (int i = tid; i < tsz; i += 256) tl[i] = a.lut[q * tsz + i];
+  uint32_t *words = a.words + a.wseg[q];
+  auto row_of = [&](uint32_t t, int &p) {
+    while (t >= s_end[p]) ++p;
+    return a.codes + ((int64_t)t + s_row[p]) * a.cstride;
+  };
+  for (int p0 = 0; p0 < a.np; p0 += PB) {
+    const int n = a.np - p0 < PB ? a.np - p0 : PB;
+    if (p0) __syncthreads();
+    if (tid < n) {
+      const int32_t l = a.probes[q * a.np + p0 + tid];
+      const int64_t base = a.pos_base[q * a.np + p0 + tid];
+      const int64_t v0 = l < 0 ? 0 : a.list_off[l], v1 = l < 0 ? 0 : a.list_off[l + 1];
+      s_end[tid] = (uint32_t)(base + (v1 - v0));
+      s_row[tid] = v0 - base;
+    }
+    __syncthreads();
+    const uint32_t hi = s_end[n - 1];
+    int p = 0;
+    for (uint32_t t = (uint32_t)a.pos_base[q * a.np + p0] + tid; t < hi; t += 512) {
+      const bool two = t + 256 < hi;  // (else the first row again)
+      const uint8_t *x0 = row_of(t, p);
+      const uint8_t *x1 = two ? row_of(t + 256, p) : x0;
+      float s0 = 0.f, s1 = 0.f;
+      if constexpr (MW > 0) {
+        typedef uint32_t wv __attribute__((ext_vector_type(MW)));
+        const wv w0 = *reinterpret_cast<const wv *>(x0), w1 = *reinterpret_cast<const wv *>(x1);
+#pragma unroll
+        for (int m = 0; m < 4 * MW; ++m) {
+          s0 = s0 + tl[m * 256 + ((w0[m >> 2] >> (8 * (m & 3))) & 0xFFu)];
+          s1 = s1 + tl[m * 256 + ((w1[m >> 2] >> (8 * (m & 3))) & 0xFFu)];
+        }
+      } else {
+        for (int m0 = 0; m0 < a.M; m0 += 4) {
+          const uint32_t w0 = *reinterpret_cast<const uint32_t *>(x0 + m0);
+          const uint32_t w1 = *reinterpret_cast<const uint32_t *>(x1 + m0);
+          const int mm = a.M - m0 < 4 ? a.M - m0 : 4;
+          for (int u = 0; u < mm; ++u) {
+            s0 = s0 + tl[(m0 + u) * a.ksub + (int)((w0 >> (8 * u)) & 0xFFu)];
+            s1 = s1 + tl[(m0 + u) * a.ksub + (int)((w1 >> (8 * u)) & 0xFFu)];
+          }
+        }
       }
-      a.words[seg + tb + (v - v0)] = vsk_f2ord(acc);
+      words[t] = vsk_f2ord(s0);
+      if (two) words[t + 256] = vsk_f2ord(s1);
     }
   }
 }
@@ -2379,7 +2419,13 @@ static vsk_status ivf_search_any(vsk_ctx *ctx, const vsk_ivf *ivf, const float *
       } else if (kind == 1) {
         VSK_SCAN_QG(k_list_scan_sq8)
       } else {
-        k_list_scan_pq_q<<<(unsigned)nb, 256, (size_t)per_q, ctx->stream>>>(la);
+        // (code rows are aligned to their stride's powers of two)
+        if (la.ksub == 256 && la.M == 16 && la.cstride % 16 == 0)
+          k_list_scan_pq_q<4><<<(unsigned)nb, 256, (size_t)per_q, ctx->stream>>>(la);
+        else if (la.ksub == 256 && la.M == 8 && la.cstride % 8 == 0)
+          k_list_scan_pq_q<2><<<(unsigned)nb, 256, (size_t)per_q, ctx->stream>>>(la);
+        else
+          k_list_scan_pq_q<0><<<(unsigned)nb, 256, (size_t)per_q, ctx->stream>>>(la);
       }
 #undef VSK_SCAN_QG
       check_launch(names[kind]);
