@@ -345,6 +345,21 @@ def test_query_tile_groups(sctx, nq):
         c.close()
 
 
+def test_chunk_counters_between_batches(sctx):
+    """Chunk counters cleared by the chunk before: several filtered chunks a
+    call, the same call again, and calls of more and
+    of fewer queries in between (the counters' two sets move with the number
+    of queries); bit for bit the oracle."""
+    x, q = _data(77, 60_000, 300, 32)
+    db = VectorDatabase(sctx, x)
+    ref = {m: O.search_flat(q[:m], x, 9, METRIC_L2SQ) for m in (1, 37, 300)}
+    for m in (37, 300, 1, 37, 37, 300):
+        print(f"chunk counters nq={m}", flush=True)
+        gd, gi = db.search(q[:m], 9, METRIC_L2SQ)
+        np.testing.assert_array_equal(gi, ref[m][1])
+        np.testing.assert_array_equal(gd, ref[m][0])
+
+
 @pytest.mark.parametrize("metric", SCREEN)
 def test_small_problem_exact_scan(ctx, metric):
     """Config 1's size (at most 2^28 query x row x dimension terms) takes the

@@ -72,6 +72,7 @@ struct FlatArgs {
   // screen kernel, filter mode: segmented lists (segment = row split, at
   // q*cap + split*sub) with their key counts here (nq x nseg), else null
   int32_t *seg_n;
+  int32_t nseg;  // their number: the row splits that have rows
   // MODE_ARGMIN: the winning distance per query (optional)
   float *amin;
 };

@@ -1292,7 +1292,7 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
       // past the slots: the query re-scans the chunk
       if (n > lim) atomicAdd(&a.counts[q0 + tid], (int32_t)a.cap + 1);
       if (a.seg_n) {
-        a.seg_n[(q0 + tid) * (int64_t)(8 * a.splits_per_xcd) + split] = n < lim ? n : lim;
+        a.seg_n[(q0 + tid) * (int64_t)a.nseg + split] = n < lim ? n : lim;
       } else if (n <= lim) {
         const int64_t pb = s_pb[tid];
         for (int32_t i = n; i < lim; ++i) a.cand[pb + i] = VSK_KEY_NONE;
@@ -1436,9 +1436,10 @@ void launch_flat_screen(vsk_ctx *ctx, FlatArgs a, const SplitPtrs &s, int mode,
   }
   if (mode != MODE_FILTER || splits > VSK_MAX_SEG || !nseg || !stride) a.seg_n = nullptr;
   if (a.seg_n) {
-    // splits without rows launch no writes: their segments start empty
-    fill_i32(ctx, a.seg_n, (int64_t)a.nq * splits, 0);
-    *nseg = (int32_t)splits;
+    // every split with rows writes its active queries' counts
+    a.nseg = (int32_t)ceil_div(tiles, a.rows_per_split / XS_N);
+    if (a.active) fill_i32(ctx, a.seg_n, (int64_t)a.nq * a.nseg, 0);
+    *nseg = a.nseg;
     *stride = a.sub;
   }
   const int64_t nblocks = a.qtiles_per_xcd ? 8 * (int64_t)a.qtiles_per_xcd * splits

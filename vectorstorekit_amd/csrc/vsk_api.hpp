@@ -87,6 +87,9 @@ struct SelectArgs {
   // best_out[(q * split_n + s) * k] (split_n = ceil(cap / split_len); no
   // counts, previous list, segments or thresholds)
   int32_t split_len = 0;
+  // the next chunk's append counters (one a query) and the call's overflow
+  // counter, cleared here where set: a launch each otherwise
+  int32_t *next_counts = nullptr, *next_overflow = nullptr;
 };
 // the largest k of a split selection
 constexpr int32_t VSK_SPLIT_K = 128;
