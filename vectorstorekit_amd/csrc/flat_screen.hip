@@ -1,12 +1,14 @@
 // flat_screen.hip -- exact flat top-k for L2^2, L2, cosine (the reference's
-// epsilon form), normalised cosine and dot: a one-pass bf16 MFMA screen, a
+// epsilon form), normalised cosine and dot: a one-pass 16-bit MFMA screen, a
 // proven bound on its error, and an fp32 rescore of the survivors in the CPU
 // reference's own summation order.
 //
-// Bound.  With qh = bf16(q), xh = bf16(x) and the exact residuals
+// Bound.  With qh, xh the 16-bit values the screen multiplies (fp16 under a
+// power of two per query and per database; bf16 for normalised cosine; the
+// epsilon cosine's rows divided by their norms first) and the exact residuals
 // dq = q - qh, dx = x - xh, Cauchy-Schwarz gives
 //   |q.x - qh.xh| <= |qh||dx| + |dq||xh| + |dq||dx|.
-// Each product qh_i xh_i is exact in fp32 (8-bit significands), and any fp32
+// Each product qh_i xh_i is exact in fp32 (11-bit significands), and any fp32
 // summation of d of them, in any order and with round-to-nearest or
 // truncation, errs by at most 2(d-1)u sum|qh_i xh_i| <= 2(d-1)u |qh||xh|,
 // u = 2^-24.  Taking the maxima of |xh| and |dx| over the rows bounds every

@@ -35,7 +35,7 @@ struct vsk_pq {
   std::vector<float> host_codebooks;  // the same, for identity checks and files
   vsk::DevBuf codes;      // n x M uint8
   int64_t n = 0, cap_rows = 0;
-  // the bf16 screen of the ADC scan: the decoded rows x^ (each segment's
+  // the fp16 screen of the ADC scan: the decoded rows x^ (each segment's
   // codeword) as an fp16 plane of xldb columns, |x^|^2 per row, and the
   // maxima over the rows of |h| and |x^ - h|; made by the
   // first screened search and again when rows were added since (xrows)
@@ -617,11 +617,11 @@ static void launch_adc16(vsk_ctx *ctx, const AdcArgs &in, bool dense) {
 }
 
 // ---------------------------------------------------------------------------
-// The ADC scan through the bf16 matrix cores.  The ADC distance of a row is
+// The ADC scan through the 16-bit matrix cores.  The ADC distance of a row is
 // a sequential fp32 sum of d squared differences q_j - x^_j (segment by
 // segment, then over the segments), x^ the row's decoded codewords: the
 // same kind of sum the flat screen's L2^2 bound covers.  So the flat screen
-// kernel runs over the decoded rows (a bf16 plane) and keeps every row whose
+// kernel runs over the decoded rows (an fp16 plane) and keeps every row whose
 // screened distance a(x) is within eps(q) of the query's exact threshold
 // key: a row whose ADC key is at most that threshold has a(x) <= ADC + eps.
 // The survivors' keys are then rescored exactly (the LUT sum in m order,
@@ -695,7 +695,7 @@ __global__ __launch_bounds__(256) void k_pq_plane(const uint8_t *codes, int64_t 
 // distance plus eps(q), every row id (NONE stays NONE).  eps is the flat
 // screen's L2^2 bound with x^ for x: 2 e_dot + (2d + 8) u (|q| + |x^|)^2,
 // where e_dot = |qh||dx| + |dq||xh| + |dq||dx| + 2(d-1)u|qh||xh| bounds the
-// bf16 dot's error and the second term the rounding of |q|^2, |x^|^2, the
+// screened dot's error and the second term the rounding of |q|^2, |x^|^2, the
 // screen's last operations and the ADC sum itself (at most d + 2 roundings of
 // a sum bounded by (|q| + |x^|)^2).
 __global__ void k_pq_screen_thresh(const uint64_t *thresh, int64_t nq, const float *qnh,
@@ -1212,7 +1212,7 @@ static vsk_status pq_search_body(vsk_ctx *ctx, const vsk_pq *pq, const float *q,
   pq_lut_device(ctx, pq, dq, nq, lut);
   uint64_t *best = static_cast<uint64_t *>(
       ctx->scratch_ptr("pq.best", sizeof(uint64_t) * nq * k_adc));
-  // the bf16 screen: decoded rows (kept with the codes), the queries' bf16
+  // the fp16 screen: decoded rows (kept with the codes), the queries' fp16
   // plane and norms, a threshold slot per query.  Its chunks grow at most
   // 4-8x: the survivors (k_adc times the growth, plus the bound's band) then
   // stay well inside the screen's 256 slots per (row split, query), whose
@@ -1239,7 +1239,7 @@ static vsk_status pq_search_body(vsk_ctx *ctx, const vsk_pq *pq, const float *q,
     base.nq = (int32_t)nb;
     ScanFn scan = [&](const ScanRequest &r) {
       if (!r.dense && screen) {
-        // filtered chunks: the bf16 screen over the decoded rows, then the
+        // filtered chunks: the fp16 screen over the decoded rows, then the
         // survivors' exact keys
         k_pq_screen_thresh<<<(unsigned)ceil_div(nb, 256), 256, 0, ctx->stream>>>(
             r.thresh, nb, qp.qnh + b0, qp.qnr + b0, pq->xh_max, pq->xr_max, pq->d, sthr);
