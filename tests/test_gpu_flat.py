@@ -297,6 +297,27 @@ def test_stream_scan_edges(ctx, metric):
         np.testing.assert_array_equal(db.distances(q, metric), O.distances(q, x, metric))
 
 
+@pytest.mark.parametrize("shape", [(64, 70, 32), (111, 1798, 32), (505, 513, 40), (4032, 130, 33),
+                                   (4033, 130, 33), (4097, 900, 33), (2000, 1251, 128),
+                                   (10_001, 257, 97)])
+def test_exact_scan_many_queries(ctx, shape):
+    """The exact scan of many queries over few rows: row tiles on both sides
+    of the 64 where the stream gives each tile an XCD of its own, one to eight
+    queries a wave, and the 64 x 32 tiles; bit for bit the oracle."""
+    n, nq, d = shape
+    x, q = _data(n + nq + d, n, nq, d)
+    x[n // 2] = np.inf
+    x[n // 3, d - 1] = np.nan
+    print(f"exact scan many queries {shape}", flush=True)
+    db = VectorDatabase(ctx, x)
+    for metric in (METRIC_L2SQ, METRIC_COSINE, METRIC_L1):
+        gd, gi = db.search(q, 10, metric)
+        od, oi = O.search_flat(q, x, 10, metric)
+        np.testing.assert_array_equal(gi, oi)
+        np.testing.assert_array_equal(gd, od)
+    np.testing.assert_array_equal(db.distances(q, METRIC_L2), O.distances(q, x, METRIC_L2))
+
+
 @pytest.mark.parametrize("metric", SCREEN)
 @pytest.mark.parametrize("scale", [2.0 ** -60, 1.0, 2.0 ** 40])
 def test_screen_planes_and_chunks(sctx, metric, scale):

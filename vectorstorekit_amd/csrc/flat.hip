@@ -359,7 +359,7 @@ __global__ __launch_bounds__(256) void k_flat_valu(FlatArgs a, int32_t *argmin) 
 // queries 95 against 167, 32 queries 159 against 173; 10,000 x 128, 1 query
 // 4.7 against 16 us, 100 queries about 15 against 18.
 template <int MODE, int OP, int V, int C>
-__global__ __launch_bounds__(64) void k_flat_stream(FlatArgs a, int32_t groups) {
+__global__ __launch_bounds__(64) void k_flat_stream(FlatArgs a, int32_t groups, int32_t few) {
 #pragma clang fp contract(off)
   constexpr int NL = C / 4;      // row loads a chunk, 16 bytes a lane
   constexpr int LD = C + 4;      // LDS row stride (floats): conflict-free 16-byte reads
@@ -369,10 +369,14 @@ __global__ __launch_bounds__(64) void k_flat_stream(FlatArgs a, int32_t groups) 
   __shared__ __attribute__((aligned(16))) float tile[64 * LD];
   __shared__ __attribute__((aligned(16))) float qt[V * C];
   const int lane = threadIdx.x;
-  // block L runs on XCD L % 8: there, groups of one row tile in turn
-  const int64_t l8 = blockIdx.x >> 3;
-  const int64_t q0 = (l8 % groups) * V;
-  const int64_t row0 = a.r0 + ((l8 / groups) * 8 + (blockIdx.x & 7)) * 64;
+  // block L runs on XCD L % 8: there, groups of one row tile in turn; with
+  // few row tiles (their number, else 0) all tiles of a group in turn
+  const uint32_t l = few ? blockIdx.x : blockIdx.x >> 3;
+  const uint32_t g = few ? l / (uint32_t)few : l % (uint32_t)groups;
+  const uint32_t t = few ? l - g * (uint32_t)few
+                         : l / (uint32_t)groups * 8 + (blockIdx.x & 7);
+  const int64_t q0 = (int64_t)g * V;
+  const int64_t row0 = a.r0 + (int64_t)t * 64;
   if (row0 >= a.r1) return;
   const int seg = lane % LPR, sub = lane / LPR;
   const int64_t last = a.r1 - 1 - row0;  // rows past the end read the last one
@@ -454,15 +458,20 @@ __global__ __launch_bounds__(64) void k_flat_stream(FlatArgs a, int32_t groups) 
 template <int OP, int V, int C>
 static void launch_stream_v(vsk_ctx *ctx, const FlatArgs &a, int mode) {
   const int64_t groups = ceil_div(a.nq, V);
-  const int64_t tiles = ceil_div(ceil_div(a.r1 - a.r0, 64), 8) * 8;
+  // A tile of its own XCD leaves up to seven XCDs of eight without work where
+  // the tiles are few (an index's centroids: 111 rows x 32, 1,798 queries used
+  // two of them: 10.5 us, now 5.6), and up to 1/8 of them at 64 tiles.
+  int64_t tiles = ceil_div(a.r1 - a.r0, 64);
+  const int32_t few = tiles < 64 ? (int32_t)tiles : 0;
+  if (!few) tiles = ceil_div(tiles, 8) * 8;
   const dim3 grid((unsigned)(groups * tiles));
   const int32_t g = (int32_t)groups;
   if (mode == MODE_DENSE)
-    k_flat_stream<MODE_DENSE, OP, V, C><<<grid, 64, 0, ctx->stream>>>(a, g);
+    k_flat_stream<MODE_DENSE, OP, V, C><<<grid, 64, 0, ctx->stream>>>(a, g, few);
   else if (mode == MODE_FILTER)
-    k_flat_stream<MODE_FILTER, OP, V, C><<<grid, 64, 0, ctx->stream>>>(a, g);
+    k_flat_stream<MODE_FILTER, OP, V, C><<<grid, 64, 0, ctx->stream>>>(a, g, few);
   else
-    k_flat_stream<MODE_MATRIX, OP, V, C><<<grid, 64, 0, ctx->stream>>>(a, g);
+    k_flat_stream<MODE_MATRIX, OP, V, C><<<grid, 64, 0, ctx->stream>>>(a, g, few);
 }
 
 // Queries a wave: as few as leave the launch about one round of resident
