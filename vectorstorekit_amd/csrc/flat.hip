@@ -500,18 +500,18 @@ static void launch_mfma(vsk_ctx *ctx, dim3 grid, const FlatArgs &a, int mode) {
     k_flat_mfma<MODE_MATRIX, METRIC><<<grid, 256, 0, ctx->stream>>>(a);
 }
 
-// the exact VALU scan in tiles of 128 rows x 64 queries
-template <int OP>
+// the exact VALU scan in tiles of 32 U rows x 8 V queries (argmin: 128 x 64)
+template <int OP, int U, int V>
 static void launch_valu_tiles(vsk_ctx *ctx, dim3 grid, const FlatArgs &a, int mode,
                               int32_t *argmin) {
   if (mode == MODE_DENSE)
-    k_flat_valu<MODE_DENSE, OP, 4, 8><<<grid, 256, 0, ctx->stream>>>(a, argmin);
+    k_flat_valu<MODE_DENSE, OP, U, V><<<grid, 256, 0, ctx->stream>>>(a, argmin);
   else if (mode == MODE_FILTER)
-    k_flat_valu<MODE_FILTER, OP, 4, 8><<<grid, 256, 0, ctx->stream>>>(a, argmin);
+    k_flat_valu<MODE_FILTER, OP, U, V><<<grid, 256, 0, ctx->stream>>>(a, argmin);
   else if (mode == MODE_MATRIX)
-    k_flat_valu<MODE_MATRIX, OP, 4, 8><<<grid, 256, 0, ctx->stream>>>(a, argmin);
-  else
-    k_flat_valu<MODE_ARGMIN, OP, 4, 8><<<grid, 256, 0, ctx->stream>>>(a, argmin);
+    k_flat_valu<MODE_MATRIX, OP, U, V><<<grid, 256, 0, ctx->stream>>>(a, argmin);
+  else if constexpr (V == 8)
+    k_flat_valu<MODE_ARGMIN, OP, U, V><<<grid, 256, 0, ctx->stream>>>(a, argmin);
 }
 
 // metrics of the exact VALU scan
@@ -521,11 +521,13 @@ static bool metric_is_valu(int32_t metric) {
 
 template <int OP>
 static void launch_exact(vsk_ctx *ctx, dim3 grid, const FlatArgs &a, int mode,
-                         int32_t *argmin, bool stream) {
+                         int32_t *argmin, bool stream, bool small) {
   if (stream)
     launch_stream<OP>(ctx, a, mode);
+  else if (small)
+    launch_valu_tiles<OP, 2, 4>(ctx, grid, a, mode, argmin);
   else
-    launch_valu_tiles<OP>(ctx, grid, a, mode, argmin);
+    launch_valu_tiles<OP, 4, 8>(ctx, grid, a, mode, argmin);
 }
 
 // grid: query tiles x row splits, enough workgroups to fill 256 CUs (argmin
@@ -533,17 +535,34 @@ static void launch_exact(vsk_ctx *ctx, dim3 grid, const FlatArgs &a, int mode,
 void launch_flat(vsk_ctx *ctx, FlatArgs a, int mode, int32_t *argmin) {
   const int64_t rows = a.r1 - a.r0;
   if (rows <= 0 || a.nq <= 0) return;
-  const int64_t qt = ceil_div(a.nq, FB_Q);
-  int64_t splits = mode == MODE_ARGMIN ? 1 : ceil_div(4096, qt);
-  const int64_t max_splits = ceil_div(rows, FB_N);
-  if (splits > max_splits) splits = max_splits;
-  if (splits > 65535) splits = 65535;
-  if (splits < 1) splits = 1;
-  a.rows_per_split = ceil_div(ceil_div(rows, splits), FB_N) * FB_N;
-  splits = ceil_div(rows, a.rows_per_split);
+  const bool valu = metric_is_valu(a.metric);
+  int64_t tq = FB_Q, tn = FB_N, qt, splits;
+  auto split = [&] {
+    qt = ceil_div(a.nq, tq);
+    splits = mode == MODE_ARGMIN ? 1 : ceil_div(4096, qt);
+    const int64_t max_splits = ceil_div(rows, tn);
+    if (splits > max_splits) splits = max_splits;
+    if (splits > 65535) splits = 65535;
+    if (splits < 1) splits = 1;
+    a.rows_per_split = ceil_div(ceil_div(rows, splits), tn) * tn;
+    splits = ceil_div(rows, a.rows_per_split);
+  };
+  split();
+  // few 128 x 64 tiles and more than 64 queries: from some ten waves of the
+  // stream a CU on, short rows are faster in tiles of 64 x 32, which read a
+  // row half as often (us, tiles and stream: 2,048 x 32, 1,000 queries 15.9
+  // and 13.1, 4,000 queries 28.8 and 34.3; 10,000 x 128, 256 queries 33.6 and
+  // 35.3; of 512 columns, 1,800 queries x 4,096 rows, 281 and 269)
+  const bool few = valu && mode != MODE_ARGMIN && qt * splits < 4 * (int64_t)ctx->cu_count;
+  const bool small = few && a.nq > 64 && a.kdim <= 128 &&
+                     a.nq * rows >= 10000 * (int64_t)ctx->cu_count;
+  if (small) {
+    tq = 32;
+    tn = 64;
+    split();
+  }
   if (qt > 0x7FFFFFFF) fail(VSK_ERR_INVALID_BUFFER_SIZE, "too many queries");
   dim3 grid((unsigned)qt, (unsigned)splits);
-  const bool valu = metric_is_valu(a.metric);
   static const char *names[2][4] = {
       {"flat_mfma_dense", "flat_mfma_filter", "flat_mfma_matrix", "flat_mfma_argmin"},
       {"flat_valu_dense", "flat_valu_filter", "flat_valu_matrix", "flat_valu_argmin"}};
@@ -554,17 +573,16 @@ void launch_flat(vsk_ctx *ctx, FlatArgs a, int mode, int32_t *argmin) {
     // (at 64 queries the two take the same time over 100,000 x 768, 346 and
     // 355 us; at 128 the tiles need 501, the stream 529)
     // (a grid of at most 2^25 waves)
-    const bool stream = mode != MODE_ARGMIN &&
-                        (a.nq <= 64 || qt * splits < 4 * (int64_t)ctx->cu_count) &&
+    const bool stream = mode != MODE_ARGMIN && !small && (a.nq <= 64 || few) &&
                         ceil_div(rows, 64) * ceil_div(a.nq, 8) <= 1 << 25;
     switch (a.metric) {
-    case VSK_METRIC_L1: launch_exact<OP_L1>(ctx, grid, a, mode, argmin, stream); break;
-    case VSK_METRIC_HAMMING: launch_exact<OP_HAM>(ctx, grid, a, mode, argmin, stream); break;
-    case METRIC_L2_EXACT: launch_exact<OP_L2SEQ>(ctx, grid, a, mode, argmin, stream); break;
-    case METRIC_L2SQ_EXACT: launch_exact<OP_L2SQSEQ>(ctx, grid, a, mode, argmin, stream); break;
-    case METRIC_CN_EXACT: launch_exact<OP_CNSEQ>(ctx, grid, a, mode, argmin, stream); break;
-    case METRIC_DOT_EXACT: launch_exact<OP_DOTSEQ>(ctx, grid, a, mode, argmin, stream); break;
-    case METRIC_COS_EXACT: launch_exact<OP_COSSEQ>(ctx, grid, a, mode, argmin, stream); break;
+    case VSK_METRIC_L1: launch_exact<OP_L1>(ctx, grid, a, mode, argmin, stream, small); break;
+    case VSK_METRIC_HAMMING: launch_exact<OP_HAM>(ctx, grid, a, mode, argmin, stream, small); break;
+    case METRIC_L2_EXACT: launch_exact<OP_L2SEQ>(ctx, grid, a, mode, argmin, stream, small); break;
+    case METRIC_L2SQ_EXACT: launch_exact<OP_L2SQSEQ>(ctx, grid, a, mode, argmin, stream, small); break;
+    case METRIC_CN_EXACT: launch_exact<OP_CNSEQ>(ctx, grid, a, mode, argmin, stream, small); break;
+    case METRIC_DOT_EXACT: launch_exact<OP_DOTSEQ>(ctx, grid, a, mode, argmin, stream, small); break;
+    case METRIC_COS_EXACT: launch_exact<OP_COSSEQ>(ctx, grid, a, mode, argmin, stream, small); break;
     default: fail(VSK_ERR_INVALID_ARGUMENT, "no exact kernel for this metric");
     }
   } else {
