@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
-from vectorstorekit_amd import Context, VectorDatabase, VSKError
+from vectorstorekit_amd import Context, IVFConfiguration, IVFIndex, VectorDatabase, VSKError
 
 OUT_OF_MEMORY, EXECUTION_FAILED = -5, -6  # vsk_status (vsk_hip.h)
 
@@ -102,3 +102,70 @@ def test_profile_reset_after_failed_profiled_call(spec):
     assert stats and all(v[0] >= 1 for v in stats.values())
     db.free()
     ctx.close()
+
+
+def _after_every_fault(kinds, make, search, want):
+    """Fails event n = 1, 2, ... of a fresh context in turn until a run of
+    make and search meets none; whenever the search is what failed, the same
+    call on the same object must then return ``want``."""
+    tried = 0
+    for kind in kinds:
+        for n in range(1, 200):
+            print(f"fault {kind}:{n}", flush=True)
+            ctx = _armed(f"{kind}:{n}")
+            obj = None
+            try:
+                obj = make(ctx)
+                search(obj)
+                break
+            except VSKError as e:
+                assert "injected fault" in str(e)
+                if obj is not None:
+                    tried += 1
+                    gd, gi = search(obj)
+                    np.testing.assert_array_equal(gi, want[1])
+                    np.testing.assert_array_equal(gd, want[0])
+            finally:
+                if obj is not None:
+                    obj.free()
+                ctx.close()
+        else:
+            raise AssertionError("every event failed")
+    assert tried > 3
+
+
+def _close_rows(n, nq, d):
+    """Rows whose distances differ by less than a 16-bit plane's rounding,
+    and by more than fp32's: a screen that took its planes for exact would
+    return other rows."""
+    rng = np.random.default_rng(n + d)
+    return ((1 + 0.05 * rng.standard_normal((n, d))).astype(np.float32),
+            (1 + 0.05 * rng.standard_normal((nq, d))).astype(np.float32))
+
+
+@pytest.mark.parametrize("metric", ["euclideanSquared", "cosine", "cosineNormalized"])
+def test_fault_while_the_screen_plane_is_made(metric, monkeypatch):
+    """A search that fails while the database's 16-bit plane is made, or
+    before the plane's error bound is read back, leaves no plane behind that
+    the next search would trust: that one is bit for bit the oracle."""
+    monkeypatch.setenv("VSK_FLAT_KERNEL", "screen")
+    x, q = _close_rows(30_000, 40, 16)
+    if metric == "cosineNormalized":
+        x /= np.linalg.norm(x, axis=1, keepdims=True)
+        q /= np.linalg.norm(q, axis=1, keepdims=True)
+    code = {"euclideanSquared": O.L2SQ, "cosine": O.COSINE,
+            "cosineNormalized": O.COSINE_NORMALIZED}[metric]
+    _after_every_fault(("launch", "alloc", "sync"), lambda ctx: VectorDatabase(ctx, x),
+                       lambda db: db.search(q, 10, metric), O.search_flat(q, x, 10, code))
+
+
+def test_fault_while_the_probe_plane_is_made(monkeypatch):
+    """The same for the centroids' plane of the IVF probe's screen."""
+    monkeypatch.setenv("VSK_FLAT_KERNEL", "screen")
+    x, q = _close_rows(9000, 40, 16)
+    c = _close_rows(3000, 1, 16)[0]
+    lists = O.ivf_assign(x, c)
+    cfg = IVFConfiguration(dimensions=16, numberOfCentroids=len(c), numberOfProbes=5)
+    _after_every_fault(("launch", "alloc", "sync"), lambda ctx: IVFIndex.build(ctx, cfg, c, x),
+                       lambda idx: idx.search(q, 10),
+                       O.ivf_search(q, x, np.arange(len(x)), lists, c, 5, 10))

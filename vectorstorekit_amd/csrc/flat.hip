@@ -614,8 +614,10 @@ const float *x_aux(const vsk_db *db, int32_t metric) {
 
 void ensure_seq_norms(vsk_ctx *ctx, const vsk_db *db) {
   if (db->seqnorm.p) return;
-  db->seqnorm.reserve(sizeof(float) * (size_t)db->n);
-  seq_norms(ctx, db->x.as<float>(), db->n, db->d, db->ld, db->seqnorm.as<float>());
+  DevBuf norms;
+  norms.reserve(sizeof(float) * (size_t)db->n);
+  seq_norms(ctx, db->x.as<float>(), db->n, db->d, db->ld, norms.as<float>());
+  db->seqnorm.swap(norms);
 }
 
 float *q_aux(vsk_ctx *ctx, const float *dq, int64_t nq, int32_t d, int32_t ld,
@@ -642,26 +644,32 @@ SplitPtrs make_split(vsk_ctx *ctx, const vsk_db *db, const float *dq,
   // whole 64-dimension stages of the screen (zero padding)
   const int32_t ldb = (db->d + 63) & ~63;
   if (!db->split.p) {
-    // the hi plane (all the screen reads) and the maxima of its bound
-    db->split.reserve(sizeof(uint16_t) * (size_t)db->n * ldb);
-    db->ldb = ldb;
+    // the hi plane (all the IVF probe's screen reads) and the maxima of its
+    // bound (the database gets it when both are whole: a plane whose maxima
+    // were never read would pass for exact)
+    DevBuf hi;
+    hi.reserve(sizeof(uint16_t) * (size_t)db->n * ldb);
     uint32_t *mb =
         static_cast<uint32_t *>(ctx->scratch_ptr("flat.splitmax", 2 * sizeof(uint32_t)));
     fill_i32(ctx, reinterpret_cast<int32_t *>(mb), 2, 0);
-    split_bf16(ctx, db->x.as<float>(), db->n, db->d, db->ld, db->split.as<uint16_t>(), nullptr,
-               ldb, nullptr, nullptr, mb);
+    split_bf16(ctx, db->x.as<float>(), db->n, db->d, db->ld, hi.as<uint16_t>(), nullptr, ldb,
+               nullptr, nullptr, mb);
     uint32_t hb[2];
     VSK_HIP(hipMemcpyAsync(hb, mb, sizeof(hb), hipMemcpyDeviceToHost, ctx->stream));
     stream_sync(ctx);
     std::memcpy(&db->split_max_hi, &hb[0], sizeof(float));
     std::memcpy(&db->split_max_res, &hb[1], sizeof(float));
+    db->ldb = ldb;
+    db->split.swap(hi);
   }
   if (qlo && !db->split_lo.p) {
     // the lo plane only for the bf16x3 kernel (hi is written again, the
     // same values)
-    db->split_lo.reserve(sizeof(uint16_t) * (size_t)db->n * ldb);
+    DevBuf lo;
+    lo.reserve(sizeof(uint16_t) * (size_t)db->n * ldb);
     split_bf16(ctx, db->x.as<float>(), db->n, db->d, db->ld, db->split.as<uint16_t>(),
-               db->split_lo.as<uint16_t>(), ldb, nullptr, nullptr, nullptr);
+               lo.as<uint16_t>(), ldb, nullptr, nullptr, nullptr);
+    db->split_lo.swap(lo);
   }
   uint16_t *qs = static_cast<uint16_t *>(ctx->scratch_ptr(
       "flat.qsplit", sizeof(uint16_t) * (qlo ? 2 : 1) * (size_t)nq * ldb));
@@ -688,15 +696,17 @@ static SplitPtrs make_half(vsk_ctx *ctx, const vsk_db *db, const float *dq, int6
   auto &pl = db->plane[bf16 ? 1 : 0];
   if (!cosine && !pl.h.p) {
     pl.state.reserve(4 * sizeof(uint32_t));
-    pl.h.reserve(plane_bytes(db->n, ldb));
+    DevBuf h;  // (the database gets it with its maxima, as in make_split)
+    h.reserve(plane_bytes(db->n, ldb));
     uint32_t *st = pl.state.as<uint32_t>();
     half_rows(ctx, bf16 ? PLANE_BF16 : PLANE_HALF, db->x.as<float>(), db->sqnorm.as<float>(),
-              nullptr, db->n, db->d, db->ld, pl.h.as<uint16_t>(), ldb, nullptr, st);
+              nullptr, db->n, db->d, db->ld, h.as<uint16_t>(), ldb, nullptr, st);
     uint32_t hb[2];
     VSK_HIP(hipMemcpyAsync(hb, st, sizeof(hb), hipMemcpyDeviceToHost, ctx->stream));
     stream_sync(ctx);
     std::memcpy(&pl.max_hi, &hb[0], sizeof(float));
     std::memcpy(&pl.max_res, &hb[1], sizeof(float));
+    pl.h.swap(h);
   }
   uint16_t *qh = static_cast<uint16_t *>(
       ctx->scratch_ptr("flat.qhalf", sizeof(uint16_t) * (size_t)nq * ldb));

@@ -9,6 +9,7 @@
 #include <map>
 #include <memory>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "vsk_hip.h"
@@ -66,6 +67,10 @@ struct DevBuf {
   ~DevBuf();
   void reserve(size_t b);  // grow (contents not kept)
   void release();
+  void swap(DevBuf &o) {
+    std::swap(p, o.p);
+    std::swap(bytes, o.bytes);
+  }
   template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
