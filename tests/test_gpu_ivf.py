@@ -302,6 +302,44 @@ def test_ivf_ungrouped_scan_bit_exact(ctx, shape):
             assert np.isinf(gd[i, m:]).all()
 
 
+def test_ivf_search_by_several_contexts(ctx):
+    """Contexts of their own searching one index at the same time, right
+    after inserts (what a search keeps of the lists' sizes is made by the
+    first one, whichever context that is); bit for bit the oracle."""
+    import threading
+
+    from vectorstorekit_amd import Context
+    from vectorstorekit_amd._lib import METRIC_L2
+
+    x, q, c = _mixture(21, 700, 6000, 24, 8)
+    lists = O.ivf_assign(x, c)
+    idx = _index(ctx, c, None, nprobe=3)
+    others = [Context(0) for _ in range(4)]
+    out = [(np.empty((8, 5), np.float32), np.empty((8, 5), np.int64)) for _ in others]
+    status = [0] * len(others)
+
+    def search(t):
+        d, i = out[t]
+        status[t] = others[t].lib.vsk_ivf_search(others[t].handle, idx.handle, q.ctypes.data, 8, 3,
+                                                 5, METRIC_L2, d.ctypes.data, i.ctypes.data)
+
+    for m in range(1000, 6001, 1000):
+        print(f"ivf several contexts n={m}", flush=True)
+        idx.insert(x[m - 1000:m])
+        threads = [threading.Thread(target=search, args=(t,)) for t in range(len(others))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        od, oi = O.ivf_search(q, x[:m], np.arange(m), lists[:m], c, 3, 5)
+        for st, (gd, gi) in zip(status, out):
+            assert st == 0
+            np.testing.assert_array_equal(gi, oi)
+            np.testing.assert_array_equal(gd, od)
+    for o in others:
+        o.close()
+
+
 def test_ivf_squared_metric_bit_exact(ctx):
     x, q, c = _mixture(12, 48, 12_000, 64, 60)
     ids = np.arange(len(x), dtype=np.int64)

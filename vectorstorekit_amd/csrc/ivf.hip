@@ -30,6 +30,7 @@
 #include <cstring>
 #include <functional>
 #include <memory>
+#include <mutex>
 #include <numeric>
 
 #include "flat.hpp"
@@ -74,7 +75,9 @@ struct vsk_ivf {
   // list scan's per-query bound), valid with the plane
   mutable vsk::DevBuf xrad;
   // top_rows[i]: the rows of the i largest lists together (i <= nlist),
-  // valid while tversion == version
+  // valid while tversion == version; filled by the first search after a
+  // change, which may be several contexts' searches at once (top_mutex)
+  mutable std::mutex top_mutex;
   mutable std::vector<int64_t> top_rows;
   mutable int64_t tversion = -1;
 };
@@ -1377,6 +1380,7 @@ static bool list_screen_applies(vsk_ctx *ctx, const vsk_ivf *ivf, int32_t metric
 // candidates a query can have with np probes: the sizes of the np largest
 // lists summed (every row when every list is probed)
 static int64_t probe_bound(const vsk_ivf *ivf, int32_t np) {
+  std::lock_guard<std::mutex> lock(ivf->top_mutex);
   if (ivf->tversion != ivf->version) {
     // (sorted once per change of the rows: 10 us at 1,024 lists, which a
     // search of one query would notice)
