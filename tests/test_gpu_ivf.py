@@ -302,6 +302,18 @@ def test_ivf_ungrouped_scan_bit_exact(ctx, shape):
             assert np.isinf(gd[i, m:]).all()
 
 
+def test_ivf_columns_past_the_list_scan_are_refused(ctx):
+    """More columns than the list scan takes (16,384): refused whatever the
+    number of queries and probes."""
+    rng = np.random.default_rng(4)
+    c = rng.standard_normal((3, 16_388)).astype(np.float32)
+    idx = _index(ctx, c, np.repeat(c, 4, 0), nprobe=2)
+    for nq, nprobe in ((1, 1), (1, 3), (300, 2)):
+        with pytest.raises(VSKError) as e:
+            idx.search(np.repeat(c[:1], nq, 0), 2, nprobe=nprobe)
+        assert "dimension too large" in str(e.value)
+
+
 def test_ivf_search_by_several_contexts(ctx):
     """Contexts of their own searching one index at the same time, right
     after inserts (what a search keeps of the lists' sizes is made by the

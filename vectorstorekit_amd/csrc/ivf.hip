@@ -2202,6 +2202,19 @@ static vsk_status ivf_search_any(vsk_ctx *ctx, const vsk_ivf *ivf, const float *
   const int32_t np = nprobe < ivf->nlist ? nprobe : ivf->nlist;  // .exact
   VSK_REQUIRE(np <= VSK_MAX_K || np == ivf->nlist, VSK_ERR_INVALID_ARGUMENT,
               "nprobe must be <= VSK_MAX_K or cover every list");
+  // queries per group: their rows, codes or tables fit 64 KiB of LDS
+  const int64_t per_q = kind == 0 ? (int64_t)ivf->ld * 4
+                        : kind == 1 ? (int64_t)ivf->cstride
+                                    : (int64_t)ivf->cM * ivf->cksub * 4;
+  const int QG = per_q * 16 <= 64 * 1024 ? 16
+                 : per_q * 8 <= 64 * 1024 ? 8
+                 : per_q * 4 <= 64 * 1024 ? 4
+                                           : 1;
+  // (asked before any scan is chosen: whether an index can be searched does
+  // not depend on how many queries there are)
+  VSK_REQUIRE(per_q * QG <= 64 * 1024, VSK_ERR_UNSUPPORTED,
+              kind == 2 ? "PQ tables too large for the IVF list scan (M x ksub > 16384)"
+                        : "dimension too large for the IVF list scan");
   float *dlut = nullptr;
   if (kind == 2) {
     // the tables first: that call syncs the stream itself
@@ -2279,17 +2292,6 @@ static vsk_status ivf_search_any(vsk_ctx *ctx, const vsk_ivf *ivf, const float *
   int64_t *cnt =
       static_cast<int64_t *>(ctx->scratch_ptr("ivf.cnt", sizeof(int64_t) * nq));
 
-  // queries per group: their rows, codes or tables fit 64 KiB of LDS
-  const int64_t per_q = kind == 0 ? (int64_t)ld * 4
-                        : kind == 1 ? (int64_t)ivf->cstride
-                                    : (int64_t)ivf->cM * ivf->cksub * 4;
-  const int QG = per_q * 16 <= 64 * 1024 ? 16
-                 : per_q * 8 <= 64 * 1024 ? 8
-                 : per_q * 4 <= 64 * 1024 ? 4
-                                           : 1;
-  VSK_REQUIRE(per_q * QG <= 64 * 1024, VSK_ERR_UNSUPPORTED,
-              kind == 2 ? "PQ tables too large for the IVF list scan (M x ksub > 16384)"
-                        : "dimension too large for the IVF list scan");
   // candidates per query: at most the np largest lists; query batches
   // whose bound fits 2^27 keys (one query at least).  Everything below runs
   // on the stream without a read-back: segment offsets, pairs and groups
