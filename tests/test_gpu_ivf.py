@@ -302,6 +302,46 @@ def test_ivf_ungrouped_scan_bit_exact(ctx, shape):
             assert np.isinf(gd[i, m:]).all()
 
 
+def _grouped(ctx, idx, q, k, **kw):
+    """A search, and whether it grouped its queries by list."""
+    ctx.profile(True)
+    ctx.profile_reset()
+    d, i = idx.search(q, k, **kw)
+    stats = ctx.profile_stats()
+    ctx.profile(False)
+    return d, i, "ivf_probe_bases" in stats
+
+
+@pytest.mark.parametrize("case", [
+    # nlist, rows of the longest list, of the others, columns, queries, probes, grouped
+    (64, 20_000, 20, 16, 1, 1, True), (64, 20_000, 20, 16, 1, 2, True),
+    (64, 20_000, 20, 16, 30, 10, True), (64, 300, 200, 16, 30, 10, False),
+    # 2^21 words: 8 probes of pitch 448
+    (16, 448, 390, 16, 585, 8, False), (16, 448, 390, 16, 586, 8, True),
+    # 2^27 terms, or 2^29 with two or three queries a list
+    (16, 1000, 1000, 256, 65, 8, False), (16, 1000, 1000, 256, 66, 8, True),
+    (256, 448, 448, 130, 193, 4, False), (256, 1400, 1400, 256, 193, 4, True),
+])
+def test_ivf_ungrouped_scan_rule(ctx, case):
+    """Which searches scan their lists ungrouped: few words and terms, and no
+    index whose words (laid out by its longest list) are many times what its
+    queries probe; the results are the oracle's either way."""
+    nlist, longest, others, d, nq, nprobe, grouped = case
+    print(f"ivf ungrouped rule {case}", flush=True)
+    rng = np.random.default_rng(nlist + longest)
+    c = (4.0 * rng.standard_normal((nlist, d))).astype(np.float32)
+    lists = np.repeat(np.arange(nlist), [longest] + [others] * (nlist - 1))
+    x = (c[lists] + 0.1 * rng.standard_normal((len(lists), d))).astype(np.float32)
+    q = (c[rng.integers(0, nlist, nq)] + 0.1 * rng.standard_normal((nq, d))).astype(np.float32)
+    idx = _index(ctx, c, x, nprobe=nprobe)
+    np.testing.assert_array_equal(idx.list_sizes(), np.bincount(lists))
+    gd, gi, was = _grouped(ctx, idx, q, 10)
+    assert was == grouped
+    od, oi = O.ivf_search(q, x, np.arange(len(x)), lists.astype(np.int32), c, nprobe, 10)
+    np.testing.assert_array_equal(gi, oi)
+    np.testing.assert_array_equal(gd, od)
+
+
 def test_ivf_columns_past_the_list_scan_are_refused(ctx):
     """More columns than the list scan takes (16,384): refused whatever the
     number of queries and probes."""

@@ -2094,25 +2094,33 @@ static void probe_screen(vsk_ctx *ctx, const vsk_ivf *ivf, const float *dq, int6
 
 }  // namespace vsk
 
-// kind 0: the rows (metric L2 / L2SQ); 1: SQ8 codes, qextra = nq x d int8
-// query codes; 2: PQ codes, qextra = the vsk_pq whose tables score them
-// allow (may be null): the row filter, a bitmap over the stored rows' ids
-// of allow_bits bits (k_allow_list_bits)
 // Whether a search scans its lists without grouping queries by list.  The
 // ungrouped scan reads a list once per query that probes it (from the L2
 // after the first) but needs no grouping launches, and its waves are many and
-// short.  Measured (us, ungrouped and grouped): 200,000 x 128 in 1,024 lists,
-// 10 probes: 1 query 45 and 83, 256 queries (6e7 terms) 76 and 110, 1,000
-// (2.5e8) 156 and 146; 1M x 128, 4,096 lists, 32 probes: 256 queries (2 a
-// list, 2.6e8) 234 and 282, 1,000 (8 a list) 679 and 412; 200,000 x 768, 512
-// lists, 16 probes: 64 queries (2 a list, 3e8) 231 and 381, 256 (8 a list)
-// 717 and 492.  So: up to 2^27 terms, or 2^29 with at most four queries a
-// list.  Words are laid out by the longest list, so skewed lists (twice the
-// words) are grouped too.
+// short.  Measured (us a call, ungrouped and grouped):
+//  * 200,000 x 128 in 1,024 lists: 10 probes, 1 query 45 and 95, 256 queries
+//    77 and 123; 16 probes, 256 queries (4 a list, 2^26.6 terms) 91 and 133.
+//    100,000 x 16 in 256 lists, 8 probes, 512 queries 77 and 90, 1,024
+//    (2^21.8 words) 111 and 98, 2,048 187 and 119: so up to 2^27 terms in
+//    2^21 words.
+//  * 1M x 128 in 4,096 lists, 16 probes: 512 queries (2 a list) 215 and 293,
+//    768 (3 a list) 299 and 324, 1,024 (4) 379 and 350; 1M x 64 in 1,024, 8
+//    probes: 256 (2) 132 and 152, 384 (3) 168 and 165, 512 (4) 201 and 174:
+//    so beyond that up to 2^29 terms where two (of 128 columns and more,
+//    three) queries share a list.
+//  * Words are laid out by the longest list: every query writes and selects
+//    from np * pitch of them, however short the lists it probes.  One list of
+//    500,000 rows among 4,095 of 122, one probe, one query: 1,166 and 95;
+//    lists of 7,900 / sqrt(i) rows, 2 probes 78 and 100, 10
+//    probes 220 and 119: so at most 2^14 words more than twice what a query's
+//    probes hold on average.
 static bool direct_applies(const vsk_ivf *ivf, int64_t nq, int32_t np, int64_t pitch) {
-  const double terms = (double)nq * np * ((double)ivf->total / ivf->nlist) * ivf->ld;
-  if (pitch <= 0 || np * pitch > 2 * probe_bound(ivf, np) + 4096) return false;
-  return terms <= 0x1p27 || (terms <= 0x1p29 && nq * np <= 4 * (int64_t)ivf->nlist);
+  const double rows = np * ((double)ivf->total / ivf->nlist);  // a query's, on average
+  const double words = (double)nq * np * pitch, terms = nq * rows * ivf->ld;
+  if (pitch <= 0 || np * pitch > 2 * rows + 16384) return false;
+  const int64_t share = ivf->ld >= 128 ? 3 : 2;
+  return (words <= 0x1p21 && terms <= 0x1p27) ||
+         (terms <= 0x1p29 && nq * np <= share * (int64_t)ivf->nlist);
 }
 
 // the ungrouped list scan of all queries, and one selection that writes the
@@ -2160,6 +2168,10 @@ static void direct_search(vsk_ctx *ctx, const vsk_ivf *ivf, const float *dq, int
   }
 }
 
+// kind 0: the rows (metric L2 / L2SQ); 1: SQ8 codes, qextra = nq x d int8
+// query codes; 2: PQ codes, qextra = the vsk_pq whose tables score them
+// allow (may be null): the row filter, a bitmap over the stored rows' ids
+// of allow_bits bits (k_allow_list_bits)
 static vsk_status ivf_search_any(vsk_ctx *ctx, const vsk_ivf *ivf, const float *q,
                                  const void *qextra, int64_t nq, int32_t nprobe, int32_t k,
                                  int32_t metric, int32_t kind, void *out_dist,
