@@ -69,6 +69,28 @@ def test_kmeans_plusplus_rows_out_of_scale(ctx, shape):
                                      seed=k))
 
 
+@pytest.mark.parametrize("shape", [(1_310_720, 9, 12), (1_310_721, 9, 24), (350_100, 768, 8),
+                                   (524_289, 5, 9)])
+def test_kmeans_plusplus_large(ctx, shape):
+    """Seeding past the sizes where the triangle test comes first (1,310,720
+    rows, 256 MB of codes), rows ending inside a group of 64 and a block of
+    weight sums, few clusters and more (rows that a pick covers, and rows
+    that none does); copies of one row, a row far away."""
+    n, d, k = shape
+    print(f"kmeans++ large n={n} d={d} k={k}", flush=True)
+    rng = np.random.default_rng(n + d)
+    cent = 4 * rng.standard_normal((max(3, k // 3), d), dtype=np.float32)
+    x = cent[rng.integers(0, len(cent), n)]
+    for a in range(0, n, 100_000):
+        x[a:a + 100_000] += 0.5 * rng.standard_normal(x[a:a + 100_000].shape, dtype=np.float32)
+    x[5:n:1000] = x[5]
+    x[n - 1] = 500
+    cfg = KMeansClusteringConfiguration(maxIterations=0, initMethod="kMeansPlusPlus", seed=k)
+    res = KMeansClustering(ctx, cfg).cluster(x, k)
+    ref = O.kmeans_cluster(x, k, init_method="kMeansPlusPlus", max_iter=0, tol=1e-4, seed=k)
+    np.testing.assert_array_equal(np.asarray(res.centroids), ref[0])
+
+
 def test_kmeans_custom_weights_empty_clusters(ctx):
     """Custom start with centroids far from the data (empty clusters refilled
     from the seeded stream), weights, and a run to convergence."""

@@ -325,6 +325,16 @@ constexpr int KP_T = 256;       // threads of a block, rows of an update block
 constexpr int KP_B = 4 * KP_T;  // rows of a weight-sum block
 constexpr int KP_SLOTS = 64;    // max slots per pick (a power of two, one wave's lanes)
 constexpr int KP_TILE = 33 * KP_T;  // floats of the update's row tile
+// From these bytes of codes or rows on, the triangle test first
+// (k_kpp_update_queued).  us a pick, without and with it: 1M x 768 (732 MB of
+// codes), 4,096 picks of 256 clusters 182 and 79, 512 of 512 194 and 192; 4M x
+// 128, 2,048 of 128 137 and 75; 1.5M x 32, 512 of 64 55 and 49, 512 of 512 54
+// and 55; 350,000 x 768 (257 MB), 1,024 of 64 81 and 69, 1,024 of 1,024 77 and
+// 83; but 1M x 128, 4,096 of 4,096 46 and 58; 100,000 x 128 16 and 23.
+constexpr size_t KP_NEAR = (size_t)256 << 20;
+constexpr int64_t KP_NEAR_ROWS = 5 << 18;
+// rows of 64 that make the int8 screen of k_kpp_update_queued worth its wait
+constexpr int KP_FEW = 16;
 
 // The rows as int8 for the update's screen: x_i = s_i q_i + residual, s_i =
 // max |x_ij| / 127, q_ij the nearest integer; par[i] = (s_i, |s_i q_i|^2, a
@@ -385,6 +395,52 @@ __global__ __launch_bounds__(KP_T) void k_kpp_codes(const float *x, int64_t ld, 
   }
 }
 
+// cc[a] = |x_c - x_{chosen[a]}| for the picks a < r, c = chosen[r]: one
+// wave per a, lanes over the coordinates.  Only the triangle test of
+// k_kpp_update reads it, so any summation order with a small relative error
+// serves (this one's is under (d / 64 + 11) 2^-25).
+__global__ __launch_bounds__(256) void k_kpp_cc(const float *x, int64_t ld, int32_t d,
+                                                const int64_t *chosen, int r, float *cc) {
+#pragma clang fp contract(off)
+  const int64_t c = chosen[r];
+  if (c < 0) return;
+  const int a = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (a >= r) return;  // wave-uniform
+  const float *xc = x + c * ld, *xa = x + chosen[a] * ld;
+  float s = 0.f;
+  for (int32_t j = lane; j < d; j += 64) {
+    const float t = xc[j] - xa[j];
+    s = s + t * t;
+  }
+#pragma unroll
+  for (int m = 32; m > 0; m >>= 1) s = s + __shfl_xor(s, m);
+  if (lane == 0) cc[a] = sqrtf(s);
+}
+
+// Whether row i (distance dm to its nearest pick) may come nearer to row c:
+// the int8 screen of k_kpp_update's comment
+__device__ inline bool kpp_may_move(const uint4 *__restrict__ codes,
+                                    const float4 *__restrict__ par, int64_t i, int64_t c,
+                                    int32_t nch, float dm, float skipm) {
+#pragma clang fp contract(off)
+  const float4 pi = par[i], pc = par[c];
+  const uint4 *qi = codes + (i >> 6) * nch * 64 + (i & 63);
+  const uint4 *qc = codes + (c >> 6) * nch * 64 + (c & 63);
+  int32_t dot = 0;
+#pragma unroll 8
+  for (int ch = 0; ch < nch; ++ch) {
+    const uint4 a = qi[64 * ch], o = qc[64 * ch];
+    dot = __builtin_amdgcn_sdot4((int)a.x, (int)o.x, dot, false);
+    dot = __builtin_amdgcn_sdot4((int)a.y, (int)o.y, dot, false);
+    dot = __builtin_amdgcn_sdot4((int)a.z, (int)o.z, dot, false);
+    dot = __builtin_amdgcn_sdot4((int)a.w, (int)o.w, dot, false);
+  }
+  const float t = pi.y + pc.y;
+  const float sq = (t - 2.0f * (pi.x * pc.x) * (float)dot) - 0x1p-20f * t;
+  const float lb = (sqrtf(fmaxf(sq, 0.f)) - (pi.z + pc.z)) * (1.f - 0x1p-20f);
+  return !(dm >= 0x1p-40f && dm <= 0x1p60f && t <= 0x1p100f && lb >= dm * skipm);
+}
+
 // D[i] = min(D[i], |x_i - x_c|) with c = chosen[r] (sequential sqrt-L2, as
 // computeMinDistances, :401-419); the max over rows of D^2 lands in
 // maxbits[(r + 1) * KP_SLOTS + s] for the KP_SLOTS slots s (non-negative
@@ -435,25 +491,7 @@ __global__ __launch_bounds__(KP_T) void k_kpp_update(const float *__restrict__ x
   if (c < 0) return;  // an earlier pick found degenerate data
   const float *__restrict__ xc = x + c * ld;
   uint32_t b = 0;  // max D^2 bits seen by this thread
-  bool need = live;
-  if (live && codes) {
-    const float4 pi = par[row0 + tid], pc = par[c];
-    const uint4 *qi = codes + ((row0 >> 6) + w) * nch * 64 + lane;
-    const uint4 *qc = codes + (c >> 6) * nch * 64 + (c & 63);
-    int32_t dot = 0;
-#pragma unroll 8
-    for (int ch = 0; ch < nch; ++ch) {
-      const uint4 a = qi[64 * ch], o = qc[64 * ch];
-      dot = __builtin_amdgcn_sdot4((int)a.x, (int)o.x, dot, false);
-      dot = __builtin_amdgcn_sdot4((int)a.y, (int)o.y, dot, false);
-      dot = __builtin_amdgcn_sdot4((int)a.z, (int)o.z, dot, false);
-      dot = __builtin_amdgcn_sdot4((int)a.w, (int)o.w, dot, false);
-    }
-    const float t = pi.y + pc.y;
-    const float sq = (t - 2.0f * (pi.x * pc.x) * (float)dot) - 0x1p-20f * t;
-    const float lb = (sqrtf(fmaxf(sq, 0.f)) - (pi.z + pc.z)) * (1.f - 0x1p-20f);
-    need = !(dm >= 0x1p-40f && dm <= 0x1p60f && t <= 0x1p100f && lb >= dm * skipm);
-  }
+  const bool need = live && kpp_may_move(codes, par, row0 + tid, c, nch, dm, skipm);
   if (live && !need) b = __float_as_uint(dm * dm);
   const uint64_t mask = __ballot(need);
   if (lane == 0) s_cnt[w] = __popcll(mask);
@@ -531,6 +569,133 @@ __global__ __launch_bounds__(KP_T) void k_kpp_update(const float *__restrict__ x
     for (int j = 0; j < KP_T / 64; ++j) b = s_max[j] > b ? s_max[j] : b;
     atomicMax(&maxbits[(r + 1) * KP_SLOTS + blockIdx.x % KP_SLOTS], b);
   }
+}
+
+// The same for codes that do not stay in the caches, which would be read
+// from HBM on every pick long after most rows are covered: the triangle test
+// comes first.  near[i] is the pick a that set D[i], and a row with
+// |x_c - x_a| >= 2 D skipm is left alone, its code unread.  The exact distance
+// is at least |x_c - x_a| - |x_i - x_a|, and (d + 4) 2^-22 exceeds the
+// relative errors of the three computed distances taken together (a
+// sequential one: under (d + 4) 2^-25; k_kpp_cc's: under (d / 64 + 11) 2^-25,
+// counted twice), so the computed distance would not be below D (for 2^-60 <=
+// D <= 2^60, where no sum under- or overflows enough to break the relative
+// bounds).  Without codes (null) the triangle test stands alone.
+//
+// One wave a block strides over groups of 64 rows: few rows of a group need
+// anything, so those that need the distance queue in LDS across the groups.
+// 64 of them, or what is left at the end, are staged in column chunks as wide
+// as the tile allows (32 columns for 64 rows, 512 for up to 4), the next
+// chunk's loads in flight, and every lane sums its own row in order.
+__global__ __launch_bounds__(64) void k_kpp_update_queued(
+    const float *__restrict__ x, int64_t ld, int32_t d, int64_t n,
+    const int64_t *__restrict__ chosen, int r, const uint4 *__restrict__ codes,
+    const float4 *__restrict__ par, int32_t nch, float skipm, const float *__restrict__ cc,
+    int32_t *__restrict__ near, float *__restrict__ D, uint32_t *__restrict__ maxbits) {
+#pragma clang fp contract(off)
+  constexpr int E = 2048;  // floats of a chunk
+  __shared__ float tile[E + 64];
+  __shared__ int64_t l_row[128];
+  __shared__ float l_dm[128];
+  const int64_t c = chosen[r];
+  if (c < 0) return;  // an earlier pick found degenerate data
+  const int lane = threadIdx.x;
+  const float *__restrict__ xc = x + c * ld;
+  uint32_t b = 0;  // max D^2 bits seen by this lane
+  // the distances of the first m <= 64 queued rows
+  auto run = [&](int m) {
+    const int sh = m <= 4 ? 9 : m <= 8 ? 8 : m <= 16 ? 7 : m <= 32 ? 6 : 5;
+    const int cw = 1 << sh, stride = cw + 1;
+    float v[E / 64];
+    auto load = [&](int32_t j0) {
+#pragma unroll
+      for (int u = 0; u < E / 64; ++u) {
+        const int e = u * 64 + lane, rr = e >> sh, col = j0 + (e & (cw - 1));
+        v[u] = rr < m && col < d ? x[l_row[rr] * ld + col] : 0.f;
+      }
+    };
+    load(0);
+    float s = 0.f;
+    for (int32_t j0 = 0; j0 < d; j0 += cw) {
+      if (j0 > 0) __syncthreads();  // the previous chunk has been read
+#pragma unroll
+      for (int u = 0; u < E / 64; ++u) {
+        const int e = u * 64 + lane;
+        tile[(e >> sh) * stride + (e & (cw - 1))] = v[u];
+      }
+      __syncthreads();
+      if (j0 + cw < d) load(j0 + cw);
+      if (lane < m) {
+        const int jn = d - j0 < cw ? d - j0 : cw;
+        const float *t = tile + lane * stride;
+#pragma unroll 8
+        for (int j = 0; j < jn; ++j) {
+          const float e = t[j] - xc[j0 + j];
+          s = s + e * e;
+        }
+      }
+    }
+    if (lane < m) {
+      float dm = l_dm[lane];
+      const float dist = sqrtf(s);
+      if (dist < dm) {
+        dm = dist;
+        const int64_t i = l_row[lane];
+        D[i] = dm;
+        near[i] = r;
+      }
+      const uint32_t bw = __float_as_uint(dm * dm);
+      b = bw > b ? bw : b;
+    }
+  };
+  int cnt = 0;  // queued rows (wave-uniform)
+  for (int64_t row0 = (int64_t)blockIdx.x * 64; row0 < n; row0 += (int64_t)gridDim.x * 64) {
+    const int64_t i = row0 + lane;
+    bool need = false;
+    float dm = 0.f;
+    if (i < n) {
+      dm = D[i];
+      const int32_t a = near[i];
+      need = !(a >= 0 && dm >= 0x1p-60f && dm <= 0x1p60f && cc[a] >= 2.0f * dm * skipm);
+    }
+    // (a wait for a few rows' codes costs more than their distances: 10M x 32,
+    // 512 picks of 64 clusters, late ones 133 us with it and 70 without)
+    if (codes && __popcll(__ballot(need)) >= KP_FEW && need)
+      need = kpp_may_move(codes, par, i, c, nch, dm, skipm);
+    if (i < n && !need) {
+      const uint32_t bw = __float_as_uint(dm * dm);
+      b = bw > b ? bw : b;
+    }
+    const uint64_t mask = __ballot(need);
+    if (need) {
+      const int pos = cnt + (int)__builtin_amdgcn_mbcnt_hi(
+                                (uint32_t)(mask >> 32),
+                                __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+      l_row[pos] = i;
+      l_dm[pos] = dm;
+    }
+    cnt += __popcll(mask);
+    if (cnt >= 64) {
+      __syncthreads();
+      run(64);
+      __syncthreads();
+      if (lane < cnt - 64) {
+        l_row[lane] = l_row[64 + lane];
+        l_dm[lane] = l_dm[64 + lane];
+      }
+      cnt -= 64;
+    }
+  }
+  if (cnt > 0) {
+    __syncthreads();
+    run(cnt);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint32_t v = __shfl_xor(b, o);
+    b = v > b ? v : b;
+  }
+  if (lane == 0) atomicMax(&maxbits[(r + 1) * KP_SLOTS + blockIdx.x % KP_SLOTS], b);
 }
 
 // the max of pick r + 1's KP_SLOTS slots, through LDS to the whole block
@@ -817,17 +982,31 @@ static bool init_plusplus(vsk_ctx *ctx, const float *dx, int64_t n, int32_t d,
   const int32_t nch = (int32_t)ceil_div(d, 16);
   uint4 *codes = nullptr;
   float4 *par = nullptr;
+  const size_t code_bytes = sizeof(uint4) * (size_t)ceil_div(n, 64) * 64 * nch;
   if (d <= 1 << 17) {
-    codes = static_cast<uint4 *>(ctx->scratch_ptr(
-        "km.kppcodes", sizeof(uint4) * (size_t)ceil_div(n, 64) * 64 * nch));
+    codes = static_cast<uint4 *>(ctx->scratch_ptr("km.kppcodes", code_bytes));
     par = static_cast<float4 *>(ctx->scratch_ptr("km.kpppar", sizeof(float4) * (size_t)n));
     k_kpp_codes<<<(unsigned)std::min<int64_t>(ceil_div(n, KP_T / 64), 16384), KP_T, 0,
                   ctx->stream>>>(
         dx, ld, d, n, nch, reinterpret_cast<uint32_t *>(codes), par);
   }
+  float *cc = nullptr;
+  int32_t *near = nullptr;
+  if (!codes || code_bytes > KP_NEAR || n > KP_NEAR_ROWS) {
+    cc = static_cast<float *>(ctx->scratch_ptr("km.kppcc", sizeof(float) * (size_t)k));
+    near = static_cast<int32_t *>(ctx->scratch_ptr("km.kppnear", sizeof(int32_t) * (size_t)n));
+    fill_i32(ctx, near, n, -1);
+  }
   for (int r = 0; r + 1 < k; ++r) {
-    k_kpp_update<<<(unsigned)ceil_div(n, KP_T), KP_T, 0, ctx->stream>>>(
-        dx, ld, d, n, chosen, r, codes, par, nch, skipm, D, maxbits);
+    if (near && r > 0)
+      k_kpp_cc<<<(unsigned)ceil_div(r, 4), 256, 0, ctx->stream>>>(dx, ld, d, chosen, r, cc);
+    if (near)
+      k_kpp_update_queued<<<(unsigned)std::min<int64_t>(ceil_div(n, 64), 16 * ctx->cu_count), 64,
+                            0, ctx->stream>>>(dx, ld, d, n, chosen, r, codes, par, nch, skipm,
+                                              cc, near, D, maxbits);
+    else
+      k_kpp_update<<<(unsigned)ceil_div(n, KP_T), KP_T, 0, ctx->stream>>>(
+          dx, ld, d, n, chosen, r, codes, par, nch, skipm, D, maxbits);
     k_kpp_pick<<<(unsigned)nb, KP_T, 0, ctx->stream>>>(bsum, nb, D, n, maxbits, rng, r,
                                                        chosen, done);
   }
