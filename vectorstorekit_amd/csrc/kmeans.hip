@@ -322,7 +322,8 @@ __global__ void k_gather_rows_i64(const float *src, int64_t ld, const int64_t *r
 // k-means++ on the device
 // ---------------------------------------------------------------------------
 constexpr int KP_T = 256;       // threads of a block, rows of an update block
-constexpr int KP_B = 4 * KP_T;  // rows of a weight-sum block
+constexpr int KP_B = 4 * KP_T;  // rows of a weight-sum chunk
+constexpr int KP_BLOCKS = 512;  // weight-sum blocks at most
 constexpr int KP_SLOTS = 64;    // max slots per pick (a power of two, one wave's lanes)
 constexpr int KP_TILE = 33 * KP_T;  // floats of the update's row tile
 // From these bytes of codes or rows on, the triangle test first
@@ -753,15 +754,18 @@ __device__ uint64_t block_excl_u64(uint64_t v, uint64_t *wsum, uint64_t *total) 
 // fixed-weight prefix exceeds u.  total = 0 (every row on a chosen centroid)
 // is the reference's degenerateData (:235-237): chosen[r + 1] = -1.
 //
-// Every block sums the fixed weights of its 1024 rows; the block that counts
-// itself last in *done has them all and picks: one launch of 7.2 us at
-// 100,000 rows instead of a sum and a pick launch of 4.4 and 6.6 us.  No
+// Every block sums the fixed weights of its m chunks of 1024 rows; the block
+// that counts itself last in *done has them all and picks: one launch of 7.2
+// us at 100,000 rows instead of a sum and a pick launch of 4.4 and 6.6 us.  m
+// keeps the blocks to KP_BLOCKS, since their counts queue on one address: 4M
+// rows with m = 1 took 55 us, now 20 (39 as two launches).  No
 // fence is needed, and none is used (an agent-scope release writes back the
 // XCD's whole L2): a block's sum goes out by a returning exchange at agent
 // scope, its arrival is counted only after that returned, and the last block
 // reads the sums by agent-scope loads.  No block waits for another.
-__global__ __launch_bounds__(KP_T) void k_kpp_pick(uint64_t *bsum, int64_t nb, const float *D,
-                                                   int64_t n, const uint32_t *maxbits,
+__global__ __launch_bounds__(KP_T) void k_kpp_pick(uint64_t *bsum, int64_t nb, int32_t m,
+                                                   const float *D, int64_t n,
+                                                   const uint32_t *maxbits,
                                                    uint64_t *rng, int r, int64_t *chosen,
                                                    uint32_t *done) {
   __shared__ uint64_t wsum[KP_T / 64];
@@ -770,13 +774,16 @@ __global__ __launch_bounds__(KP_T) void k_kpp_pick(uint64_t *bsum, int64_t nb, c
   __shared__ uint32_t s_mx;
   __shared__ bool s_last;
   const int t = threadIdx.x;
-  const int64_t i0 = (int64_t)blockIdx.x * KP_B;
+  const int64_t i0 = (int64_t)blockIdx.x * m * KP_B;
   float dv[KP_B / KP_T];
+  auto load = [&](int64_t c0) {
 #pragma unroll
-  for (int u = 0; u < KP_B / KP_T; ++u) {
-    const int64_t i = i0 + u * KP_T + t;
-    dv[u] = i < n ? D[i] : 0.f;  // (a zero distance weighs 0)
-  }
+    for (int u = 0; u < KP_B / KP_T; ++u) {
+      const int64_t i = c0 + u * KP_T + t;
+      dv[u] = i < n ? D[i] : 0.f;  // (a zero distance weighs 0)
+    }
+  };
+  load(i0);
   uint64_t st = *rng;  // (only the last block writes it, after its count)
   if (chosen[r] < 0) {
     if (blockIdx.x == 0 && t == 0) chosen[r + 1] = -1;
@@ -784,8 +791,14 @@ __global__ __launch_bounds__(KP_T) void k_kpp_pick(uint64_t *bsum, int64_t nb, c
   }
   const float maxw = kpp_maxw(maxbits, r, &s_mx);
   uint64_t f = 0;
+  for (int32_t j = 0; j < m; ++j) {
+    float cur[KP_B / KP_T];
 #pragma unroll
-  for (int u = 0; u < KP_B / KP_T; ++u) f += kpp_fixed(dv[u], maxw);
+    for (int u = 0; u < KP_B / KP_T; ++u) cur[u] = dv[u];
+    if (j + 1 < m) load(i0 + (j + 1) * KP_B);
+#pragma unroll
+    for (int u = 0; u < KP_B / KP_T; ++u) f += kpp_fixed(cur[u], maxw);
+  }
   uint64_t sum;
   (void)block_excl_u64(f, wsum, &sum);
   if (t == 0) {
@@ -839,19 +852,24 @@ __global__ __launch_bounds__(KP_T) void k_kpp_pick(uint64_t *bsum, int64_t nb, c
     return;
   }
   // consecutive rows per thread, so that thread order is row order
-  const int64_t i1 = blk * KP_B + (int64_t)t * (KP_B / KP_T);
-  uint64_t fx[KP_B / KP_T], mine = 0;
+  uint64_t chunk = s_base;
+  for (int32_t j = 0; j < m; ++j) {
+    const int64_t i1 = (blk * m + j) * KP_B + (int64_t)t * (KP_B / KP_T);
+    uint64_t fx[KP_B / KP_T], mine = 0;
 #pragma unroll
-  for (int j = 0; j < KP_B / KP_T; ++j) {
-    fx[j] = i1 + j < n ? kpp_fixed(D[i1 + j], maxw) : 0;
-    mine += fx[j];
-  }
-  uint64_t tot2;
-  uint64_t ex = s_base + block_excl_u64(mine, wsum, &tot2);
+    for (int v = 0; v < KP_B / KP_T; ++v) {
+      fx[v] = i1 + v < n ? kpp_fixed(D[i1 + v], maxw) : 0;
+      mine += fx[v];
+    }
+    uint64_t tot2;
+    uint64_t ex = chunk + block_excl_u64(mine, wsum, &tot2);
 #pragma unroll
-  for (int j = 0; j < KP_B / KP_T; ++j) {
-    if (fx[j] > 0 && ex <= u && u < ex + fx[j]) s_row = i1 + j;
-    ex += fx[j];
+    for (int v = 0; v < KP_B / KP_T; ++v) {
+      if (fx[v] > 0 && ex <= u && u < ex + fx[v]) s_row = i1 + v;
+      ex += fx[v];
+    }
+    chunk += tot2;
+    if (u < chunk) break;  // (every thread's)
   }
   __syncthreads();
   if (t == 0) chosen[r + 1] = s_row;
@@ -963,7 +981,8 @@ static bool init_plusplus(vsk_ctx *ctx, const float *dx, int64_t n, int32_t d,
   uint32_t *maxbits = static_cast<uint32_t *>(
       ctx->scratch_ptr("km.kppmax", sizeof(uint32_t) * (size_t)(k + 1) * KP_SLOTS));
   fill_i32(ctx, reinterpret_cast<int32_t *>(maxbits), (int64_t)(k + 1) * KP_SLOTS, 0);
-  const int64_t nb = ceil_div(n, KP_B);
+  const int32_t m = (int32_t)ceil_div(n, (int64_t)KP_BLOCKS * KP_B);
+  const int64_t nb = ceil_div(n, (int64_t)m * KP_B);
   uint64_t *bsum = static_cast<uint64_t *>(
       ctx->scratch_ptr("km.kppbsum", sizeof(uint64_t) * (size_t)nb));
   uint32_t *done =
@@ -1007,8 +1026,8 @@ static bool init_plusplus(vsk_ctx *ctx, const float *dx, int64_t n, int32_t d,
     else
       k_kpp_update<<<(unsigned)ceil_div(n, KP_T), KP_T, 0, ctx->stream>>>(
           dx, ld, d, n, chosen, r, codes, par, nch, skipm, D, maxbits);
-    k_kpp_pick<<<(unsigned)nb, KP_T, 0, ctx->stream>>>(bsum, nb, D, n, maxbits, rng, r,
-                                                       chosen, done);
+    k_kpp_pick<<<(unsigned)nb, KP_T, 0, ctx->stream>>>(bsum, nb, m, D, n, maxbits, rng,
+                                                       r, chosen, done);
   }
   check_launch("kmeans_plusplus");
   std::vector<int64_t> h((size_t)k);
