@@ -1003,7 +1003,9 @@ static bool init_plusplus(vsk_ctx *ctx, const float *dx, int64_t n, int32_t d,
   float4 *par = nullptr;
   const size_t code_bytes = sizeof(uint4) * (size_t)ceil_div(n, 64) * 64 * nch;
   if (d <= 1 << 17) {
-    codes = static_cast<uint4 *>(ctx->scratch_ptr("km.kppcodes", code_bytes));
+    // (in the memory that the Lloyd iterations' plane of the rows takes next:
+    // twice as large, and written after the last pick)
+    codes = static_cast<uint4 *>(ctx->scratch_ptr("km.q.qh", code_bytes));
     par = static_cast<float4 *>(ctx->scratch_ptr("km.kpppar", sizeof(float4) * (size_t)n));
     k_kpp_codes<<<(unsigned)std::min<int64_t>(ceil_div(n, KP_T / 64), 16384), KP_T, 0,
                   ctx->stream>>>(
