@@ -318,6 +318,23 @@ def test_exact_scan_many_queries(ctx, shape):
     np.testing.assert_array_equal(db.distances(q, METRIC_L2), O.distances(q, x, METRIC_L2))
 
 
+@pytest.mark.parametrize("n", [1, 255, 257, 4096, 4097])
+def test_screen_plane_scale_of_few_rows(sctx, n):
+    """The scale of the rows' fp16 plane comes from the largest |x|, which
+    every workgroup finds for itself up to 4,096 rows: the largest row first
+    and last, 2^30 above the others, and one that is not a number; bit for
+    bit the oracle."""
+    x, q = _data(n, n, 40, 70)
+    for at, v in ((0, 2.0 ** 30), (n - 1, 2.0 ** 30), (n // 2, np.nan)):
+        print(f"plane scale n={n} at={at} v={v}", flush=True)
+        y = x.copy()
+        y[at] *= np.float32(v)
+        gd, gi = VectorDatabase(sctx, y).search(q, 10, METRIC_L2SQ)
+        od, oi = O.search_flat(q, y, 10, METRIC_L2SQ)
+        np.testing.assert_array_equal(gi, oi)
+        np.testing.assert_array_equal(gd, od)
+
+
 @pytest.mark.parametrize("metric", SCREEN)
 @pytest.mark.parametrize("scale", [2.0 ** -60, 1.0, 2.0 ** 40])
 def test_screen_planes_and_chunks(sctx, metric, scale):

@@ -88,6 +88,21 @@ __global__ __launch_bounds__(256) void k_split_rows(
   }
 }
 
+// the larger of m and a non-negative float's bits (a NaN counts as larger
+// than everything), and the largest of a wave's
+__device__ inline uint32_t max_bits(uint32_t m, float v) {
+  const uint32_t b = __float_as_uint(v) & 0x7FFFFFFFu;
+  return b > m ? b : m;
+}
+__device__ inline uint32_t wave_max(uint32_t m) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint32_t b = __shfl_xor(m, o);
+    m = b > m ? b : m;
+  }
+  return m;
+}
+
 // The screen's row plane in the layout plane_at, one wave per row:
 //  PLANE_HALF    h = fp16(x 2^e), e one power for all rows, from their
 //                largest |x|^2 (plane_scale)
@@ -96,15 +111,30 @@ __global__ __launch_bounds__(256) void k_split_rows(
 // maxbits[0..1]: the maxima over the rows of |h 2^-e| and |x - h 2^-e| (of
 // x / |x| for cosine) as float bits, maxbits[2] set when a cosine row's norm
 // is too small or not finite (atomic max; squares summed in double, rounded
-// up).
+// up).  maxbits[3]: the largest |x|^2, from the launch before or (sq given:
+// few rows) found by every workgroup for itself, which saves that launch on
+// the centroids of every Lloyd iteration (147,541 x 128, 196 centroids: 15 ->
+// 13 us an iteration with the launch that clears maxbits).
 __global__ __launch_bounds__(256) void k_half_rows(int kind, const float *x, int64_t n, int32_t d,
-                                                   int32_t ld, const uint32_t *maxsq,
+                                                   int32_t ld, const float *sq,
                                                    const float *norm, uint16_t *h, int32_t ldb,
                                                    float *inv, uint32_t *maxbits) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
   const bool cosine = kind == PLANE_COSINE;
-  const float scale = cosine ? 0x1p11f : kind == PLANE_HALF ? plane_scale(*maxsq) : 1.f;
+  uint32_t maxsq = maxbits[3];
+  if (sq) {  // uniform
+    __shared__ uint32_t s_mx[4];
+    maxsq = 0;
+    for (int64_t i = threadIdx.x; i < n; i += 256) maxsq = max_bits(maxsq, sq[i]);
+    maxsq = wave_max(maxsq);
+    if (lane == 0) s_mx[threadIdx.x >> 6] = maxsq;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) maxsq = s_mx[j] > maxsq ? s_mx[j] : maxsq;
+    if (blockIdx.x == 0 && threadIdx.x == 0) maxbits[3] = maxsq;
+  }
+  const float scale = cosine ? 0x1p11f : kind == PLANE_HALF ? plane_scale(maxsq) : 1.f;
   const double back = 1.0 / (double)scale;
   uint32_t mh = 0, mr = 0, bad = 0;
   for (int64_t r = blockIdx.x * 4 + (threadIdx.x >> 6); r < n; r += (int64_t)gridDim.x * 4) {
@@ -196,18 +226,12 @@ __global__ __launch_bounds__(256) void k_half_queries(const float *x, int64_t n,
 }
 
 // the largest of n non-negative floats, as bits, into *out (cleared by the
-// caller; a NaN counts as larger than everything)
+// caller)
 __global__ __launch_bounds__(256) void k_max_bits(const float *v, int64_t n, uint32_t *out) {
   uint32_t m = 0;
-  for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    const uint32_t b = __float_as_uint(v[i]) & 0x7FFFFFFFu;
-    m = b > m ? b : m;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const uint32_t b = __shfl_xor(m, o);
-    m = b > m ? b : m;
-  }
+  for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+    m = max_bits(m, v[i]);
+  m = wave_max(m);
   if ((threadIdx.x & 63) == 0 && m) atomicMax(out, m);
 }
 
@@ -216,14 +240,15 @@ void half_rows(vsk_ctx *ctx, int kind, const float *x, const float *sq, const fl
                uint32_t *state) {
   KernelTimer t(ctx, "half_plane");
   fill_i32(ctx, reinterpret_cast<int32_t *>(state), 4, 0);
-  if (kind == PLANE_HALF) {
+  const bool few = n <= 4096;
+  if (kind == PLANE_HALF && !few) {
     const int64_t gm = ceil_div(n, 256);
     k_max_bits<<<(unsigned)(gm < 1024 ? gm : 1024), 256, 0, ctx->stream>>>(sq, n, state + 3);
     check_launch("half_plane_max");
   }
   const int64_t g = ceil_div(n, 4);
   k_half_rows<<<(unsigned)(g < 16384 ? g : 16384), 256, 0, ctx->stream>>>(
-      kind, x, n, d, ld, state + 3, norm, h, ldb, inv, state);
+      kind, x, n, d, ld, kind == PLANE_HALF && few ? sq : nullptr, norm, h, ldb, inv, state);
   check_launch("half_plane");
 }
 
