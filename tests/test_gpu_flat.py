@@ -318,6 +318,26 @@ def test_exact_scan_many_queries(ctx, shape):
     np.testing.assert_array_equal(db.distances(q, METRIC_L2), O.distances(q, x, METRIC_L2))
 
 
+@pytest.mark.parametrize("shape", [(40, 9, 1), (64, 2048, 32), (64, 2049, 31), (64, 10_240, 32),
+                                   (33, 10_241, 32), (65, 2100, 33), (1000, 65, 29)])
+def test_exact_scan_narrow_rows(ctx, shape):
+    """The stream over rows of at most 32 columns (one chunk of them), one,
+    four and eight queries a wave, rows that end inside a tile; bit for bit
+    the oracle."""
+    n, nq, d = shape
+    x, q = _data(n + nq + d, n, nq, d)
+    x[n // 2] = np.inf
+    x[n // 3, d - 1] = np.nan
+    print(f"exact scan narrow rows {shape}", flush=True)
+    db = VectorDatabase(ctx, x)
+    for metric in (METRIC_L2SQ, METRIC_COSINE, METRIC_L1):
+        gd, gi = db.search(q, 10, metric)
+        od, oi = O.search_flat(q, x, 10, metric)
+        np.testing.assert_array_equal(gi, oi)
+        np.testing.assert_array_equal(gd, od)
+    np.testing.assert_array_equal(db.distances(q, METRIC_L2), O.distances(q, x, METRIC_L2))
+
+
 @pytest.mark.parametrize("n", [1, 255, 257, 4096, 4097])
 def test_screen_plane_scale_of_few_rows(sctx, n):
     """The scale of the rows' fp16 plane comes from the largest |x|, which

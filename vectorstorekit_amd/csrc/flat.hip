@@ -478,16 +478,27 @@ static void launch_stream_v(vsk_ctx *ctx, const FlatArgs &a, int mode) {
 // waves (9 or so a CU), since a small launch takes one wave's time; eight
 // when there is more to do, which reads the rows least often.  (10,000 x 128:
 // 8 queries one a wave 6.4, four a wave 7.4 us; 16 queries 9.6 and 8.1; 64
-// queries four a wave 15.3, eight 16.0; 128 queries 23.5 and 20.4.)
+// queries four a wave 15.3, eight 16.0; 128 queries 23.5 and 20.4.)  Rows of
+// at most 32 columns are one chunk of 32: with 64, the loads of the absent
+// half and nine waves a CU instead of 17 made 10,000 queries over 40 rows x 32
+// take 8.1 us (in tiles 7.9), now 6.1; of 8 columns 7.0 (5.0), now 4.9.
 template <int OP>
 static void launch_stream(vsk_ctx *ctx, const FlatArgs &a, int mode) {
   const int64_t tiles = ceil_div(a.r1 - a.r0, 64), cus = ctx->cu_count;
-  if (a.nq == 1 || tiles * a.nq <= 8 * cus)
-    launch_stream_v<OP, 1, 64>(ctx, a, mode);
-  else if (tiles * ceil_div(a.nq, 4) <= 10 * cus)
-    launch_stream_v<OP, 4, 64>(ctx, a, mode);
-  else
+  const bool narrow = a.kdim <= 32;  // (one chunk of 32 columns: half the loads and LDS)
+  if (a.nq == 1 || tiles * a.nq <= 8 * cus) {
+    if (narrow)
+      launch_stream_v<OP, 1, 32>(ctx, a, mode);
+    else
+      launch_stream_v<OP, 1, 64>(ctx, a, mode);
+  } else if (tiles * ceil_div(a.nq, 4) <= 10 * cus) {
+    if (narrow)
+      launch_stream_v<OP, 4, 32>(ctx, a, mode);
+    else
+      launch_stream_v<OP, 4, 64>(ctx, a, mode);
+  } else {
     launch_stream_v<OP, 8, 32>(ctx, a, mode);
+  }
 }
 
 template <int METRIC>
