@@ -217,9 +217,9 @@ void launch_screen_tail(vsk_ctx *ctx, const ScreenTailArgs &a, const char *name)
 // ascending into best_out[q * k ...] (NONE past the words): query q's words
 // are words[wseg[q] + i], i < cnt[q] (wseg a multiple of 4); only queries
 // with active[q] (all when null).  The keys are those of a scan writing
-// (word << 32) | position.  With wseg and cnt null, every query has wstride
-// words (a multiple of 4) at q * wstride.
-// lists (keys set): instead of best_out, the results -- the word as the
+// (word << 32) | position.
+// lists (keys set): every query has wstride words (a multiple of 4) at q *
+// wstride instead, and instead of best_out the results -- the word as the
 // distance and the stored id of row position % pitch of the list that the
 // query's probe key position / pitch names; (+inf, -1) past the words.
 struct ListResults {
