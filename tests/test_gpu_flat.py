@@ -403,19 +403,36 @@ def test_query_tile_groups(sctx, nq):
         c.close()
 
 
-def test_chunk_counters_between_batches(sctx):
-    """Chunk counters cleared by the chunk before: several filtered chunks a
-    call, the same call again, and calls of more and
-    of fewer queries in between (the counters' two sets move with the number
-    of queries); bit for bit the oracle."""
-    x, q = _data(77, 60_000, 300, 32)
+@pytest.mark.parametrize("metric,k,filters", [(METRIC_L2SQ, 9, 3), (METRIC_L1, 512, 2)])
+def test_chunk_counters_between_batches(sctx, metric, k, filters):
+    """Chunk counters cleared by the chunk before: two and three filtered
+    chunks a call (a segment count per workgroup in the screen's, one counter
+    a query in the exact scan's, which fills half of a list's slots a chunk),
+    the same call again, and calls of more and of fewer queries in between
+    (the counters' two sets move with the number of queries); bit for bit the
+    oracle.  A counter left standing overflows its list, and the call runs
+    again with a wait after each chunk: no call waits more than the first."""
+    n = 1_000_000
+    x, q = _data(77, n, 300, 8)
     db = VectorDatabase(sctx, x)
-    ref = {m: O.search_flat(q[:m], x, 9, METRIC_L2SQ) for m in (1, 37, 300)}
-    for m in (37, 300, 1, 37, 37, 300):
-        print(f"chunk counters nq={m}", flush=True)
-        gd, gi = db.search(q[:m], 9, METRIC_L2SQ)
+    ref = {m: O.search_flat(q[:m], x, k, metric) for m in (1, 37, 300)}
+    db.search(q, k, metric)  # (the plane and the scratch memory)
+    waits = None
+    for m in (37, 300, 1, 37, 37, 300, 1, 300):
+        print(f"chunk counters metric={metric} nq={m}", flush=True)
+        sctx.profile(True)
+        sctx.profile_reset()
+        gd, gi = db.search(q[:m], k, metric)
+        now = sctx.last_sync_count()
+        launches = {name: v[0] for name, v in sctx.profile_stats().items()}
+        sctx.profile(False)
         np.testing.assert_array_equal(gi, ref[m][1])
         np.testing.assert_array_equal(gd, ref[m][0])
+        kind = "screen" if metric == METRIC_L2SQ else "valu"
+        assert launches[f"flat_{kind}_dense"] == 1
+        assert launches[f"flat_{kind}_filter"] == filters
+        waits = now if waits is None else waits
+        assert now == waits
 
 
 @pytest.mark.parametrize("metric", SCREEN)

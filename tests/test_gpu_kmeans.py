@@ -91,6 +91,28 @@ def test_kmeans_plusplus_large(ctx, shape):
     np.testing.assert_array_equal(np.asarray(res.centroids), ref[0])
 
 
+def test_kmeans_plusplus_memory():
+    """k-means++ needs no memory that grows with rows x columns beside what
+    the same training needs from a random start."""
+    import torch
+
+    from vectorstorekit_amd import Context
+
+    n, d = 400_000, 256
+    x = torch.randn(n, d, device="cuda")
+    torch.cuda.synchronize()
+    used = {}
+    for method in ("random", "kMeansPlusPlus"):
+        print(f"kmeans memory {method}", flush=True)
+        c = Context(0)
+        free = torch.cuda.mem_get_info()[0]
+        cfg = KMeansClusteringConfiguration(maxIterations=1, initMethod=method, seed=1)
+        KMeansClustering(c, cfg).cluster(x, 64)
+        used[method] = free - torch.cuda.mem_get_info()[0]
+        c.close()
+    assert used["kMeansPlusPlus"] - used["random"] < n * d // 2, used
+
+
 def test_kmeans_custom_weights_empty_clusters(ctx):
     """Custom start with centroids far from the data (empty clusters refilled
     from the seeded stream), weights, and a run to convergence."""
