@@ -1708,6 +1708,9 @@ void progressive_topk(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t k,
   // writes every query's list and threshold, so neither needs clearing
   // (three fewer launches per call, which small problems notice).
   if (cap > n) cap = n;  // the whole database is one dense chunk
+  // the append counters' two sets (whole cache lines: a scan's 64 queries'
+  // atomics otherwise go to one line more)
+  const int64_t count_set = (nq + 63) & ~(int64_t)63;
   TopkWorkspace w;
   if (ws) {
     w = *ws;
@@ -1715,7 +1718,7 @@ void progressive_topk(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t k,
     w.thresh = static_cast<uint64_t *>(ctx->scratch_ptr("topk.thresh", 8 * nq));
     w.cand = static_cast<uint64_t *>(
         ctx->scratch_ptr("topk.cand", sizeof(uint64_t) * (size_t)nq * cap));
-    w.counts = static_cast<int32_t *>(ctx->scratch_ptr("topk.counts", 8 * nq));
+    w.counts = static_cast<int32_t *>(ctx->scratch_ptr("topk.counts", 8 * count_set));
     w.ovf_mask = static_cast<uint8_t *>(ctx->scratch_ptr("topk.ovfmask", nq + 64));
     w.seg_n = static_cast<int32_t *>(
         ctx->scratch_ptr("topk.segn", sizeof(int32_t) * (size_t)nq * VSK_MAX_SEG));
@@ -1819,7 +1822,7 @@ void progressive_topk(vsk_ctx *ctx, int64_t nq, int64_t n, int32_t k,
       }
     }
     if (clear && r0 + c < n) {
-      counts = counts == w.counts ? w.counts + nq : w.counts;
+      counts = counts == w.counts ? w.counts + count_set : w.counts;
       sa.next_counts = counts;
       if (!ctx->ovf_armed) {
         sa.next_overflow = ctx->ovf_dev;
