@@ -338,6 +338,24 @@ def test_exact_scan_narrow_rows(ctx, shape):
     np.testing.assert_array_equal(db.distances(q, METRIC_L2), O.distances(q, x, METRIC_L2))
 
 
+@pytest.mark.parametrize("shape", [(131_073, 48, 33), (131_073, 49, 33), (131_073, 40, 32),
+                                   (131_073, 41, 32), (130_900, 64, 9), (57_000, 41, 24),
+                                   (100_000, 24, 32)])
+def test_exact_scan_some_queries_many_rows(ctx, shape):
+    """Where the stream over the rows ends: 40 (rows of at most 32 columns) and
+    48 queries, fewer than 1,024 tiles of 128 rows, and the 64 x 32 tiles of
+    narrow rows; bit for bit the oracle."""
+    n, nq, d = shape
+    x, q = _data(n + nq, n, nq, d)
+    print(f"exact scan some queries many rows {shape}", flush=True)
+    db = VectorDatabase(ctx, x)
+    gd, gi = db.search(q, 20, METRIC_L1)
+    od, oi = O.search_flat(q, x, 20, METRIC_L1)
+    np.testing.assert_array_equal(gi, oi)
+    np.testing.assert_array_equal(gd, od)
+    np.testing.assert_array_equal(db.distances(q, METRIC_COSINE), O.distances(q, x, METRIC_COSINE))
+
+
 @pytest.mark.parametrize("n", [1, 255, 257, 4096, 4097])
 def test_screen_plane_scale_of_few_rows(sctx, n):
     """The scale of the rows' fp16 plane comes from the largest |x|, which

@@ -565,8 +565,15 @@ void launch_flat(vsk_ctx *ctx, FlatArgs a, int mode, int32_t *argmin) {
   // and 13.1, 4,000 queries 28.8 and 34.3; 10,000 x 128, 256 queries 33.6 and
   // 35.3; of 512 columns, 1,800 queries x 4,096 rows, 281 and 269)
   const bool few = valu && mode != MODE_ARGMIN && qt * splits < 4 * (int64_t)ctx->cu_count;
-  const bool small = few && a.nq > 64 && a.kdim <= 128 &&
-                     a.nq * rows >= 10000 * (int64_t)ctx->cu_count;
+  // (of at most 32 columns also fewer queries, where they nearly fill a tile:
+  // 100,000 x 32, the distances of 32 queries 13.4 and 14.5, 40 21.8 and 16.4,
+  // 64 22.2 and 24.9)
+  const bool narrow = a.kdim <= 32;
+  const int64_t pairs = a.nq * rows;
+  const bool small = few && a.kdim <= 128 &&
+                     ((a.nq > 64 && pairs >= 10000 * (int64_t)ctx->cu_count) ||
+                      (narrow && (a.nq > 40 || (a.nq > 16 && a.nq <= 32)) &&
+                       pairs >= 9000 * (int64_t)ctx->cu_count));
   if (small) {
     tq = 32;
     tn = 64;
@@ -580,11 +587,16 @@ void launch_flat(vsk_ctx *ctx, FlatArgs a, int mode, int32_t *argmin) {
   const char *name = names[valu ? 1 : 0][mode];
   KernelTimer t(ctx, name, (double)a.nq * (double)rows);
   if (valu) {
-    // up to 64 queries, or fewer than 4 tiles a CU: the stream over the rows
-    // (at 64 queries the two take the same time over 100,000 x 768, 346 and
-    // 355 us; at 128 the tiles need 501, the stream 529)
+    // up to 48 queries, or fewer than 4 tiles a CU: the stream over the rows,
+    // whose waves all wait on the VALU from there on, where a tile of 64
+    // queries reads a row once (us, tiles and stream; 854,462 x 768,
+    // Manhattan: 40 queries 2,000 and 1,510, 48 1,930 and 1,800, 49 1,940 and
+    // 2,060, 64 1,930 and 2,310; the dot products of 300,000 x 128: 48 115 and
+    // 107, 49 115 and 123, 64 119 and 139; of 854,462 x 32: 40 89 and 86, 48
+    // 103 and 108; 100,000 x 768 in few tiles: 56 285 and 244, 64 290 and 294)
     // (a grid of at most 2^25 waves)
-    const bool stream = mode != MODE_ARGMIN && !small && (a.nq <= 64 || few) &&
+    const bool stream = mode != MODE_ARGMIN && !small &&
+                        (a.nq <= (narrow ? 40 : 48) || few) &&
                         ceil_div(rows, 64) * ceil_div(a.nq, 8) <= 1 << 25;
     switch (a.metric) {
     case VSK_METRIC_L1: launch_exact<OP_L1>(ctx, grid, a, mode, argmin, stream, small); break;
