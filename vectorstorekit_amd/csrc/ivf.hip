@@ -29,6 +29,7 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <numeric>
@@ -74,11 +75,11 @@ struct vsk_ivf {
   // per list the largest distance of its rows from its centroid (for the
   // list scan's per-query bound), valid with the plane
   mutable vsk::DevBuf xrad;
-  // top_rows[i]: the rows of the i largest lists together (i <= nlist),
-  // valid while tversion == version; filled by the first search after a
-  // change, which may be several contexts' searches at once (top_mutex)
+  // top_rows[i]: the rows of the i largest lists together, for the probe
+  // counts that were asked for since the rows changed (tversion == version);
+  // searches of several contexts may ask at once (top_mutex)
   mutable std::mutex top_mutex;
-  mutable std::vector<int64_t> top_rows;
+  mutable std::map<int32_t, int64_t> top_rows;
   mutable int64_t tversion = -1;
 };
 
@@ -1380,18 +1381,25 @@ static bool list_screen_applies(vsk_ctx *ctx, const vsk_ivf *ivf, int32_t metric
 // candidates a query can have with np probes: the sizes of the np largest
 // lists summed (every row when every list is probed)
 static int64_t probe_bound(const vsk_ivf *ivf, int32_t np) {
+  if (np >= ivf->nlist) return ivf->total;
   std::lock_guard<std::mutex> lock(ivf->top_mutex);
   if (ivf->tversion != ivf->version) {
-    // (sorted once per change of the rows: 10 us at 1,024 lists, which a
-    // search of one query would notice)
-    std::vector<int64_t> sz(ivf->nlist);
-    for (int32_t l = 0; l < ivf->nlist; ++l) sz[l] = ivf->off[l + 1] - ivf->off[l];
-    std::sort(sz.begin(), sz.end(), std::greater<int64_t>());
-    ivf->top_rows.assign(ivf->nlist + 1, 0);
-    for (int32_t l = 0; l < ivf->nlist; ++l) ivf->top_rows[l + 1] = ivf->top_rows[l] + sz[l];
+    ivf->top_rows.clear();
     ivf->tversion = ivf->version;
   }
-  return ivf->top_rows[np < ivf->nlist ? np : ivf->nlist];
+  // (kept: some 10 us at 1,024 lists, which a search of one query would
+  // notice.  Sorting the lists once for every probe count took a first
+  // search 20 us more.)
+  const auto it = ivf->top_rows.find(np);
+  if (it != ivf->top_rows.end()) return it->second;
+  std::vector<int64_t> sz(ivf->nlist);
+  for (int32_t l = 0; l < ivf->nlist; ++l) sz[l] = ivf->off[l + 1] - ivf->off[l];
+  std::nth_element(sz.begin(), sz.begin() + np, sz.end(), std::greater<int64_t>());
+  int64_t rows = 0;
+  for (int32_t i = 0; i < np; ++i) rows += sz[i];
+  if (ivf->top_rows.size() >= 1024) ivf->top_rows.clear();
+  ivf->top_rows[np] = rows;
+  return rows;
 }
 
 // the stored rows' bf16 plane (roundup(d, 64) columns), |x|^2 per row and
