@@ -105,30 +105,37 @@ def test_profile_reset_after_failed_profiled_call(spec):
 
 
 def _after_every_fault(kinds, make, search, want):
-    """Fails event n = 1, 2, ... of a fresh context in turn until a run of
-    make and search meets none; whenever the search is what failed, the same
-    call on the same object must then return ``want``."""
+    """Fails event n = 1, 2, ... of a fresh context in turn until three runs of
+    make and search on end meet none; whenever the search is what failed, the
+    same call on the same object must then return ``want``, as must a search
+    that answers."""
     tried = 0
     for kind in kinds:
+        clean = 0
         for n in range(1, 200):
             print(f"fault {kind}:{n}", flush=True)
             ctx = _armed(f"{kind}:{n}")
             obj = None
             try:
-                obj = make(ctx)
-                search(obj)
-                break
-            except VSKError as e:
-                assert "injected fault" in str(e)
-                if obj is not None:
+                try:
+                    obj = make(ctx)
+                    gd, gi = search(obj)
+                    clean += 1
+                except VSKError as e:
+                    assert "injected fault" in str(e)
+                    clean = 0
+                    if obj is None:
+                        continue
                     tried += 1
                     gd, gi = search(obj)
-                    np.testing.assert_array_equal(gi, want[1])
-                    np.testing.assert_array_equal(gd, want[0])
+                np.testing.assert_array_equal(gi, want[1])
+                np.testing.assert_array_equal(gd, want[0])
             finally:
                 if obj is not None:
                     obj.free()
                 ctx.close()
+            if clean == 3:
+                break
         else:
             raise AssertionError("every event failed")
     assert tried > 3
@@ -169,3 +176,43 @@ def test_fault_while_the_probe_plane_is_made(monkeypatch):
     _after_every_fault(("launch", "alloc", "sync"), lambda ctx: IVFIndex.build(ctx, cfg, c, x),
                        lambda idx: idx.search(q, 10),
                        O.ivf_search(q, x, np.arange(len(x)), lists, c, 5, 10))
+
+
+@pytest.mark.parametrize("metric", ["euclideanSquared", "cosine", "cosineNormalized"])
+def test_no_memory_for_the_screen_plane(metric, monkeypatch):
+    """A search whose plane finds no memory (the host reports that allocation
+    as failed) answers by the exact scan, bit for bit the oracle; the next
+    one makes the plane and screens."""
+    monkeypatch.setenv("VSK_FLAT_KERNEL", "screen")
+    x, q = _close_rows(20_000, 40, 16)
+    code = {"euclideanSquared": O.L2SQ, "cosine": O.COSINE,
+            "cosineNormalized": O.COSINE_NORMALIZED}[metric]
+    od, oi = O.search_flat(q, x, 10, code)
+    answered = 0
+    for n in range(1, 60):
+        print(f"no memory {metric} alloc:{n}", flush=True)
+        ctx = _armed(f"alloc:{n}")
+        ctx.profile(True)
+        db = None
+        try:
+            db = VectorDatabase(ctx, x)
+            screened = []
+            for _ in range(2):
+                ctx.profile_reset()
+                gd, gi = db.search(q, 10, metric)
+                screened.append(any(k.startswith("flat_screen") for k in ctx.profile_stats()))
+                np.testing.assert_array_equal(gi, oi)
+                np.testing.assert_array_equal(gd, od)
+            if screened == [True, True]:
+                break  # (no allocation left to fail)
+            assert screened == [False, True]
+            answered += 1
+        except VSKError as e:
+            assert "injected fault" in str(e)
+        finally:
+            if db is not None:
+                db.free()
+            ctx.close()
+    else:
+        raise AssertionError("every allocation failed")
+    assert answered >= 1

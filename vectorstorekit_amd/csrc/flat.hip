@@ -709,15 +709,17 @@ SplitPtrs make_split(vsk_ctx *ctx, const vsk_db *db, const float *dq,
   return s;
 }
 
-// the screen's planes: the database's (made once) and the query batch's
-static SplitPtrs make_half(vsk_ctx *ctx, const vsk_db *db, const float *dq, int64_t nq,
-                           int32_t metric, float *qnh, float *qnr) {
-  // whole 64-dimension stages of the screen (zero padding)
-  const int32_t ldb = (db->d + 63) & ~63;
-  const bool cosine = metric == VSK_METRIC_COSINE;
-  const bool bf16 = metric == VSK_METRIC_COSINE_NORMALIZED;
-  auto &pl = db->plane[bf16 ? 1 : 0];
-  if (!cosine && !pl.h.p) {
+// whether the screen can read the rows for this metric: their plane, made by
+// the first search that asks for it.  Without memory for one more plane (each
+// family of metrics has its own: L2, L2^2 and dot; cosine; normalised cosine)
+// the answer is no, and the exact scan serves the search.
+static bool screen_plane_ok(vsk_ctx *ctx, const vsk_db *db, int32_t metric) {
+  try {
+    if (metric == VSK_METRIC_COSINE) return cosine_screen_ok(ctx, db);
+    const bool bf16 = metric == VSK_METRIC_COSINE_NORMALIZED;
+    auto &pl = db->plane[bf16 ? 1 : 0];
+    if (pl.h.p) return true;
+    const int32_t ldb = (db->d + 63) & ~63;
     pl.state.reserve(4 * sizeof(uint32_t));
     DevBuf h;  // (the database gets it with its maxima, as in make_split)
     h.reserve(plane_bytes(db->n, ldb));
@@ -730,7 +732,21 @@ static SplitPtrs make_half(vsk_ctx *ctx, const vsk_db *db, const float *dq, int6
     std::memcpy(&pl.max_hi, &hb[0], sizeof(float));
     std::memcpy(&pl.max_res, &hb[1], sizeof(float));
     pl.h.swap(h);
+    return true;
+  } catch (const Error &e) {
+    if (e.code != VSK_ERR_OUT_OF_MEMORY) throw;
+    return false;
   }
+}
+
+// the screen's planes: the database's (screen_plane_ok) and the query batch's
+static SplitPtrs make_half(vsk_ctx *ctx, const vsk_db *db, const float *dq, int64_t nq,
+                           int32_t metric, float *qnh, float *qnr) {
+  // whole 64-dimension stages of the screen (zero padding)
+  const int32_t ldb = (db->d + 63) & ~63;
+  const bool cosine = metric == VSK_METRIC_COSINE;
+  const bool bf16 = metric == VSK_METRIC_COSINE_NORMALIZED;
+  const auto &pl = db->plane[bf16 ? 1 : 0];
   uint16_t *qh = static_cast<uint16_t *>(
       ctx->scratch_ptr("flat.qhalf", sizeof(uint16_t) * (size_t)nq * ldb));
   SplitPtrs s{};
@@ -763,13 +779,13 @@ bool flat_topk_device(vsk_ctx *ctx, const vsk_db *db, const float *dq,
     approx_topk(ctx, db, dq, nq, k, exact_metric(metric), best, 3);
     return true;
   }
-  if (screen && (metric != VSK_METRIC_COSINE || cosine_screen_ok(ctx, db))) {
+  if (screen && screen_plane_ok(ctx, db, metric)) {
     screen_topk(ctx, db, dq, nq, k, metric, best, defer);
     return true;
   }
   if (screen) {
-    // cosine over rows whose norms the screen's bound cannot cover: the
-    // exact scan
+    // cosine over rows whose norms the screen's bound cannot cover, or no
+    // memory for the plane: the exact scan
     approx_topk(ctx, db, dq, nq, k, exact_metric(metric), best, 3);
     return true;
   }
@@ -786,7 +802,8 @@ void approx_topk(vsk_ctx *ctx, const vsk_db *db, const float *dq, int64_t nq,
   // tiles spreads a query's slots over some 56 workgroups, about 18
   // candidates in 36 slots each, and of 333 queries one or two overflowed:
   // the call ran again, its chunks re-scanned (200,003 x 384, k = 50:
-  // 1.52 ms a call, with room 0.37).
+  // 1.52 ms a call, with room 0.37, and 0.28 since no workgroups are launched
+  // for absent query tiles).
   if (passes == 1 && nq <= 1024 && ctx->max_tile_bytes <= 0) {
     // (whole row tiles, so that every chunk starts on one)
     cap = std::max<int64_t>(cap, std::min<int64_t>(ceil_div(32 * (int64_t)k, 256) * 256, 16384));

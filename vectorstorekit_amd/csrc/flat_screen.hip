@@ -58,8 +58,8 @@ bool screen_applies(int32_t metric, int32_t k) {
 bool cosine_screen_ok(vsk_ctx *ctx, const vsk_db *db) {
   if (db->cos_state == 0) {
     const int32_t ldb = (db->d + 63) & ~63;
-    db->cos_half.reserve(plane_bytes(db->n, ldb));
     db->cos_inv.reserve(sizeof(float) * (size_t)db->n);
+    db->cos_half.reserve(plane_bytes(db->n, ldb));
     uint32_t *st = static_cast<uint32_t *>(ctx->scratch_ptr("screen.cosrel", 16));
     half_rows(ctx, PLANE_COSINE, db->x.as<float>(), nullptr, db->norm.as<float>(), db->n, db->d,
               db->ld, db->cos_half.as<uint16_t>(), ldb, db->cos_inv.as<float>(), st);
