@@ -298,8 +298,8 @@ def setup(c, a, ctx, dev):
             "kernels": [("flat_screen_filter", "k_flat_screen<FILTER>", "mfma_bf16"),
                         ("flat_screen_dense", "k_flat_screen<DENSE>", "mfma_bf16"),
                         # small problems: the exact sequential scan alone
-                        ("flat_valu_dense", "k_flat_valu<DENSE> (exact, dimension order)",
-                         "valu_l2" if c == "c1" else "valu_dot"),
+                        ("flat_valu_dense", "k_flat_stream / k_flat_valu<DENSE> (exact, "
+                         "dimension order)", "valu_l2" if c == "c1" else "valu_dot"),
                         ("flat_bf16x3_filter", "k_flat_bf16x3<FILTER>", "mfma"),
                         ("flat_bf16x3_dense", "k_flat_bf16x3<DENSE>", "mfma"),
                         ("flat_mfma_filter", "k_flat_mfma<FILTER>", "mfma32"),
@@ -360,11 +360,11 @@ def setup(c, a, ctx, dev):
                     "centre + 0.5 N(0,I) (seeds 5, 1)",
             "dtype": "f32", "nq": n, "n": ncent, "d": d,
             "units_per_step": n * iters, "unit": "row-iterations/s",
-            "kernels": [("kmeans_plusplus", "k-means++ seeding (k_kpp_update / blocksum / "
-                         "pick per centroid)", "kpp"),
+            "kernels": [("kmeans_plusplus", "k-means++ seeding (k_kpp_update / pick "
+                         "per centroid)", "kpp"),
                         ("flat_valu_argmin", "k_flat_valu<ARGMIN> (exact sqrt-L2, dimension "
                          "order)", "valu_l2"),
-                        ("flat_screen_top2", "k_flat_screen<TOP2> (bf16 screen, smallest two per "
+                        ("flat_screen_top2", "k_flat_screen<TOP2> (fp16 screen, smallest two per "
                          "row)", "mfma_bf16")],
             "keep": (x, cent, assign),
         }
@@ -623,7 +623,7 @@ def setup(c, a, ctx, dev):
     lut = c == "c5lut"
     sctx = ctx
     if lut:
-        # codes only: a context without the bf16 screen (VSK_FLAT_KERNEL=
+        # codes only: a context without the screen (VSK_FLAT_KERNEL=
         # exact) scans the codes with the LDS tables, no decoded plane
         from vectorstorekit_amd import Context
         old = os.environ.get("VSK_FLAT_KERNEL")
@@ -671,7 +671,7 @@ def setup(c, a, ctx, dev):
                      "pq-adc-codes-only-10Mx128-m16-q1000-kadc1000-l1rerank-k100 (BASELINE "
                      "config 5, LUT scan over the codes, no decoded plane)"),
         "ctx": sctx,
-        "device_bytes": {"codes": code_bytes, "decoded_bf16_plane": plane_bytes,
+        "device_bytes": {"codes": code_bytes, "decoded_fp16_plane": plane_bytes,
                          "note": "the search's index memory besides the fp32 rows the "
                                  "re-rank reads" + ("" if lut else
                                  "; the screen's decoded plane is 16x the codes")},
@@ -681,7 +681,7 @@ def setup(c, a, ctx, dev):
                 "centre + 0.5 N(0,I) (seeds 5, 1, 2); codebooks: 8 Lloyd iterations "
                 "per segment on the first 65,536 rows (GPU assignment)",
         "dtype": "u8 codes, f32 LUT", "nq": nq, "n": n, "d": d, "M": M,
-        # filtered chunks: the bf16 screen over the decoded rows (one bf16
+        # filtered chunks: the fp16 screen over the decoded rows (one fp16
         # product per pair), then the survivors' exact ADC sums; the dense
         # first chunk: the LUT scan
         "kernels": ([("flat_screen_filter", "k_flat_screen<FILTER> over the decoded PQ rows",

@@ -601,8 +601,12 @@ __device__ inline float xs_dist(float dot, float qa, float xa) {
 // residuals, and with them the bound and the rows rescored, are an eighth of
 // bf16's at the same MFMA rate.  200,003 x 384 clustered rows, 333 queries,
 // k = 50: with bf16 every query missed the bound and ran a second, wider
-// screen (a call 3.1 to 3.4 ms); with fp16 none does (0.37 ms).  Normalised cosine keeps the bf16 planes: which near
-// ties its tiers settle is part of what the tests pin.
+// screen (a call 3.1 to 3.4 ms); with fp16 none does (0.28 ms).  Normalised
+// cosine has the bf16 planes it always had, and with them that second screen
+// on such rows (803 us where
+// L2 takes 284); on unclustered ones (1M x 768, 10,000 queries) its
+// bound holds.  The near ties its tests plant, and the tiers that settle
+// them, are placed by bf16's bound.
 template <int METRIC>
 constexpr bool xs_bf16 = METRIC == VSK_METRIC_COSINE_NORMALIZED;
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
@@ -758,7 +762,7 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
         // max with 0, <= thf) only when dot - xa/2 >= (qa - thf)/2 less a
         // margin for the roundings of both forms.  A passing row has
         // (|x| - 1.01|q|)^2 <= 0.03 |q|^2 + thf + 1 (|dot| <= 1.01 |q||x| for
-        // the bf16 products), which bounds its |x|^2 by xq2 below; every
+        // the 16-bit products), which bounds its |x|^2 by xq2 below; every
         // rounding is then within 2^-22 (thf + qa + xq2 + 1), and the margin
         // takes four times that.
         const double qa = (double)s_qa[tid], t = (double)thf;
@@ -778,8 +782,9 @@ void k_flat_screen(FlatArgs a, SplitPtrs s) {
         s_tdot[tid] = f * sc;
       } else if constexpr (METRIC == VSK_METRIC_COSINE) {
         // cosine (with the reference's epsilon): a <= thf is
-        // dot >= (1 - thf) den, den = |q||x| + 1e-8 > 0; the bound t2 on
-        // dot / den sits 2^-20 (1 + |1 - thf|) below 1 - thf, more than
+        // dot >= (1 - thf) den, dot = q.x / |x| and den = |q| + 1e-8 / |x| >
+        // 0 (the plane's rows are divided by |x|); the bound t2 on dot / den
+        // sits 2^-20 (1 + |1 - thf|) below 1 - thf, more than
         // the roundings of either form, so no score whose exact test below
         // passes is under it
         float f;

@@ -2445,7 +2445,9 @@ static vsk_status ivf_search_any(vsk_ctx *ctx, const vsk_ivf *ivf, const float *
       } else if (kind == 1) {
         VSK_SCAN_QG(k_list_scan_sq8)
       } else {
-        // (code rows are aligned to their stride's powers of two)
+        // (code rows are aligned to their stride's powers of two.  256
+        // codewords a segment go up to M = 16, since a quantizer's four tables
+        // fit 64 KB of LDS: between, and with fewer codewords, word by word)
         if (la.ksub == 256 && la.M == 16 && la.cstride % 16 == 0)
           k_list_scan_pq_q<4><<<(unsigned)nb, 256, (size_t)per_q, ctx->stream>>>(la);
         else if (la.ksub == 256 && la.M == 8 && la.cstride % 8 == 0)

@@ -102,7 +102,7 @@ struct vsk_ctx {
   void *scratch_ptr(const std::string &key, size_t bytes);
 
   // flat top-k path, from the environment VSK_FLAT_KERNEL at context
-  // creation: unset = one-pass bf16 screen with exact fp32 rescore where the
+  // creation: unset = one-pass 16-bit screen with exact fp32 rescore where the
   // metric allows it (the exact sequential scan alone for small problems,
   // bf16x3 elsewhere); "screen" = the screen at every size; "bf16x3" =
   // bf16x3 split MFMA only; "fp32" = fp32 MFMA only
@@ -115,7 +115,7 @@ struct vsk_ctx {
   // (Acceleration/Metal/MetalDistanceCompute.swift:371-380, 450-473).  0:
   // the defaults (2 GiB of candidate keys, at least 64 queries a batch)
   int64_t max_tile_bytes = 0;
-  // "exact": no bf16 screen anywhere -- the exact scans alone (flat search
+  // "exact": no screen anywhere -- the exact scans alone (flat search
   // on the exact VALU kernel for its screenable metrics, IVF's exact probe
   // and list scans, PQ's LUT scan over the codes, the exact argmin)
   bool exact_only = false;
@@ -196,9 +196,8 @@ struct vsk_db {
   vsk::DevBuf sqnorm;  // n: sum x^2 (fp32)
   vsk::DevBuf norm;    // n: sqrt(sum x^2)
   // row-major bf16 hi/lo planes for the bf16x3 kernel and the IVF probe's
-  // screen, built
-  // on first use (the lo plane only for bf16x3), and the maxima over the rows
-  // of |hi| and |x - hi|
+  // screen, built on first use (the lo plane only for bf16x3), and the maxima
+  // over the rows of |hi| and |x - hi|
   mutable vsk::DevBuf split, split_lo;
   // the flat screen's tiled planes of the rows, [0] fp16, [1] bf16 (normalised
   // cosine), each made by the first search that screens with it: the state on
