@@ -603,10 +603,9 @@ __device__ inline float xs_dist(float dot, float qa, float xa) {
 // k = 50: with bf16 every query missed the bound and ran a second, wider
 // screen (a call 3.1 to 3.4 ms); with fp16 none does (0.28 ms).  Normalised
 // cosine has the bf16 planes it always had, and with them that second screen
-// on such rows (803 us where
-// L2 takes 284); on unclustered ones (1M x 768, 10,000 queries) its
-// bound holds.  The near ties its tests plant, and the tiers that settle
-// them, are placed by bf16's bound.
+// on such rows (803 us where L2 takes 284); on unclustered ones (1M x 768,
+// 10,000 queries) its bound holds.  The near ties its tests plant, and the
+// tiers that settle them, are placed by bf16's bound.
 template <int METRIC>
 constexpr bool xs_bf16 = METRIC == VSK_METRIC_COSINE_NORMALIZED;
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
